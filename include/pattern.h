@@ -536,21 +536,26 @@ int pat_gr_destroy(pat_gr *h);
  * api/gpu/regular_table.hpp, which defines pat_app_gr_table().  Replaces the
  * reference's regular compute_gpu with its LDS and device hash objects
  * (kmeans/regular/gpu_kernel.cu:39-183, ros.cu:15-170, rog.cu:17-310).
- * Each wavefront folds its units into an LDS hash table (lanes inserting in
- * turn); a full table is merged into the wavefront's table in device memory
- * and the refused units' maps run again; the wavefronts' tables are then
- * folded in a fixed order into the final table, so every value is the same
- * fold every run. */
+ * Each wavefront folds its units into an LDS hash table (lanes inserting
+ * together, a key's values in lane order); a full table is merged into the
+ * wavefront's table in device memory and the refused units' maps run again;
+ * the wavefronts' records are then folded key by key in wavefront order, so
+ * every value is the same fold every run. */
 typedef struct pat_gr_object { /* device memory of one run, set up by the library */
     const void *data;          /* the units' bytes */
     const int64_t *offsets;    /* byte offset of each unit in data, or NULL: unit i at i * unit_bytes */
     int64_t unit_bytes, num_units;
     const void *param;         /* the functors' parameter (may be NULL) */
-    uint32_t *wave_tables;     /* waves tables of (table_buckets + 1 + table_pool_words) words */
-    uint32_t *final_table;     /* one table of that size */
-    int32_t *status;           /* [0] error bits (1 a wavefront's table full, 2 a unit's values do not fit
-                                  an empty LDS table, 4 a map's insert refused after another was taken,
-                                  8 the final table full), [1] LDS merges, [2] maps run again */
+    uint32_t *wave_tables;     /* waves tables of (table_buckets + table_pool_words) words */
+    int32_t *wave_counts;      /* per wavefront: entries of its table's buckets in use */
+    uint32_t *matrix;          /* table_buckets rows of waves words, all 0 before and after a run */
+    unsigned long long *final_buckets; /* table_buckets */
+    int32_t *slots;            /* table_buckets: the final buckets taken */
+    uint32_t *final_pool;      /* table_pool_words: the final records, back to back */
+    int32_t *status;           /* 0 before a run.  [0] error bits (1 a wavefront's table full, 2 a unit's values
+                                  do not fit an empty LDS table, 4 a map's insert refused after another was
+                                  taken, 8 the final table full), [1] LDS merges, [2] maps run again, [3] keys,
+                                  [4] words of final records */
     int32_t waves, table_buckets, table_pool_words, lds_buckets, lds_pool_words;
 } pat_gr_object;
 typedef struct pat_gr_table {

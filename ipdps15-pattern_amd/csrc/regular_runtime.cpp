@@ -2,9 +2,9 @@
 // keyed reduction objects: RegularRuntime (kmeans/regular/regular_runtime.h:
 // 79-105, regular_runtime.cu:31-291) for any map_fp / reduce_fp pair.  The
 // input and its unit offsets are copied to the device once; each start
-// sizes the wavefront tables and the final table, runs the application
-// table's kernels (api/gpu/regular_table.hpp) and reads the final table back,
-// its records sorted by key bytes.
+// sizes the wavefront tables and the final records, runs the application
+// table's kernels (api/gpu/regular_table.hpp) and reads the final records
+// back, sorted by key bytes.
 //
 // The reference's RegularRuntime splits units over the CPU threads and GPUs
 // by a speed profile, feeds the GPU from mapped host memory and merges the
@@ -13,8 +13,6 @@
 // one start is one device pass and the object comes back whole.
 #include <algorithm>
 #include <cstring>
-#include <string>
-#include <utility>
 #include <vector>
 
 #include "pat_common.hpp"
@@ -23,8 +21,19 @@ namespace {
 
 constexpr int64_t kDefaultKeys = 4096;
 constexpr int64_t kDefaultRecordBytes = 256;
-constexpr int kMaxWaves = 1024;
-constexpr int64_t kUnitsPerWave = 4096;
+// Wavefronts: a run of at least 256 units each (four rounds of the lanes, so
+// that an LDS table's set-up and its records' way out stay small beside
+// them), and no more than eight per CU, beyond which the fold's rows grow and
+// the map gains nothing.  Each holds a table of the object's full capacity in
+// case its LDS table overflows: their number is also held to kTableWords, or
+// to one per kUnitsFew units where that takes more.
+constexpr int kMaxWaves = 2048;
+constexpr int64_t kUnitsPerWave = 256;
+constexpr int64_t kUnitsFew = 4096;
+constexpr int kMaxWavesFew = 1024;
+constexpr int64_t kTableWords = 1LL << 28;
+constexpr int kStatusWords = 8;
+constexpr int64_t kFirstWords = 65536;  // final records read back together with the status: 256 KiB, about 5 us
 
 int64_t pow2_at_least(int64_t v)
 {
@@ -45,21 +54,32 @@ struct pat_regular {
     int64_t param_bytes = 0;
     int64_t max_keys = kDefaultKeys, max_record_bytes = kDefaultRecordBytes;
     int lds_keys = 0;
-    uint32_t *tables = nullptr;  // wave tables then the final table
+    uint32_t *tables = nullptr;  // wave tables, wave counts, final buckets, slots
     int64_t tables_words = 0;
-    int32_t *status = nullptr;
+    uint32_t *matrix = nullptr;  // all 0 between starts
+    int64_t matrix_words = 0;
+    bool matrix_clear = false;
+    uint32_t *final = nullptr;  // status then the final records, read back together
+    int64_t final_words = 0;
+    uint32_t *host = nullptr;  // pinned: the status and the first kFirstWords of records
     hipStream_t stream = nullptr;
-    // last start
+    // last start: the records, back to back, and their places in key order
     bool have_result = false;
-    std::vector<std::pair<std::string, std::string>> out;
+    std::vector<uint32_t> records;
+    struct Place {
+        uint64_t prefix;  // the key's first eight bytes, big-endian, zero-padded
+        uint32_t at;
+    };
+    std::vector<Place> out;
     int64_t merges = 0, reruns = 0;
     int waves = 0;
 
     void release()
     {
         if (stream) (void)hipStreamSynchronize(stream);
-        for (void *p : {input, (void *)offsets, param, (void *)tables, (void *)status})
+        for (void *p : {input, (void *)offsets, param, (void *)tables, (void *)matrix, (void *)final})
             if (p) (void)pat::dev_free(p);
+        if (host) (void)hipHostFree(host);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -68,25 +88,77 @@ struct pat_regular {
     int64_t buckets() const { return pow2_at_least(2 * max_keys); }
     int64_t pool_words() const { return max_keys * (1 + (max_record_bytes + 3) / 4 + 1); }
 
+    // The final record at word 'at': header, key and value, each in whole words.
+    static int64_t record_words(uint32_t hdr) { return 1 + (int64_t)((hdr >> 16) + 3) / 4 + ((hdr & 0xffffu) + 3) / 4; }
+    int key_size(uint32_t at) const { return (int)(records[at] >> 16); }
+    int value_size(uint32_t at) const { return (int)(records[at] & 0xffffu); }
+    const unsigned char *key(uint32_t at) const { return (const unsigned char *)(records.data() + at + 1); }
+    const unsigned char *value(uint32_t at) const
+    {
+        return (const unsigned char *)(records.data() + at + 1 + (key_size(at) + 3) / 4);
+    }
+
+    // Sorts 'out' by key bytes: a byte-wise radix sort of the prefixes, least
+    // byte first (bytes all keys share are skipped: 5,003 four-byte keys take
+    // two passes, some 20 us, where comparing took 0.25 ms), then runs of one
+    // prefix by the rest.
+    void sort_places()
+    {
+        std::vector<Place> other(out.size());
+        for (int shift = 0; shift < 64; shift += 8) {
+            size_t first[257] = {0};
+            for (const Place &e : out) first[(e.prefix >> shift & 255) + 1]++;
+            if (*std::max_element(first + 1, first + 257) == out.size()) continue;
+            for (int i = 0; i < 256; i++) first[i + 1] += first[i];
+            for (const Place &e : out) other[first[e.prefix >> shift & 255]++] = e;
+            out.swap(other);
+        }
+        auto rest = [this](const Place &a, const Place &b) {
+            const int ka = key_size(a.at), kb = key_size(b.at);
+            const int c = memcmp(key(a.at), key(b.at), (size_t)std::min(ka, kb));
+            if (c || ka != kb) return c ? c < 0 : ka < kb;
+            // one key with values of two sizes: two records
+            const int va = value_size(a.at), vb = value_size(b.at);
+            const int d = memcmp(value(a.at), value(b.at), (size_t)std::min(va, vb));
+            return d ? d < 0 : va < vb;
+        };
+        for (size_t i = 0, j; i < out.size(); i = j) {
+            for (j = i + 1; j < out.size() && out[j].prefix == out[i].prefix;) j++;
+            if (j > i + 1) std::sort(out.begin() + (int64_t)i, out.begin() + (int64_t)j, rest);
+        }
+    }
+
+    int grow(uint32_t **p, int64_t *have, int64_t words)
+    {
+        if (words <= *have) return PAT_OK;
+        if (*p) (void)pat::dev_free(*p);
+        *p = nullptr;
+        *have = 0;
+        if (pat::dev_malloc(p, sizeof(uint32_t) * (size_t)words) != hipSuccess) {
+            (void)hipGetLastError();
+            *p = nullptr;
+            pat::set_error("pat_regular_start: hipMalloc of %lld table bytes failed", (long long)(4 * words));
+            return PAT_ERR_NOMEM;
+        }
+        *have = words;
+        return PAT_OK;
+    }
+
     int start()
     {
         PAT_REQUIRE(table, PAT_ERR_STATE, "pat_regular_start: no application table (pat_regular_set_table)");
         const int64_t nb = buckets(), pw = pool_words();
         PAT_REQUIRE(nb <= (1 << 24) && pw < (1LL << 31), PAT_ERR_INVALID, "pat_regular_start: object too large");
-        waves = (int)std::min<int64_t>(kMaxWaves, std::max<int64_t>(1, (num_units + kUnitsPerWave - 1) / kUnitsPerWave));
-        const int64_t words = (nb + 1 + pw) * (waves + 1);
-        if (words > tables_words) {
-            if (tables) (void)pat::dev_free(tables);
-            tables = nullptr;
-            tables_words = 0;
-            if (pat::dev_malloc(&tables, sizeof(uint32_t) * (size_t)words) != hipSuccess) {
-                (void)hipGetLastError();
-                tables = nullptr;
-                pat::set_error("pat_regular_start: hipMalloc of %lld table bytes failed", (long long)(4 * words));
-                return PAT_ERR_NOMEM;
-            }
-            tables_words = words;
-        }
+        // a wavefront's words: its table, its column of the matrix, its count
+        const int64_t per_wave = 2 * nb + pw + 1;
+        const int64_t few = std::min<int64_t>(kMaxWavesFew, std::max<int64_t>(1, (num_units + kUnitsFew - 1) / kUnitsFew));
+        const int64_t fit = std::max(few, kTableWords / per_wave);
+        waves = (int)std::min<int64_t>(std::min<int64_t>(kMaxWaves, fit),
+                                       std::max<int64_t>(1, (num_units + kUnitsPerWave - 1) / kUnitsPerWave));
+        PAT_TRY(grow(&tables, &tables_words, (nb + pw) * waves + (waves + (waves & 1)) + 3 * nb));
+        if (nb * waves > matrix_words) matrix_clear = false;
+        PAT_TRY(grow(&matrix, &matrix_words, nb * waves));
+        PAT_TRY(grow(&final, &final_words, kStatusWords + pw));
         // LDS table: buckets a power of two covering lds_keys (or the
         // kernels' largest), pool words for that many records
         int lnb = table->max_lds_buckets, lpw = table->max_lds_pool_words;
@@ -100,24 +172,32 @@ struct pat_regular {
         o.unit_bytes = unit_bytes;
         o.num_units = num_units;
         o.param = param;
-        o.wave_tables = tables;
-        o.final_table = tables + (nb + 1 + pw) * waves;
-        o.status = status;
+        // the final buckets first: they are 8-byte words
+        o.final_buckets = (unsigned long long *)tables;
+        o.slots = (int32_t *)(tables + 2 * nb);
+        o.wave_counts = (int32_t *)(tables + 3 * nb);
+        o.wave_tables = tables + 3 * nb + (waves + (waves & 1));
+        o.matrix = matrix;
+        o.status = (int32_t *)final;
+        o.final_pool = final + kStatusWords;
         o.waves = waves;
         o.table_buckets = (int32_t)nb;
         o.table_pool_words = (int32_t)pw;
         o.lds_buckets = lnb;
         o.lds_pool_words = lpw;
-        PAT_HIP(hipMemsetAsync(status, 0, 4 * sizeof(int32_t), stream));
+        if (!matrix_clear) PAT_HIP(hipMemsetAsync(matrix, 0, sizeof(uint32_t) * (size_t)matrix_words, stream));
+        matrix_clear = false;  // until the run has ended well: its fold leaves the matrix clear
+        PAT_HIP(hipMemsetAsync(o.status, 0, kStatusWords * sizeof(int32_t), stream));
         const int rc = table->map_reduce(map_idx, reduce_idx, &o, stream);
         PAT_REQUIRE(rc == PAT_OK, rc, "pat_regular_start: the table's kernels for map %d / reduce %d failed (%d)",
                     map_idx, reduce_idx, rc);
-        int32_t st[4] = {0, 0, 0, 0};
-        PAT_HIP(hipMemcpyAsync(st, status, sizeof(st), hipMemcpyDeviceToHost, stream));
-        std::vector<uint32_t> fin((size_t)(nb + 1 + pw));
-        PAT_HIP(hipMemcpyAsync(fin.data(), o.final_table, sizeof(uint32_t) * fin.size(), hipMemcpyDeviceToHost,
+        const int64_t head = std::min(pw, kFirstWords);
+        PAT_HIP(hipMemcpyAsync(host, final, sizeof(uint32_t) * (size_t)(kStatusWords + head), hipMemcpyDeviceToHost,
                                stream));
         PAT_HIP(hipStreamSynchronize(stream));
+        matrix_clear = true;
+        int32_t st[kStatusWords];
+        memcpy(st, host, sizeof(st));
         PAT_REQUIRE(!(st[0] & 1), PAT_ERR_UNSUPPORTED,
                     "pat_regular_start: a wavefront met more keys than the object holds (%lld keys of %lld bytes; "
                     "pat_regular_set_capacity)", (long long)max_keys, (long long)max_record_bytes);
@@ -131,22 +211,29 @@ struct pat_regular {
                     (long long)max_keys, (long long)max_record_bytes);
         merges = st[1];
         reruns = st[2];
-        // decode the final table's records, sorted by key bytes
-        out.clear();
-        for (int64_t b = 0; b < nb; b++) {
-            const uint32_t s = fin[(size_t)b];
-            if (s == 0u) continue;
-            PAT_REQUIRE(s != 0xffffffffu && (int64_t)s - 1 < pw, PAT_ERR_INVALID,
-                        "pat_regular_start: damaged final table");
-            const uint32_t *r = fin.data() + nb + 1 + (s - 1u);
-            const int ks = (int)(r[0] >> 16), vs = (int)(r[0] & 0xffffu);
-            PAT_REQUIRE((int64_t)s - 1 + 1 + (ks + 3) / 4 + (vs + 3) / 4 <= pw, PAT_ERR_INVALID,
-                        "pat_regular_start: damaged final table record");
-            const char *kp = (const char *)(r + 1);
-            const char *vp = (const char *)(r + 1 + (ks + 3) / 4);
-            out.emplace_back(std::string(kp, (size_t)ks), std::string(vp, (size_t)vs));
+        const int64_t words = st[4];
+        PAT_REQUIRE(words >= 0 && words <= pw && st[3] >= 0 && st[3] <= nb, PAT_ERR_INVALID,
+                    "pat_regular_start: damaged final table");
+        records.resize((size_t)words);
+        memcpy(records.data(), host + kStatusWords, sizeof(uint32_t) * (size_t)std::min(words, head));
+        if (words > head) {
+            PAT_HIP(hipMemcpyAsync(records.data() + head, final + kStatusWords + head,
+                                   sizeof(uint32_t) * (size_t)(words - head), hipMemcpyDeviceToHost, stream));
+            PAT_HIP(hipStreamSynchronize(stream));
         }
-        std::sort(out.begin(), out.end());
+        // the records' places, sorted by key bytes (a prefix of a key first)
+        out.clear();
+        out.reserve((size_t)st[3]);
+        for (int64_t at = 0; at < words;) {
+            const int64_t need = record_words(records[(size_t)at]);
+            PAT_REQUIRE(at + need <= words, PAT_ERR_INVALID, "pat_regular_start: damaged final table record");
+            uint64_t prefix = 0;
+            const unsigned char *k = key((uint32_t)at);
+            for (int i = 0; i < 8; i++) prefix = prefix << 8 | (i < key_size((uint32_t)at) ? k[i] : 0);
+            out.push_back(Place{prefix, (uint32_t)at});
+            at += need;
+        }
+        sort_places();
         have_result = true;
         return PAT_OK;
     }
@@ -189,7 +276,13 @@ int pat_regular_create(const void *input, int64_t input_bytes, int64_t num_units
         }
     };
     am(&h->input, (size_t)input_bytes);
-    am((void **)&h->status, 4 * sizeof(int32_t));
+    if (rc == PAT_OK && hipHostMalloc((void **)&h->host, sizeof(uint32_t) * (size_t)(kStatusWords + kFirstWords),
+                                      hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        h->host = nullptr;
+        pat::set_error("pat_regular_create: pinned memory for the read-back failed");
+        rc = PAT_ERR_NOMEM;
+    }
     if (offsets) am((void **)&h->offsets, sizeof(int64_t) * (size_t)num_units);
     if (rc == PAT_OK &&
         (hipMemcpyAsync(h->input, input, (size_t)input_bytes, hipMemcpyHostToDevice, h->stream) != hipSuccess ||
@@ -289,26 +382,22 @@ int pat_regular_get_output(pat_regular *h, int64_t *num_keys, int64_t *key_bytes
 {
     PAT_REQUIRE(h && num_keys, PAT_ERR_INVALID, "pat_regular_get_output: null argument");
     PAT_REQUIRE(h->have_result, PAT_ERR_STATE, "pat_regular_get_output: no result (pat_regular_start)");
-    int64_t kb = 0, vb = 0;
-    for (const auto &e : h->out) {
-        kb += (int64_t)e.first.size();
-        vb += (int64_t)e.second.size();
-    }
-    *num_keys = (int64_t)h->out.size();
-    if (key_bytes) *key_bytes = kb;
-    if (val_bytes) *val_bytes = vb;
     int64_t ko = 0, vo = 0, i = 0;
     for (const auto &e : h->out) {
-        if (keys) memcpy((char *)keys + ko, e.first.data(), e.first.size());
-        if (vals) memcpy((char *)vals + vo, e.second.data(), e.second.size());
+        const int ks = h->key_size(e.at), vs = h->value_size(e.at);
+        if (keys) memcpy((char *)keys + ko, h->key(e.at), (size_t)ks);
+        if (vals) memcpy((char *)vals + vo, h->value(e.at), (size_t)vs);
         if (key_index) key_index[i] = (uint32_t)ko;
         if (val_index) val_index[i] = (uint32_t)vo;
-        if (key_size) key_size[i] = (uint32_t)e.first.size();
-        if (val_size) val_size[i] = (uint32_t)e.second.size();
-        ko += (int64_t)e.first.size();
-        vo += (int64_t)e.second.size();
+        if (key_size) key_size[i] = (uint32_t)ks;
+        if (val_size) val_size[i] = (uint32_t)vs;
+        ko += ks;
+        vo += vs;
         i++;
     }
+    *num_keys = i;
+    if (key_bytes) *key_bytes = ko;
+    if (val_bytes) *val_bytes = vo;
     return PAT_OK;
 }
 

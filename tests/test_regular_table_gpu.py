@@ -144,3 +144,49 @@ def test_capacity_errors(pa, gpu, tab):
     with pytest.raises(pa.PatternError, match="not in the table"):
         pa.call("pat_regular_set_map_idx", r.h, 5)
     r.close()
+
+
+def keyed_by_hand(v, m):
+    """{key bytes: value bytes} of apps/keys' functor m over the values v."""
+    want = {}
+
+    def add(key, value):
+        key = np.array(key, np.uint32).tobytes()
+        want[key] = want[key] + value if key in want else np.array(value, np.uint32)
+
+    for x in v.tolist():
+        r = np.uint32(x % 1000)
+        if m == 0:
+            add([x % 601, 7, x % 601 // 3], np.array([1, r], np.uint32))
+        elif m == 1:
+            k = x % 97
+            add([k, 5] if k % 2 else [k], np.full(1 + k % 3, r, np.uint32))
+        elif m == 2:
+            add([x % 33], r + np.arange(20, dtype=np.uint32))
+        else:
+            add([x % 50], np.ones(1, np.uint32))
+            add([50 + x % 7], np.ones(1, np.uint32))
+    return {k: a.astype(np.uint32).tobytes() for k, a in want.items()}
+
+
+@pytest.mark.parametrize("m", [0, 1, 2, 3])
+@pytest.mark.parametrize("n", [1, 63, 65, 257, 5000, 70001])
+@pytest.mark.parametrize("lds_keys", [0, 5])
+def test_key_and_value_forms(pa, gpu, m, n, lds_keys):
+    """Keys beyond eight bytes (placed in turn), keys and values of several
+    sizes in one wavefront, values folded in place, two inserts per unit; one
+    partial wavefront, runs and wavefronts with a remainder.  Whole numbers:
+    the same bytes as a serial reduction.  With 5 keys per LDS table a unit of
+    two inserts can lose the second: that is refused."""
+    v = np.random.default_rng(n + m).integers(0, 2 ** 31, n, dtype=np.uint32)
+    r = pa.Regular(v, n, 4, table=pa.app_table("keys", "gr"))
+    r.set_capacity(1024, 96, lds_keys)
+    if m == 3 and lds_keys and n > 1:
+        with pytest.raises(pa.PatternError, match="inserting twice"):
+            r.run(m, reduce_idx=0)
+    else:
+        want = keyed_by_hand(v, m)
+        assert r.run(m, reduce_idx=0) == want
+        r.set_capacity(2048, 96, lds_keys)  # another geometry on the same buffers
+        assert r.run(m, reduce_idx=0) == want
+    r.close()
