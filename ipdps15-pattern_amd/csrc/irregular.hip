@@ -54,22 +54,7 @@ __global__ void fill_i32(int *__restrict__ p, int64_t n, int v)
         p[i] = v;
 }
 
-__global__ void copy_i32(int *__restrict__ dst, const int *__restrict__ src, int64_t n)
-{
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        dst[i] = src[i];
-}
-
 static unsigned grid_for(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256 + 1, 4096); }
-
-__global__ void csr_degree(const int2 *__restrict__ edges, int64_t E, int *__restrict__ deg)
-{
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E; e += (int64_t)gridDim.x * blockDim.x) {
-        int2 ij = edges[e];
-        atomicAdd(&deg[ij.x], 1);
-        atomicAdd(&deg[ij.y], 1);
-    }
-}
 
 constexpr int kScanBlock = 1024;
 
@@ -108,39 +93,6 @@ __global__ __launch_bounds__(kScanBlock) void scan_add(int *__restrict__ out, in
 {
     const int64_t g = (int64_t)blockIdx.x * kScanBlock + threadIdx.x;
     if (g < n) out[g] += offs[blockIdx.x];
-}
-
-__global__ void csr_scatter(const int2 *__restrict__ edges, int64_t E, int *__restrict__ cursor, int *__restrict__ tmp,
-                            int *__restrict__ tmpe)
-{
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E; e += (int64_t)gridDim.x * blockDim.x) {
-        int2 ij = edges[e];
-        int p = atomicAdd(&cursor[ij.x], 1);
-        tmp[p] = ij.y;
-        tmpe[p] = (int)e;
-        int q = atomicAdd(&cursor[ij.y], 1);
-        tmp[q] = ij.x;
-        tmpe[q] = (int)e;
-    }
-}
-
-// One wavefront per row: places each entry at the rank of its edge id, so a
-// row lists its neighbours in the order their edges appear in the input list
-// -- the order in which a serial scatter over that list adds them.
-__global__ __launch_bounds__(256) void csr_row_sort_by_edge(const int *__restrict__ rowptr, int64_t N,
-                                                            const int *__restrict__ tmp, const int *__restrict__ tmpe,
-                                                            int *__restrict__ cols)
-{
-    const int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int lane = threadIdx.x % kWave;
-    if (row >= N) return;
-    const int b = rowptr[row], e = rowptr[row + 1];
-    for (int k = b + lane; k < e; k += kWave) {
-        const int v = tmpe[k];
-        int rank = 0;
-        for (int m = b; m < e; m++) rank += tmpe[m] < v;
-        cols[b + rank] = tmp[k];
-    }
 }
 
 // Value held by lane ^ M (M < 64), by the cheapest cross-lane form: DPP
@@ -207,6 +159,45 @@ __device__ __forceinline__ void sort_merge(unsigned (&a)[2 * kSortRows], int lan
     sort_half_clean<K / 4>(a, lane);
 }
 
+// sort_merge for rows of at most 64 columns: value 0 of each lane only.
+template <int J>
+__device__ __forceinline__ void sort_half_clean64(unsigned (&a)[2 * kSortRows], int lane)
+{
+    if constexpr (J >= 1) {
+        sort_cx<J, J>(a, 0, lane);
+        sort_half_clean64<J / 2>(a, lane);
+    }
+}
+
+template <int K>
+__device__ __forceinline__ void sort_merge64(unsigned (&a)[2 * kSortRows], int lane)
+{
+    sort_cx<K - 1, K / 2>(a, 0, lane);
+    sort_half_clean64<K / 4>(a, lane);
+}
+
+// The lanes' values a[2t] (entry lane of row t) and, when wide, a[2t + 1]
+// (entry 64 + lane) sorted row by row.
+__device__ __forceinline__ void sort_rows(unsigned (&a)[2 * kSortRows], bool wide, int lane)
+{
+    if (wide) {
+        sort_merge<2>(a, lane);
+        sort_merge<4>(a, lane);
+        sort_merge<8>(a, lane);
+        sort_merge<16>(a, lane);
+        sort_merge<32>(a, lane);
+        sort_merge<64>(a, lane);
+        sort_merge<128>(a, lane);
+    } else {
+        sort_merge64<2>(a, lane);
+        sort_merge64<4>(a, lane);
+        sort_merge64<8>(a, lane);
+        sort_merge64<16>(a, lane);
+        sort_merge64<32>(a, lane);
+        sort_merge64<64>(a, lane);
+    }
+}
+
 // kSortRows rows per wavefront, each row of at most 128 columns sorted by
 // the bitonic network held two values per lane (padding sorts last); the
 // rows' pointers and values are all loaded before the networks run, which
@@ -234,13 +225,10 @@ __global__ __launch_bounds__(256) void csr_row_sort(const int *__restrict__ rowp
         a[2 * t] = lane < m ? (unsigned)src[lane] : 0xffffffffu;
         a[2 * t + 1] = kWave + lane < m ? (unsigned)src[kWave + lane] : 0xffffffffu;
     }
-    sort_merge<2>(a, lane);
-    sort_merge<4>(a, lane);
-    sort_merge<8>(a, lane);
-    sort_merge<16>(a, lane);
-    sort_merge<32>(a, lane);
-    sort_merge<64>(a, lane);
-    sort_merge<128>(a, lane);
+    bool wide = false;  // uniform per wavefront
+#pragma unroll
+    for (int t = 0; t < kSortRows; t++) wide |= n[t] > kWave;
+    sort_rows(a, wide, lane);
 #pragma unroll
     for (int t = 0; t < kSortRows; t++) {
         if (n[t] > 2 * kWave) {  // uniform per wavefront
@@ -265,6 +253,275 @@ __global__ __launch_bounds__(256) void csr_row_sort(const int *__restrict__ rowp
 static inline unsigned row_sort_grid(int64_t N)
 {
     return (unsigned)(((N + kSortRows - 1) / kSortRows * kWave + 255) / 256);
+}
+
+// ------------------------------------------------------------ CSR build
+//
+// Two passes over the edge list and one over its entries, in place of a
+// degree histogram and a scatter by one returning atomic per entry into
+// global memory (13.3 M entries of 256,000 rows: 0.50 + 1.14 of 1.6 ms, bound
+// by the atomics; 0.27 ms now, csr_scatter 0.13 of it, bound by its partial
+// lines).  Rows are grouped into buckets of 2^shift; csr_count counts
+// each workgroup's entries per bucket in LDS and reserves its part of every
+// bucket with one atomic; csr_scatter writes the entries there, so a bucket
+// gets runs of neighbouring 8-byte words; csr_rows takes a bucket into LDS,
+// counts and places its rows, sorts them and writes row pointers and columns.
+//
+// Entry: the row within the bucket << 32 | a 32-bit key that orders the row:
+// the neighbour (rows in node order) or the place 2 e + side of this endpoint
+// in the list (edge order: the neighbour is read from the list at the end, so
+// that one word is enough).
+
+enum CsrOut { kCsrEdgeOrder = 0, kCsrNodeOrder = 1, kCsrEdgeIds = 2 };
+
+constexpr int kCsrThreads = 512;
+constexpr int kCsrMaxBuckets = 8192;   // counted in LDS: 32 KB
+constexpr int kCsrCap = 10240;         // entries of a group of rows held in LDS (40 KB)
+constexpr int kCsrRows = 2048;         // rows counted in LDS at a time (8 KB): three workgroups per CU
+
+// Edges [c0, c1) of workgroup blockIdx.x, four in flight per thread: f(edge
+// id, edge).
+template <typename F>
+__device__ __forceinline__ void csr_edges(const int2 *__restrict__ edges, int64_t E, int64_t chunk, F f)
+{
+    const int64_t c0 = (int64_t)blockIdx.x * chunk, c1 = min(c0 + chunk, E);
+    int64_t e = c0 + threadIdx.x;
+    for (; e + 3 * kCsrThreads < c1; e += 4 * kCsrThreads) {
+        const int2 v0 = edges[e], v1 = edges[e + kCsrThreads], v2 = edges[e + 2 * kCsrThreads],
+                   v3 = edges[e + 3 * kCsrThreads];
+        f(e, v0);
+        f(e + kCsrThreads, v1);
+        f(e + 2 * kCsrThreads, v2);
+        f(e + 3 * kCsrThreads, v3);
+    }
+    for (; e < c1; e += kCsrThreads) f(e, edges[e]);
+}
+
+// part[b * wgs + workgroup] = where this workgroup's entries of bucket b start
+// within the bucket; total[b] += their number.
+__global__ __launch_bounds__(kCsrThreads) void csr_count(const int2 *__restrict__ edges, int64_t E, int64_t chunk,
+                                                         int shift, int B, int *__restrict__ total,
+                                                         int *__restrict__ part)
+{
+    __shared__ int h[kCsrMaxBuckets];
+    for (int b = threadIdx.x; b < B; b += kCsrThreads) h[b] = 0;
+    __syncthreads();
+    csr_edges(edges, E, chunk, [&](int64_t, int2 ij) {
+        atomicAdd(&h[ij.x >> shift], 1);
+        atomicAdd(&h[ij.y >> shift], 1);
+    });
+    __syncthreads();
+    for (int b = threadIdx.x; b < B; b += kCsrThreads)
+        part[(int64_t)blockIdx.x * B + b] = h[b] ? atomicAdd(&total[b], h[b]) : 0;
+}
+
+// start[0..B]: exclusive sums of total[0..B) (one workgroup of kScanBlock
+// threads).
+__global__ __launch_bounds__(kScanBlock) void csr_starts(const int *__restrict__ total, int B, int *__restrict__ start)
+{
+    __shared__ int sums[kScanBlock];
+    const int per = (B + kScanBlock - 1) / kScanBlock;
+    const int b0 = min(B, (int)threadIdx.x * per), b1 = min(B, b0 + per);
+    int sum = 0;
+    for (int b = b0; b < b1; b++) sum += total[b];
+    sums[threadIdx.x] = sum;
+    __syncthreads();
+    for (int d = 1; d < kScanBlock; d <<= 1) {
+        const int v = (int)threadIdx.x >= d ? sums[threadIdx.x - d] : 0;
+        __syncthreads();
+        sums[threadIdx.x] += v;
+        __syncthreads();
+    }
+    int run = sums[threadIdx.x] - sum;
+    for (int b = b0; b < b1; b++) {
+        start[b] = run;
+        run += total[b];
+    }
+    if (threadIdx.x == kScanBlock - 1) start[B] = sums[kScanBlock - 1];
+}
+
+__global__ __launch_bounds__(kCsrThreads) void csr_scatter(const int2 *__restrict__ edges, int64_t E, int64_t chunk,
+                                                           int shift, int B, const int *__restrict__ start,
+                                                           const int *__restrict__ part, int node_order,
+                                                           unsigned long long *__restrict__ ent)
+{
+    __shared__ int cur[kCsrMaxBuckets];
+    for (int b = threadIdx.x; b < B; b += kCsrThreads) cur[b] = start[b] + part[(int64_t)blockIdx.x * B + b];
+    __syncthreads();
+    const int low = (1 << shift) - 1;
+    csr_edges(edges, E, chunk, [&](int64_t e, int2 ij) {
+        const unsigned ki = node_order ? (unsigned)ij.y : 2u * (unsigned)e;
+        const unsigned kj = node_order ? (unsigned)ij.x : 2u * (unsigned)e + 1u;
+        const int p = atomicAdd(&cur[ij.x >> shift], 1);
+        const int q = atomicAdd(&cur[ij.y >> shift], 1);
+        ent[p] = (unsigned long long)(unsigned)(ij.x & low) << 32 | ki;
+        ent[q] = (unsigned long long)(unsigned)(ij.y & low) << 32 | kj;
+    });
+}
+
+// One workgroup per bucket.  Its rows are counted kCsrRows at a time and
+// taken into LDS in groups of rows of at most kCsrCap entries (usually the
+// whole bucket at once; further groups read the bucket's entries again).
+// Rows of at most 128 entries are sorted in registers, four per wavefront;
+// longer ones by the workgroup in LDS; a row beyond kCsrCap by ranks.
+template <int OUT>
+__global__ __launch_bounds__(kCsrThreads) void csr_rows(const unsigned long long *__restrict__ ent,
+                                                        const int *__restrict__ start, int64_t N, int shift,
+                                                        const int *__restrict__ flat, int *__restrict__ rowptr,
+                                                        int *__restrict__ cols)
+{
+    __shared__ unsigned buf[kCsrCap];
+    __shared__ int cnt[kCsrRows];  // a row's entries, then the place of its next entry
+    __shared__ int wsum[kCsrThreads / kWave], carry;
+    const int t = (int)threadIdx.x, lane = t % kWave, wv = pat::wave_in_block();
+    const int s = start[blockIdx.x], e = start[blockIdx.x + 1];
+    const int64_t r0 = (int64_t)blockIdx.x << shift;
+    const int rows = (int)min((int64_t)1 << shift, N - r0);
+    auto out = [&](unsigned key) {
+        return OUT == kCsrNodeOrder ? (int)key : (OUT == kCsrEdgeOrder ? flat[key ^ 1u] : (int)(key >> 1));
+    };
+    // entries of rows [w, w + n) of the bucket, four in flight per thread
+    auto entries = [&](int w, int n, auto f) {
+        int i = s + t;
+        for (; i + 3 * kCsrThreads < e; i += 4 * kCsrThreads) {
+            unsigned long long v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = ent[i + u * kCsrThreads];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int r = (int)(v[u] >> 32) - w;
+                if (r >= 0 && r < n) f(r, (unsigned)v[u], i + u * kCsrThreads);
+            }
+        }
+        for (; i < e; i += kCsrThreads) {
+            const unsigned long long v = ent[i];
+            const int r = (int)(v >> 32) - w;
+            if (r >= 0 && r < n) f(r, (unsigned)v, i);
+        }
+    };
+    int base = s;  // place of the window's first entry
+    for (int w = 0; w < rows; w += kCsrRows) {
+        const int nr = min(kCsrRows, rows - w);
+        for (int r = t; r < kCsrRows; r += kCsrThreads) cnt[r] = 0;
+        __syncthreads();
+        entries(w, nr, [&](int r, unsigned, int) { atomicAdd(&cnt[r], 1); });
+        __syncthreads();
+        // cnt = the rows' places (exclusive sums from base), and rowptr
+        constexpr int PER = kCsrRows / kCsrThreads;
+        int c[PER], mine = 0;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            c[k] = cnt[t * PER + k];
+            mine += c[k];
+        }
+        int x = mine;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int y = __shfl_up(x, o, kWave);
+            if (lane >= o) x += y;
+        }
+        if (lane == kWave - 1) wsum[wv] = x;
+        __syncthreads();
+        int at = base + x - mine;
+        for (int v = 0; v < wv; v++) at += wsum[v];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int r = t * PER + k;
+            cnt[r] = at;
+            if (r < nr) rowptr[r0 + w + r] = at;
+            at += c[k];
+        }
+        if (t == kCsrThreads - 1) carry = at;
+        __syncthreads();
+        const int wend = carry;  // place after the window's last entry
+        // groups of rows [g, ge); cnt[g] is row g's place until its entries move it
+        for (int g = 0; g < nr;) {
+            const int gs = cnt[g];
+            int ge = nr;
+            if (wend - gs > kCsrCap) {  // the last row end within kCsrCap entries, at least one row
+                int lo = g + 1, hi = nr;
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if ((mid == nr ? wend : cnt[mid]) - gs <= kCsrCap) lo = mid;
+                    else hi = mid - 1;
+                }
+                ge = lo;
+            }
+            const int gend = ge == nr ? wend : cnt[ge];
+            __syncthreads();  // every thread has read the bounds
+            if (gend - gs > kCsrCap) {  // one row beyond LDS: each entry to its rank
+                entries(w + g, 1, [&](int, unsigned key, int i) {
+                    int rank = 0;
+                    for (int j = s; j < e; j++) {
+                        const unsigned long long v = ent[j];
+                        rank += (int)(v >> 32) == w + g && ((unsigned)v < key || ((unsigned)v == key && j < i));
+                    }
+                    cols[gs + rank] = out(key);
+                });
+                g = ge;
+                continue;
+            }
+            entries(w + g, ge - g, [&](int r, unsigned key, int) { buf[atomicAdd(&cnt[g + r], 1) - gs] = key; });
+            __syncthreads();
+            // now cnt[r] is the end of row r, and the start of row r + 1
+            bool any_long = false;
+            for (int q0 = g + wv * kSortRows; q0 < ge; q0 += kCsrThreads / kWave * kSortRows) {
+                int b[kSortRows], n[kSortRows];
+                unsigned a[2 * kSortRows];
+                bool wide = false;
+#pragma unroll
+                for (int u = 0; u < kSortRows; u++) {
+                    const int q = q0 + u;
+                    b[u] = q >= ge ? gs : (q == g ? gs : cnt[q - 1]);
+                    n[u] = q >= ge ? 0 : cnt[q] - b[u];
+                    if (n[u] > 2 * kWave) {
+                        any_long = true;
+                        n[u] = 0;
+                    }
+                    wide |= n[u] > kWave;
+                    a[2 * u] = lane < n[u] ? buf[b[u] - gs + lane] : 0xffffffffu;
+                    a[2 * u + 1] = kWave + lane < n[u] ? buf[b[u] - gs + kWave + lane] : 0xffffffffu;
+                }
+                sort_rows(a, __any(wide), lane);
+#pragma unroll
+                for (int u = 0; u < kSortRows; u++) {
+                    if (lane < n[u]) cols[b[u] + lane] = out(a[2 * u]);
+                    if (kWave + lane < n[u]) cols[b[u] + kWave + lane] = out(a[2 * u + 1]);
+                }
+            }
+            // longer rows: the bitonic network in its flip form over LDS
+            // (every comparison ascending; places past the row's end hold
+            // the largest value, so a comparison with one moves nothing)
+            if (__syncthreads_or(any_long))
+                for (int q = g; q < ge; q++) {
+                    const int qb = q == g ? gs : cnt[q - 1], n = cnt[q] - qb;
+                    if (n <= 2 * kWave) continue;  // uniform
+                    unsigned *v = buf + (qb - gs);
+                    auto cx = [&](int i, int j) {
+                        if (j < n && v[i] > v[j]) {
+                            const unsigned y = v[i];
+                            v[i] = v[j];
+                            v[j] = y;
+                        }
+                    };
+                    for (int k = 2; k < 2 * n; k <<= 1) {
+                        for (int p = t; p < n; p += kCsrThreads)
+                            if (!(p & (k >> 1))) cx(p, p ^ (k - 1));
+                        __syncthreads();
+                        for (int j = k >> 2; j > 0; j >>= 1) {
+                            for (int p = t; p < n; p += kCsrThreads)
+                                if (!(p & j)) cx(p, p ^ j);
+                            __syncthreads();
+                        }
+                    }
+                    for (int p = t; p < n; p += kCsrThreads) cols[qb + p] = out(v[p]);
+                }
+            __syncthreads();  // buf and cnt are free
+            g = ge;
+        }
+        base = wend;
+    }
+    if (blockIdx.x == gridDim.x - 1 && t == 0) rowptr[N] = e;
 }
 
 // ------------------------------------------------------------ neighbour build
@@ -1750,38 +2007,72 @@ static int scan_exclusive(const int *in, int *out, int64_t n, int *ws, hipStream
     return PAT_OK;
 }
 
+// The bucket build (csr_count .. csr_rows).  out: a CsrOut.
+static int csr_buckets(const char *who, const int32_t *edges, int64_t E, int64_t N, int out, int32_t *rowptr,
+                       int32_t *cols, void *work, int64_t work_bytes, hipStream_t st)
+{
+    PAT_REQUIRE(N > 0 && N < (1LL << 31) - 1 && E >= 0 && 2 * E < (1LL << 31), PAT_ERR_INVALID,
+                "%s: sizes out of range (N=%lld, E=%lld)", who, (long long)N, (long long)E);
+    PAT_REQUIRE(work_bytes >= csr_workspace_bytes(N, E), PAT_ERR_INVALID, "%s: workspace too small", who);
+    if (E == 0) {
+        hipLaunchKernelGGL(fill_i32, dim3(grid_for(N + 1)), dim3(256), 0, st, rowptr, N + 1, 0);
+        PAT_LAUNCH_CHECK();
+        return PAT_OK;
+    }
+    // Rows per bucket: as many as hold about 8,192 entries, so that most
+    // buckets fit LDS, or fewer where that gives the chip less than 1,024
+    // buckets to work on (down to 512 entries, below which a bucket's fixed
+    // work outweighs its rows), and no more than csr_rows counts at a time --
+    // but with no more buckets than a workgroup counts in LDS.
+    const int64_t want = std::max<int64_t>(512, std::min<int64_t>(8192, 2 * E / 1024));
+    int shift = 0;
+    while (((2LL << shift) <= kCsrRows && (2LL << shift) * 2 * E <= want * N) ||
+           ((N - 1) >> shift) + 1 > kCsrMaxBuckets)
+        shift++;
+    const int B = (int)(((N - 1) >> shift) + 1);
+    // Edges per workgroup: enough for runs of several entries per bucket, and
+    // about 400 workgroups where the list is that long.  The totals (B) and
+    // the workgroups' parts (wgs x B) lie behind the starts (B + 1) where the
+    // N + 1 words hold them, else in cols (2 E words) until csr_rows writes
+    // it; one of the two holds them at the latest with one workgroup, since
+    // buckets of fewer than four rows mean over 64 entries per row.
+    int64_t chunk = std::max<int64_t>(2048, std::min<int64_t>(16384, (E + 399) / 400));
+    int64_t wgs = (E + chunk - 1) / chunk;
+    auto beside = [&] { return (wgs + 2) * B <= N; };
+    while (wgs > 1 && !beside() && (wgs + 1) * B > 2 * E) {
+        chunk *= 2;
+        wgs = (E + chunk - 1) / chunk;
+    }
+    PAT_REQUIRE(beside() || (wgs + 1) * B <= 2 * E, PAT_ERR_STATE, "%s: no room for the bucket counts", who);
+    int *start = (int *)work, *total = beside() ? start + B + 1 : cols, *part = total + B;
+    // the entries: 2 E eight-byte words behind the N + 1 words (rounded up to
+    // 16 bytes within the work space's 256 spare ones)
+    auto *ent = (unsigned long long *)(((uintptr_t)work + sizeof(int) * (size_t)(N + 1) + 15) & ~(uintptr_t)15);
+    const int2 *e2 = (const int2 *)edges;
+    hipLaunchKernelGGL(fill_i32, dim3(grid_for(B)), dim3(256), 0, st, total, (int64_t)B, 0);
+    PAT_LAUNCH_CHECK();
+    hipLaunchKernelGGL(csr_count, dim3((unsigned)wgs), dim3(kCsrThreads), 0, st, e2, E, chunk, shift, B, total, part);
+    PAT_LAUNCH_CHECK();
+    hipLaunchKernelGGL(csr_starts, dim3(1), dim3(kScanBlock), 0, st, (const int *)total, B, start);
+    PAT_LAUNCH_CHECK();
+    hipLaunchKernelGGL(csr_scatter, dim3((unsigned)wgs), dim3(kCsrThreads), 0, st, e2, E, chunk, shift, B,
+                       (const int *)start, (const int *)part, out == kCsrNodeOrder, ent);
+    PAT_LAUNCH_CHECK();
+    auto k = out == kCsrNodeOrder ? csr_rows<kCsrNodeOrder>
+                                  : (out == kCsrEdgeOrder ? csr_rows<kCsrEdgeOrder> : csr_rows<kCsrEdgeIds>);
+    hipLaunchKernelGGL(k, dim3((unsigned)B), dim3(kCsrThreads), 0, st, (const unsigned long long *)ent,
+                       (const int *)start, N, shift, (const int *)edges, rowptr, cols);
+    PAT_LAUNCH_CHECK();
+    return PAT_OK;
+}
+
 // The edge ids of the CSR by destination (row r: every edge with r as an
 // endpoint, in increasing edge id -- the serial scatter's order for r);
 // rowptr as csr_build writes it.  Same workspace as csr_build.
 int csr_edge_ids(const int32_t *edges, int64_t E, int64_t N, int32_t *rowptr, int32_t *eids, void *work,
                  int64_t work_bytes, hipStream_t st)
 {
-    PAT_REQUIRE(N > 0 && N < (1LL << 31) - 1 && E >= 0 && 2 * E < (1LL << 31), PAT_ERR_INVALID,
-                "csr_edge_ids: sizes out of range (N=%lld, E=%lld)", (long long)N, (long long)E);
-    PAT_REQUIRE(work_bytes >= csr_workspace_bytes(N, E), PAT_ERR_INVALID, "csr_edge_ids: workspace too small");
-    const int64_t nb = (N + 1 + kScanBlock - 1) / kScanBlock;
-    int *deg = (int *)work;
-    int *ws = deg + (N + 1);
-    int *tmp = ws + 2 * nb + 2 * ((nb + kScanBlock - 1) / kScanBlock) + 2;
-    hipLaunchKernelGGL(fill_i32, dim3(grid_for(N + 1)), dim3(256), 0, st, deg, N + 1, 0);
-    PAT_LAUNCH_CHECK();
-    const unsigned grid = (unsigned)std::min<int64_t>((E + 255) / 256 + 1, 65536);
-    if (E > 0) {
-        hipLaunchKernelGGL(csr_degree, dim3(grid), dim3(256), 0, st, (const int2 *)edges, E, deg);
-        PAT_LAUNCH_CHECK();
-    }
-    PAT_TRY(scan_exclusive(deg, rowptr, N + 1, ws, st));
-    hipLaunchKernelGGL(copy_i32, dim3(grid_for(N + 1)), dim3(256), 0, st, deg, (const int *)rowptr, N + 1);
-    PAT_LAUNCH_CHECK();
-    if (E > 0) {
-        int *tmpe = tmp + 2 * E;
-        hipLaunchKernelGGL(csr_scatter, dim3(grid), dim3(256), 0, st, (const int2 *)edges, E, deg, tmp, tmpe);
-        PAT_LAUNCH_CHECK();
-        const unsigned g2 = (unsigned)((N * kWave + 255) / 256);
-        hipLaunchKernelGGL(csr_row_sort_by_edge, dim3(g2), dim3(256), 0, st, rowptr, N, tmpe, tmpe, eids);
-        PAT_LAUNCH_CHECK();
-    }
-    return PAT_OK;
+    return csr_buckets("csr_edge_ids", edges, E, N, kCsrEdgeIds, rowptr, eids, work, work_bytes, st);
 }
 
 // order 0: rows in edge-list order; 1: rows sorted by neighbour index.
@@ -1789,36 +2080,8 @@ int csr_build(const int32_t *edges, int64_t E, int64_t N, int order, int32_t *ro
               int64_t work_bytes, hipStream_t st)
 {
     PAT_REQUIRE(order == 0 || order == 1, PAT_ERR_INVALID, "csr_build: row order %d not in {0, 1}", order);
-    PAT_REQUIRE(N > 0 && N < (1LL << 31) - 1 && E >= 0 && 2 * E < (1LL << 31), PAT_ERR_INVALID,
-                "csr_build: sizes out of range (N=%lld, E=%lld)", (long long)N, (long long)E);
-    PAT_REQUIRE(work_bytes >= csr_workspace_bytes(N, E), PAT_ERR_INVALID, "csr_build: workspace too small");
-    const int64_t nb = (N + 1 + kScanBlock - 1) / kScanBlock;
-    int *deg = (int *)work;
-    int *ws = deg + (N + 1);
-    int *tmp = ws + 2 * nb + 2 * ((nb + kScanBlock - 1) / kScanBlock) + 2;
-    hipLaunchKernelGGL(fill_i32, dim3(grid_for(N + 1)), dim3(256), 0, st, deg, N + 1, 0);
-    PAT_LAUNCH_CHECK();
-    const unsigned grid = (unsigned)std::min<int64_t>((E + 255) / 256 + 1, 65536);
-    if (E > 0) {
-        hipLaunchKernelGGL(csr_degree, dim3(grid), dim3(256), 0, st, (const int2 *)edges, E, deg);
-        PAT_LAUNCH_CHECK();
-    }
-    PAT_TRY(scan_exclusive(deg, rowptr, N + 1, ws, st));
-    // cursor = rowptr (reuse deg)
-    hipLaunchKernelGGL(copy_i32, dim3(grid_for(N + 1)), dim3(256), 0, st, deg, (const int *)rowptr, N + 1);
-    PAT_LAUNCH_CHECK();
-    if (E > 0) {
-        int *tmpe = tmp + 2 * E;
-        hipLaunchKernelGGL(csr_scatter, dim3(grid), dim3(256), 0, st, (const int2 *)edges, E, deg, tmp, tmpe);
-        PAT_LAUNCH_CHECK();
-        const unsigned g2 = (unsigned)((N * kWave + 255) / 256);
-        if (order == 0)
-            hipLaunchKernelGGL(csr_row_sort_by_edge, dim3(g2), dim3(256), 0, st, rowptr, N, tmp, tmpe, cols);
-        else
-            hipLaunchKernelGGL(csr_row_sort, dim3(row_sort_grid(N)), dim3(256), 0, st, rowptr, N, tmp, cols, 0);
-        PAT_LAUNCH_CHECK();
-    }
-    return PAT_OK;
+    return csr_buckets("csr_build", edges, E, N, order == 0 ? kCsrEdgeOrder : kCsrNodeOrder, rowptr, cols, work,
+                       work_bytes, st);
 }
 
 using CsrKernel = void (*)(const float4 *, const int *, const int *, int, LJParams, float4 *, float4 *, float4 *, int);

@@ -84,6 +84,44 @@ def test_csr_build_edge_cases(pa, gpu):
     assert rp[251] - rp[250] == 0
 
 
+def csr_list(kind):
+    """(num_nodes, edges) of the forms that take different ways through the
+    bucket build."""
+    rng = np.random.default_rng(31)
+    if kind == "two nodes":
+        return 2, np.array([[0, 1], [1, 0], [0, 1]])
+    if kind == "one edge, many nodes":  # counts beside the starts, row windows without entries
+        return 100003, np.array([[99998, 3]])
+    if kind == "rows in windows":  # more nodes than 8,192 buckets of 2,048 rows hold
+        return 8192 * 2048 + 77, rng.integers(0, 8192 * 2048 + 77, (5000, 2))
+    if kind == "short and long rows":  # 64, 65, 128, 129, 130 and 1,000 entries among empty ones
+        deg = {10: 64, 11: 65, 500: 128, 501: 129, 502: 130, 2047: 1000}
+        return 5000, np.concatenate([np.stack([np.full(d, r), 3000 + rng.permutation(1990)[:d]], 1)
+                                     for r, d in deg.items()])
+    if kind == "hubs":  # one row beyond LDS, groups of rows beyond it in one bucket
+        e = [np.stack([np.full(11000, 5), rng.integers(6, 600, 11000)], 1)]
+        e += [np.stack([np.full(3000, r), rng.integers(100, 600, 3000)], 1) for r in (6, 7, 8, 20, 21)]
+        return 600, np.concatenate(e)
+    if kind == "dense":  # duplicates, buckets of one row
+        return 40, rng.integers(0, 40, (60000, 2))
+    return 30011, rng.integers(0, 30011, (400000, 2))  # ragged: B, chunks and rows with remainders
+
+
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("kind", ["two nodes", "one edge, many nodes", "rows in windows", "short and long rows", "hubs",
+                                  "dense", "ragged"])
+def test_csr_build_forms(pa, gpu, kind, order):
+    n, edges = csr_list(kind)
+    edges = edges[edges[:, 0] != edges[:, 1]]
+    edges = np.ascontiguousarray(np.random.default_rng(5).permutation(edges), dtype=np.int32)
+    rowptr, cols = pa.csr_build_dev(pa.DeviceArray.from_numpy(edges), len(edges), n, order=order)
+    both = np.concatenate([edges, edges[:, ::-1]])
+    eid = np.concatenate([np.arange(len(edges))] * 2)
+    both = both[np.lexsort((both[:, 1] if order else eid, both[:, 0]))]
+    assert np.array_equal(rowptr.numpy(), np.concatenate([[0], np.cumsum(np.bincount(both[:, 0], minlength=n))]))
+    assert np.array_equal(cols.numpy(), both[:, 1])
+
+
 @pytest.mark.parametrize("lpr", [1, 4, 8, 16, 32, -4, -8, -16, -32, -64])
 def test_force_csr_vs_oracle(pa, orc, gpu, small, lpr):
     pos, box, edges = small
