@@ -27,23 +27,17 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "pat_common.hpp"
+#include "pat_device.hpp"
 #include "stencil_dev.hpp"
 
 namespace {
 
-constexpr int kXcds = 8;
-
-// Maps a hardware workgroup id to a tile id so that the tiles one XCD gets
-// are contiguous in tile order.
-__device__ __forceinline__ int xcd_swizzle(int bid, int nblocks)
-{
-    const int per = nblocks / kXcds;  // full rounds of kXcds
-    if (bid >= per * kXcds) return bid;  // ragged tail keeps its id
-    return (bid % kXcds) * per + bid / kXcds;
-}
+using pat::kWave;
+using pat::xcd_swizzle;
 
 template <int BX, int BY, int RY>
 __global__ __launch_bounds__(BX *BY) void heat_lds25d(const float *__restrict__ in, float *__restrict__ out, int nx,
@@ -305,11 +299,275 @@ __global__ __launch_bounds__(256) void heat_tb2(const float *__restrict__ in, fl
     tb2_window<RY>(in, out, nx, ny, nz, zc, alpha, t % tiles_x, (t / tiles_x) % tiles_y, t / (tiles_x * tiles_y));
 }
 
-// The same two fused sweeps over several grids in one launch: workgroup t
-// takes window t - first of the last grid whose first workgroup is <= t.
-template <int RY>
-__global__ __launch_bounds__(256) void heat_tb2_batch(const pat::HeatBatchGrid *__restrict__ grids, int ngrids,
-                                                      int nblocks, float alpha)
+// T sweeps fused per pass, in registers.  A wavefront holds a strip of 64 * CX
+// columns by RY rows, each lane CX neighbouring columns; W wavefronts stacked
+// in y make the window, which marches a z-chunk.  In the step of plane z the
+// input (level 0) of plane z arrives and level s of plane z - s follows from
+// three planes of level s - 1, for s = 1 .. T; the last is the output.  A cell's
+// z neighbours are registers of its own lane, its y neighbours registers of
+// its own lane or, at a strip's edge, the next strip's edge row, which goes
+// through LDS (two rows per strip and level, double-buffered, one barrier a
+// plane), and its x neighbours come from the next lanes by a DPP wavefront
+// shift that the add itself does.  So a cell update takes 10 to 11 vector
+// instructions and 4 / RY LDS ones, where a window held in LDS (tb2_window)
+// reads four neighbours from LDS and writes one cell.  Measured per step, us,
+// two-sweep windows or cubes before: 64^3 2.74 -> 1.55, 128^3 5.0 -> 3.6,
+// 384^3 59.3 -> 32; at 384^3 vector issue bounds it (72 M instructions of a
+// launch take 123 of its 134 us, 430 MB of traffic).
+//
+// Each cell is read and written once per T steps, plus the window's margins:
+// a window's outer T columns and rows are not output, except at the grid's
+// edge, where the halo beyond the window is zero at every level, which the
+// lane shifts and the zero rows beyond the strips give by themselves.  Windows
+// therefore never reach beyond the grid, and no cell needs a test, unless the
+// grid is smaller than a window (EDGE): then the cells beyond it are kept at
+// zero by a select, so values that are not finite stay where the single sweep
+// has them.  A chunk reads T planes more on either side; level s is computed
+// from the first plane that a written cell depends on.  Each cell's arithmetic
+// is the single sweep's: the same bits as T sweeps.
+__device__ __forceinline__ float lane_below(float v)  // lane l gets lane l - 1's, lane 0 gets 0
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float lane_above(float v)  // lane l gets lane l + 1's, lane 63 gets 0
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xF, 0xF, true));
+}
+
+// A plane as a buffer: accesses add a lane's byte offset (vector) and a row's
+// (scalar) to its base, so that a row costs no address arithmetic.  The base
+// stays in scalar registers and out of the compiler's sight, which would
+// otherwise compute the unrolled loop's addresses ahead, in up to 245 vector
+// registers.  A plane is below 4 GiB (the launcher sees to it).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_buffer(const float *p)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, -1, 0x00027000);
+}
+__device__ __forceinline__ const float *opaque_scalar(const float *p)
+{
+    asm("" : "+s"(p));
+    return p;
+}
+
+// Window i of 'tiles' (as many as cover the axis, or more) over an axis of n
+// cells: its first cell, and the cells [lo, hi] that it writes.
+template <int S, int T>
+__device__ __forceinline__ void strip_place(int n, int i, int tiles, int &first, int &lo, int &hi)
+{
+    const int at = 1 + i * (S - 2 * T);
+    first = n >= S ? min(at, n - S + 1) : 1;
+    lo = i == 0 ? 1 : at + T;
+    hi = i == tiles - 1 ? n : min(at + S - T - 1, n);
+}
+
+template <int T, int CX, int RY, int W, bool EDGE>
+__device__ __forceinline__ void strip_window(const float *__restrict__ in, float *__restrict__ out, int nx, int ny,
+                                             int nz, int zc, float alpha, int tiles_x, int tiles_y, int bx, int by,
+                                             int bz)
+{
+    typedef float Row __attribute__((ext_vector_type(CX)));
+    // edge rows of the strips per level: [0] a strip's first row, [1] its
+    // last; strip w at index w + 1, the rows beyond the window zero
+    __shared__ Row edge[2][T][W + 2][2][kWave];
+
+    const int w = pat::wave_in_block(), lane = (int)threadIdx.x % kWave;
+    const int sx = nx + 2;
+    const int64_t sxy = (int64_t)sx * (ny + 2);
+    int x0, y0, xlo, xhi, ylo, yhi;
+    strip_place<kWave * CX, T>(nx, bx, tiles_x, x0, xlo, xhi);
+    strip_place<RY * W, T>(ny, by, tiles_y, y0, ylo, yhi);
+    x0 += lane * CX;  // this lane's first column
+    y0 += w * RY;     // this strip's first row
+    const int z0 = bz * zc + 1, z1 = min(z0 + zc, nz + 1);  // output planes [z0, z1)
+
+    for (int i = (int)threadIdx.x; i < 2 * T * 2 * kWave; i += kWave * W) {
+        const int l = i % kWave, side = i / kWave % 2, s = i / (2 * kWave) % T, p = i / (2 * kWave * T);
+        edge[p][s][side ? W + 1 : 0][side ? 0 : 1][l] = Row(0.0f);
+    }
+
+    bool xin[CX], xw[CX];
+#pragma unroll
+    for (int j = 0; j < CX; j++) {
+        const int x = x0 + j;
+        xin[j] = !EDGE || x <= nx;
+        xw[j] = x >= xlo && x <= xhi;
+    }
+    // byte offsets of this lane's columns in a row (for loads moved inside the
+    // halo-inclusive row) and of the strip's rows in a plane
+    const int xl = 4 * (EDGE ? min(x0, nx + 2 - CX) : x0), xs = 4 * x0;
+    const bool all_w = xw[0] & xw[CX - 1];
+    bool yw[RY];       // uniform per wavefront
+    bool cin[RY][CX];  // the cell lies inside the grid
+    int yo[RY];
+#pragma unroll
+    for (int r = 0; r < RY; r++) {
+        const int y = y0 + r;
+        yw[r] = y >= ylo && y <= yhi;
+        yo[r] = (int)(4u * (uint32_t)sx * (uint32_t)(EDGE ? min(y, ny + 1) : y));
+#pragma unroll
+        for (int j = 0; j < CX; j++) cin[r][j] = xin[j] & (!EDGE || y <= ny);
+    }
+
+    // Level 0 of plane z in slot z % 4 (loaded two planes ahead), level s of
+    // plane z - s in slot z % 3; the z loop is unrolled by twelve so that the
+    // slots are fixed registers.
+    float A[4][RY][CX], L[T > 1 ? T - 1 : 1][3][RY][CX];
+#pragma unroll
+    for (int r = 0; r < RY; r++)
+#pragma unroll
+        for (int j = 0; j < CX; j++) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) A[q][r][j] = 0.0f;
+#pragma unroll
+            for (int s = 0; s < T - 1; s++)
+#pragma unroll
+                for (int q = 0; q < 3; q++) L[s][q][r][j] = 0.0f;
+        }
+    // The plane at p, with no branch: a wait for one plane's loads then leaves
+    // the next one's in flight.
+    auto load = [&](const float *__restrict__ p, float (&v)[RY][CX]) {
+        const auto q = plane_buffer(p);
+#pragma unroll
+        for (int r = 0; r < RY; r++) {
+            if (CX == 1) {
+                v[r][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(q, xl, yo[r], 0));
+            } else {
+                const auto c = __builtin_amdgcn_raw_buffer_load_b64(q, xl, yo[r], 0);
+#pragma unroll
+                for (int j = 0; j < CX; j++) v[r][j] = __uint_as_float(c[j]);
+            }
+        }
+    };
+
+    const int zs = max(z0 - T, 1), ze = z1 - 1 + T;  // first and last step
+    // planes zs + 2 (at most the upper halo plane, zero) and zs - T, moved on
+    // with every step
+    const float *__restrict__ pin = in + (int64_t)min(zs + 2, nz + 1) * sxy;
+    const float *pout = out + (int64_t)(zs - T) * sxy;
+    load(in + (int64_t)zs * sxy, A[0]);
+    load(in + (int64_t)(zs + 1) * sxy, A[1]);
+    __syncthreads();  // the zero rows
+
+    auto step = [&](auto phase, int z) {
+        constexpr int K = decltype(phase)::value;  // z - zs modulo 12
+        if (EDGE && CX > 1) {  // columns beyond the grid of a pair moved inside the row (the others read the zero halo)
+#pragma unroll
+            for (int r = 0; r < RY; r++)
+#pragma unroll
+                for (int j = 0; j < CX; j++) A[K & 3][r][j] = xin[j] ? A[K & 3][r][j] : 0.0f;
+        }
+        Row up[T], dn[T];
+#pragma unroll
+        for (int s = 0; s < T; s++) {
+            up[s] = edge[(K + 1) & 1][s][w][1][lane];
+            dn[s] = edge[(K + 1) & 1][s][w + 2][0][lane];
+        }
+        auto put_edge = [&](int s, const float (&v)[RY][CX]) {
+            Row a, b;
+#pragma unroll
+            for (int j = 0; j < CX; j++) {
+                a[j] = v[0][j];
+                b[j] = v[RY - 1][j];
+            }
+            edge[K & 1][s][w + 1][0][lane] = a;
+            edge[K & 1][s][w + 1][1][lane] = b;
+        };
+        put_edge(0, A[K & 3]);
+        // level s of plane z - s: m, c, a hold level s - 1 of planes z - s - 1,
+        // z - s, z - s + 1
+        auto stage = [&](int s, const float (&m)[RY][CX], const float (&c)[RY][CX], const float (&a)[RY][CX],
+                         float (&v)[RY][CX]) {
+            if (z - s >= 1) {  // uniform; below the grid the slots hold their first zeros
+#pragma unroll
+                for (int r = 0; r < RY; r++)
+#pragma unroll
+                    for (int j = 0; j < CX; j++) {
+                        const float cc = c[r][j];
+                        const float left = j == 0 ? lane_below(c[r][CX - 1]) : c[r][j > 0 ? j - 1 : 0];
+                        const float right = j == CX - 1 ? lane_above(c[r][0]) : c[r][j < CX - 1 ? j + 1 : 0];
+                        float sum = left + right;
+                        sum = sum + (r == 0 ? up[s - 1][j] : c[r > 0 ? r - 1 : 0][j]);
+                        sum = sum + (r == RY - 1 ? dn[s - 1][j] : c[r < RY - 1 ? r + 1 : 0][j]);
+                        sum = sum + m[r][j];
+                        sum = sum + a[r][j];
+                        const float n = cc + alpha * (sum - 6.0f * cc);
+                        v[r][j] = !EDGE || cin[r][j] ? n : 0.0f;
+                        // not to be moved into a later branch, where the adds
+                        // could not take the lane shifts along
+                        asm volatile("" : "+v"(v[r][j]));
+                    }
+            }
+            if (z - s > nz) {  // uniform: the halo plane above the grid
+#pragma unroll
+                for (int r = 0; r < RY; r++)
+#pragma unroll
+                    for (int j = 0; j < CX; j++) v[r][j] = 0.0f;
+            }
+        };
+        float o[RY][CX];
+#pragma unroll
+        for (int s = 1; s <= T; s++) {
+            if (z < z0 - T + 2 * s) break;  // uniform: no written cell depends on it (nor on the later levels')
+            const auto &src = L[s > 1 ? s - 2 : 0];
+            const auto &m = s == 1 ? A[(K + 2) & 3] : src[(K + 1) % 3];
+            const auto &c = s == 1 ? A[(K + 3) & 3] : src[(K + 2) % 3];
+            const auto &a = s == 1 ? A[K & 3] : src[K % 3];
+            if (s < T) {
+                stage(s, m, c, a, L[s - 1][K % 3]);
+                put_edge(s, L[s - 1][K % 3]);
+            } else {
+                stage(s, m, c, a, o);
+                if (z - T >= z0) {
+                    const auto q = plane_buffer(pout);
+#pragma unroll
+                    for (int r = 0; r < RY; r++) {
+                        if (!yw[r]) continue;
+                        if (CX == 2 && all_w) {
+                            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+                            const u32x2 c = {__float_as_uint(o[r][0]), __float_as_uint(o[r][CX - 1])};
+                            __builtin_amdgcn_raw_buffer_store_b64(c, q, xs, yo[r], 0);
+                        } else {
+#pragma unroll
+                            for (int j = 0; j < CX; j++)
+                                if (xw[j])
+                                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[r][j]), q, xs + 4 * j, yo[r], 0);
+                        }
+                    }
+                }
+            }
+        }
+        // level 0 of plane z + 2 over plane z - 2
+        load(pin, A[(K + 2) & 3]);
+        pin = opaque_scalar(pin + (z + 2 <= nz ? sxy : 0));
+        pout = opaque_scalar(pout + sxy);
+        __syncthreads();
+    };
+    for (int z = zs; z <= ze; z += 12) {
+#define PAT_STEP(K_)                                                                                                   \
+    if (K_ > 0 && z + K_ > ze) break;                                                                                  \
+    step(std::integral_constant<int, K_>(), z + K_);
+        PAT_STEP(0) PAT_STEP(1) PAT_STEP(2) PAT_STEP(3) PAT_STEP(4) PAT_STEP(5)
+        PAT_STEP(6) PAT_STEP(7) PAT_STEP(8) PAT_STEP(9) PAT_STEP(10) PAT_STEP(11)
+#undef PAT_STEP
+    }
+}
+
+template <int T, int CX, int RY, int W, int M, bool EDGE>
+__global__ __launch_bounds__(kWave *W, M) void heat_strip(const float *__restrict__ in, float *__restrict__ out,
+                                                          int nx, int ny, int nz, int zc, float alpha, int tiles_x,
+                                                          int tiles_y, int tiles_z)
+{
+    const int t = xcd_swizzle(blockIdx.x, tiles_x * tiles_y * tiles_z);
+    strip_window<T, CX, RY, W, EDGE>(in, out, nx, ny, nz, zc, alpha, tiles_x, tiles_y, t % tiles_x,
+                                     (t / tiles_x) % tiles_y, t / (tiles_x * tiles_y));
+}
+
+// The same sweeps over several grids in one launch: workgroup t takes window
+// t - first of the last grid whose first workgroup is <= t.  Grids of any
+// size share the launch, so the form that keeps cells beyond the grid at zero.
+template <int T>
+__global__ __launch_bounds__(512) void heat_strip_batch(const pat::HeatBatchGrid *__restrict__ grids, int ngrids,
+                                                        int nblocks, float alpha)
 {
     const int t = xcd_swizzle(blockIdx.x, nblocks);
     int lo = 0, hi = ngrids - 1;
@@ -320,8 +578,8 @@ __global__ __launch_bounds__(256) void heat_tb2_batch(const pat::HeatBatchGrid *
     }
     const pat::HeatBatchGrid g = grids[lo];
     const int u = t - g.first;
-    tb2_window<RY>(g.in, g.out, g.nx, g.ny, g.nz, g.zc, alpha, u % g.tiles_x, (u / g.tiles_x) % g.tiles_y,
-                   u / (g.tiles_x * g.tiles_y));
+    strip_window<T, 1, 4, 8, true>(g.in, g.out, g.nx, g.ny, g.nz, g.zc, alpha, g.tiles_x, g.tiles_y, u % g.tiles_x,
+                                   (u / g.tiles_x) % g.tiles_y, u / (g.tiles_x * g.tiles_y));
 }
 
 // Several sweeps per launch on blocks of the grid held in LDS, for small
@@ -543,6 +801,71 @@ int cube_prepare()
     return rc;
 }
 
+// Strip windows: columns per lane, rows per strip, strips, and the wavefronts
+// per SIMD the registers must leave room for.
+struct StripShape {
+    int cx, ry, w, m;
+};
+constexpr StripShape kStrips[] = {{1, 2, 8, 1}, {1, 4, 8, 1}, {2, 2, 8, 1}, {1, 6, 8, 4}, {1, 4, 16, 4}};
+constexpr int kNumStrips = sizeof(kStrips) / sizeof(kStrips[0]);
+
+template <int T, bool EDGE, int I = 0>
+HeatKernel strip_kernel_of(int shape)
+{
+    if constexpr (I < kNumStrips) {
+        constexpr StripShape S = kStrips[I];
+        if (shape == I) return heat_strip<T, S.cx, S.ry, S.w, S.m, EDGE>;
+        return strip_kernel_of<T, EDGE, I + 1>(shape);
+    } else {
+        return nullptr;
+    }
+}
+
+HeatKernel strip_kernel(int shape, int sweeps, bool edge)
+{
+    switch (sweeps) {
+    case 1: return edge ? strip_kernel_of<1, true>(shape) : strip_kernel_of<1, false>(shape);
+    case 2: return edge ? strip_kernel_of<2, true>(shape) : strip_kernel_of<2, false>(shape);
+    case 3: return edge ? strip_kernel_of<3, true>(shape) : strip_kernel_of<3, false>(shape);
+    case 4: return edge ? strip_kernel_of<4, true>(shape) : strip_kernel_of<4, false>(shape);
+    case 6: return edge ? strip_kernel_of<6, true>(shape) : strip_kernel_of<6, false>(shape);
+    default: return nullptr;
+    }
+}
+
+// Most sweeps that a launch of at most n takes (5 has no kernel).
+int strip_sweeps(int n) { return n >= 6 ? 6 : (n == 5 ? 3 : n); }
+
+// Windows of s cells over an axis of n (see strip_place); 0 where the margins
+// leave no output.
+int64_t strip_tiles(int64_t n, int s, int sweeps)
+{
+    if (n <= s) return 1;
+    return s > 2 * sweeps ? (n - 2 * sweeps + s - 2 * sweeps - 1) / (s - 2 * sweeps) : 0;
+}
+
+// The strip tile of a shape with z-chunks that give each of 256 CUs 'fill'
+// workgroups (fewer, longer chunks where that does not come out even: a last
+// round of few workgroups costs more than idle CUs).  False where the shape
+// has no output beside its margins or a plane reaches 4 GiB.
+bool strip_tile(int shape, int sweeps, int fill, int64_t nx, int64_t ny, int64_t nz, pat::HeatTile *t)
+{
+    const StripShape &c = kStrips[shape];
+    const int64_t tx = strip_tiles(nx, kWave * c.cx, sweeps), ty = strip_tiles(ny, c.ry * c.w, sweeps);
+    if (!tx || !ty || (nx + 2) * (ny + 2) >= (1LL << 30)) return false;
+    const int64_t tz = std::max<int64_t>(1, std::min<int64_t>(nz, 256 * fill / (tx * ty)));
+    *t = pat::HeatTile{3, kWave * c.cx, c.w, c.ry, (int)((nz + tz - 1) / tz), shape, sweeps, fill};
+    return true;
+}
+
+// Strips without tuning: narrow ones while the grid has too few cells for
+// 256 wider windows.
+bool strip_default(int64_t nx, int64_t ny, int64_t nz, pat::HeatTile *t)
+{
+    const bool small = nx * ny * nz < (1 << 19);
+    return strip_tile(small ? 0 : 1, 4, small ? 1 : 2, nx, ny, nz, t);
+}
+
 // Default tile for a grid: 64-wide rows, 4x2 thread rows, and a z-chunk that
 // yields enough workgroups (>= ~4 per CU on 256 CUs) without making chunks so
 // short that the two extra halo planes per chunk dominate.
@@ -632,29 +955,47 @@ int heat3d_cube(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz,
     return PAT_OK;
 }
 
-// One launch of tile t: a single sweep (fused == 0), two (fused == 1) or
-// t.ry on LDS cubes (fused == 2).
+// sweeps sweeps in -> out by strips of shape 'shape', z-chunk zc.
+int heat3d_strip(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha, int shape, int sweeps,
+                 int zc, hipStream_t stream)
+{
+    PAT_REQUIRE(shape >= 0 && shape < kNumStrips && sweeps > 0, PAT_ERR_UNSUPPORTED,
+                "heat3d: strip shape %d with %d sweeps not instantiated", shape, sweeps);
+    const StripShape &c = kStrips[shape];
+    const int xw = kWave * c.cx, yw = c.ry * c.w;
+    const HeatKernel k = strip_kernel(shape, sweeps, nx < xw || ny < yw);
+    PAT_REQUIRE(k, PAT_ERR_UNSUPPORTED, "heat3d: strip shape %d with %d sweeps not instantiated", shape, sweeps);
+    PAT_REQUIRE(zc > 0, PAT_ERR_INVALID, "heat3d: z-chunk must be positive");
+    const int64_t tx = strip_tiles(nx, xw, sweeps), ty = strip_tiles(ny, yw, sweeps), tz = (nz + zc - 1) / zc;
+    PAT_REQUIRE(tx > 0 && ty > 0, PAT_ERR_UNSUPPORTED, "heat3d: strip shape %d has no output beside its margins", shape);
+    PAT_REQUIRE(tx * ty * tz < (1LL << 31), PAT_ERR_INVALID, "heat3d: grid too large");
+    PAT_REQUIRE((nx + 2) * (ny + 2) < (1LL << 30), PAT_ERR_UNSUPPORTED, "heat3d: planes of 4 GiB and more have no strip form");
+    hipLaunchKernelGGL(k, dim3((unsigned)(tx * ty * tz)), dim3((unsigned)(kWave * c.w)), 0, stream, in, out, (int)nx,
+                       (int)ny, (int)nz, zc, alpha, (int)tx, (int)ty, (int)tz);
+    PAT_LAUNCH_CHECK();
+    return PAT_OK;
+}
+
+// One launch of tile t: a single sweep (fused == 0), two (fused == 1), t.ry
+// on LDS cubes (fused == 2) or t.ry by strips (fused == 3).
 int heat3d_launch(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha, const HeatTile &t,
                   int variant, hipStream_t stream)
 {
+    if (t.fused == 3) return heat3d_strip(in, out, nx, ny, nz, alpha, t.shape, t.sweeps, t.zc, stream);
     if (t.fused == 2) return heat3d_cube(in, out, nx, ny, nz, alpha, t.bx, stream);
     if (t.fused) return heat3d_sweep2(in, out, nx, ny, nz, alpha, t.ry, t.zc, stream);
     return heat3d_sweep(in, out, nx, ny, nz, alpha, variant, t.bx, t.by, t.ry, t.zc, stream);
 }
 
-// nsteps sweeps ping-ponging buf[start] -> buf[1-start] ...: fused pairs
-// while two or more steps remain, a plain sweep for an odd last one.
-// Returns the buffer index holding the result in *end.
 int heat3d_batch_table(int n, float *const *a, float *const *b, const int64_t *nx, const int64_t *ny,
                        const int64_t *nz, HeatBatchGrid *table, hipStream_t st, int *nblocks)
 {
     PAT_REQUIRE(n > 0 && a && b && nx && ny && nz && table && nblocks, PAT_ERR_INVALID, "heat3d batch: bad arguments");
-    constexpr int OX = 60, OY = 12;  // output window of the 64 x 16 fused window (4 rows per thread)
     std::vector<HeatBatchGrid> h(2 * (size_t)n);
     int64_t total = 0;
     for (int i = 0; i < n; i++) {
         PAT_REQUIRE(a[i] && b[i] && a[i] != b[i] && nx[i] > 0 && ny[i] > 0 && nz[i] > 0 &&
-                        (nx[i] + 2) * (ny[i] + 2) * (nz[i] + 2) < (1LL << 40),
+                        (nx[i] + 2) * (ny[i] + 2) < (1LL << 30) && (nx[i] + 2) * (ny[i] + 2) * (nz[i] + 2) < (1LL << 40),
                     PAT_ERR_INVALID, "heat3d batch: grid %d has bad buffers or sizes", i);
         HeatBatchGrid g;
         g.in = a[i];
@@ -663,8 +1004,8 @@ int heat3d_batch_table(int n, float *const *a, float *const *b, const int64_t *n
         g.ny = (int)ny[i];
         g.nz = (int)nz[i];
         g.zc = (int)std::min<int64_t>(8, nz[i]);
-        g.tiles_x = (int)((nx[i] + OX - 1) / OX);
-        g.tiles_y = (int)((ny[i] + OY - 1) / OY);
+        g.tiles_x = (int)strip_tiles(nx[i], 64, 4);  // heat_strip_batch<4>'s windows, which cover fewer sweeps too
+        g.tiles_y = (int)strip_tiles(ny[i], 32, 4);
         g.first = (int)total;
         g.pad = 0;
         total += (int64_t)g.tiles_x * g.tiles_y * ((nz[i] + g.zc - 1) / g.zc);
@@ -686,25 +1027,20 @@ int heat3d_batch_enqueue(int n, float *const *a, float *const *b, const int64_t 
 {
     PAT_REQUIRE(n > 0 && nblocks > 0 && nsteps >= 0 && table && in_b, PAT_ERR_INVALID, "heat3d batch: bad arguments");
     int c = 0;
-    for (int k = 0; k + 2 <= nsteps; k += 2) {
-        hipLaunchKernelGGL(heat_tb2_batch<4>, dim3((unsigned)nblocks), dim3(64, 4), 0, st, table + (size_t)c * n, n,
-                           nblocks, alpha);
+    for (int k = 0, r; k < nsteps; k += r, c = 1 - c) {
+        r = std::min(nsteps - k, 4);
+        auto f = r == 4 ? heat_strip_batch<4>
+                        : (r == 3 ? heat_strip_batch<3> : (r == 2 ? heat_strip_batch<2> : heat_strip_batch<1>));
+        hipLaunchKernelGGL(f, dim3((unsigned)nblocks), dim3(512), 0, st, table + (size_t)c * n, n, nblocks, alpha);
         PAT_LAUNCH_CHECK();
-        c = 1 - c;
-    }
-    if (nsteps % 2) {
-        for (int i = 0; i < n; i++) {
-            int bx, by, ry, zc;
-            default_tile(nx[i], ny[i], nz[i], &bx, &by, &ry, &zc);
-            PAT_TRY(heat3d_sweep(c ? b[i] : a[i], c ? a[i] : b[i], nx[i], ny[i], nz[i], alpha, PAT_STENCIL_LDS25D, bx,
-                                 by, ry, zc, st));
-        }
-        c = 1 - c;
     }
     *in_b = c;
     return PAT_OK;
 }
 
+// nsteps sweeps ping-ponging buf[start] -> buf[1-start] ...: the tile's sweeps
+// per launch while as many remain, then launches of fewer (strips) or plain
+// sweeps.  Returns the buffer index holding the result in *end.
 int heat3d_steps(float *const buf[2], int start, int64_t nx, int64_t ny, int64_t nz, float alpha, const HeatTile &t,
                  int variant, int nsteps, hipStream_t stream, int *end)
 {
@@ -714,6 +1050,14 @@ int heat3d_steps(float *const buf[2], int start, int64_t nx, int64_t ny, int64_t
     if (spl > 1) {
         for (; k + spl <= nsteps; k += spl) {
             PAT_TRY(heat3d_launch(buf[c], buf[1 - c], nx, ny, nz, alpha, t, variant, stream));
+            c = 1 - c;
+        }
+    }
+    if (k < nsteps && t.fused == 3) {  // the sweeps left over, in launches of fewer
+        HeatTile p = t;
+        for (; k < nsteps; k += p.sweeps) {
+            p.sweeps = strip_sweeps(nsteps - k);
+            PAT_TRY(heat3d_launch(buf[c], buf[1 - c], nx, ny, nz, alpha, p, variant, stream));
             c = 1 - c;
         }
     }
@@ -732,55 +1076,47 @@ int heat3d_steps(float *const buf[2], int start, int64_t nx, int64_t ny, int64_t
     return PAT_OK;
 }
 
-// Autotuner: times every instantiated tile shape with z-chunks of 2..64
-// planes on the caller's grid (in -> out; out is scratch until the first
-// real sweep writes it, and no kernel writes the halo), keeps the fastest,
-// and caches it for the process per size class: each extent's half octave
-// (floor(2 log2 n)), so a stream of grids of many sizes (a serving mix)
-// tunes once per class; every tile gives the same bits on any grid.
-static std::map<std::tuple<int, int, int, int>, HeatTile> g_tile_cache;
+// Autotuner: times every strip shape with 3, 4 and 6 sweeps and 1 to 4
+// workgroups per CU on the caller's grid (in -> out; out is scratch until the
+// first real sweep writes it, and no kernel writes the halo), keeps the
+// fastest, and caches it for the process per size class: each extent's half
+// octave (floor(2 log2 n)), so a stream of grids of many sizes (a serving mix)
+// tunes once per class; the z-chunk is worked out again for each grid, and
+// every tile gives the same bits on any grid.  The other kernels are no
+// candidates: strips were faster on every grid tried from 1 cell to 384^3 (us
+// per step, strips against the fastest other: 32^3 1.4 and 2.2, 64^3 1.6 and
+// 2.9, 128^3 3.3 and 5.3, 256^3 10.3 and 15.8, 384^3 32.0 and 59.1).
+static std::map<std::tuple<int, int, int>, HeatTile> g_tile_cache;
 static std::mutex g_tile_mutex;
 
 static int size_class(int64_t n) { return (int)std::floor(2.0 * std::log2((double)n)); }
 
-// allow_fused: whether two-sweep tiles may be chosen (the caller runs
-// pairs of steps); their time is compared per step.
 int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha, hipStream_t st,
-                 bool allow_fused, HeatTile *t)
+                 HeatTile *t)
 {
-    const auto key = std::make_tuple(size_class(nx), size_class(ny), size_class(nz), (int)allow_fused);
+    const auto key = std::make_tuple(size_class(nx), size_class(ny), size_class(nz));
     {
         std::lock_guard<std::mutex> g(g_tile_mutex);
         auto it = g_tile_cache.find(key);
-        if (it != g_tile_cache.end()) {
-            *t = it->second;
-            t->zc = (int)std::min<int64_t>(t->zc, nz);
+        if (it != g_tile_cache.end() &&
+            strip_tile(it->second.shape, it->second.sweeps, it->second.fill, nx, ny, nz, t))
             return PAT_OK;
-        }
     }
-    t->fused = 0;
-    default_tile(nx, ny, nz, &t->bx, &t->by, &t->ry, &t->zc);
-    if (!pat::tuning_enabled()) {
-        // untuned: the two-sweep window the tuner picks at 128^3 and 384^3
-        // where two sweeps per launch are allowed (same values either way)
-        if (allow_fused) *t = HeatTile{1, 64, 4, 4, (int)std::min<int64_t>(8, nz)};
+    if (!strip_default(nx, ny, nz, t)) {  // planes of 4 GiB and more
+        *t = HeatTile{1, 64, 4, 4, (int)std::min<int64_t>(64, nz)};
         return PAT_OK;
     }
+    if (!pat::tuning_enabled()) return PAT_OK;
     std::vector<HeatTile> cands;
-    for (const auto &sh : kShapes)
-        for (int z : {2, 4, 8, 16, 32, 64}) {
-            if (z > nz && z != 2) continue;
-            cands.push_back(HeatTile{0, sh.bx, sh.by, sh.ry, (int)std::min<int64_t>(z, nz)});
-        }
-    if (allow_fused) {
-        for (int r : {2, 4, 8})
-            for (int z : {2, 4, 8, 16, 32, 64, 128}) {
-                if (z > nz && z != 2) continue;
-                cands.push_back(HeatTile{1, 64, 4, r, (int)std::min<int64_t>(z, nz)});
+    for (int c = 0; c < kNumStrips; c++)
+        for (int sweeps : {3, 4, 6})
+            for (int fill : {1, 2, 3, 4}) {
+                HeatTile h;
+                if (!strip_tile(c, sweeps, fill, nx, ny, nz, &h)) continue;
+                if (!cands.empty() && cands.back().shape == c && cands.back().sweeps == sweeps && cands.back().zc == h.zc)
+                    continue;
+                cands.push_back(h);
             }
-        PAT_TRY(cube_prepare());  // before any capture
-        for (int c = 0; c < kNumCubes; c++) cands.push_back(HeatTile{2, c, 0, kCubes[c].t, 0});
-    }
     pat::EventPair ev;
     PAT_HIP(ev.create());
     hipEvent_t a = ev.a, b = ev.b;
@@ -865,24 +1201,12 @@ int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz
         if (tm[c] < tm[bi]) bi = c;
     if (pat::tune_log())
         for (size_t c = 0; c < cands.size(); c++)
-            fprintf(stderr, "[tune heat3d %lldx%lldx%lld] fused %d bx %d by %d ry %d zc %d: %.2f us/step%s\n",
-                    (long long)nx, (long long)ny, (long long)nz, cands[c].fused, cands[c].bx, cands[c].by,
-                    cands[c].ry, cands[c].zc, 1000.0f * tm[c], c == bi ? "  <- chosen" : "");
+            fprintf(stderr, "[tune heat3d %lldx%lldx%lld] %d x %d window, %d rows a strip, zc %d, %d sweeps: %.2f us/step%s\n",
+                    (long long)nx, (long long)ny, (long long)nz, cands[c].bx, cands[c].by * cands[c].ry, cands[c].ry,
+                    cands[c].zc, cands[c].sweeps, 1000.0f * tm[c], c == bi ? "  <- chosen" : "");
     *t = cands[bi];
     std::lock_guard<std::mutex> g(g_tile_mutex);
     g_tile_cache[key] = *t;
-    return PAT_OK;
-}
-
-int heat3d_tuned_tile(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha, hipStream_t st,
-                      int *bx, int *by, int *ry, int *zc)
-{
-    HeatTile t;
-    PAT_TRY(heat3d_tuned(in, out, nx, ny, nz, alpha, st, false, &t));
-    *bx = t.bx;
-    *by = t.by;
-    *ry = t.ry;
-    *zc = t.zc;
     return PAT_OK;
 }
 
@@ -913,6 +1237,15 @@ int heat3d_shapes(const int **triples)
 
 }  // namespace pat
 
+// One launch of a strip form by its place in the table, for the tests; not
+// part of the public interface.
+extern "C" int pat_internal_heat_strip(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha,
+                                       int shape, int sweeps, int zc, void *stream)
+{
+    PAT_REQUIRE(in && out && in != out && nx > 0 && ny > 0 && nz > 0, PAT_ERR_INVALID, "heat strip: bad arguments");
+    return pat::heat3d_strip(in, out, nx, ny, nz, alpha, shape, sweeps, zc, (hipStream_t)stream);
+}
+
 extern "C" int pat_heat3d_run_dev(float *a, float *b, int64_t nx, int64_t ny, int64_t nz, int nsteps, float alpha,
                                   int variant, int bx, int by, int zc, int *result_in_b, void *stream)
 {
@@ -924,7 +1257,7 @@ extern "C" int pat_heat3d_run_dev(float *a, float *b, int64_t nx, int64_t ny, in
     hipStream_t st = (hipStream_t)stream;
     pat::HeatTile t;
     if (variant == PAT_STENCIL_AUTO && bx == 0 && by == 0 && zc == 0) {
-        PAT_TRY(pat::heat3d_tuned(a, b, nx, ny, nz, alpha, st, true, &t));
+        PAT_TRY(pat::heat3d_tuned(a, b, nx, ny, nz, alpha, st, &t));
     } else if (variant == PAT_STENCIL_CUBES) {
         PAT_TRY(pat::heat3d_cube_tile(bx, &t));
     } else if (variant == PAT_STENCIL_TEMPORAL2) {

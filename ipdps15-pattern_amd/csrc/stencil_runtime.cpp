@@ -97,7 +97,7 @@ struct pat_stencil {
     int resolve_tile(pat::HeatTile *t)
     {
         if (variant == PAT_STENCIL_AUTO && bx == 0 && by == 0 && zc == 0 && loaded) {
-            PAT_TRY(pat::heat3d_tuned(buf[cur], buf[1 - cur], n[0], n[1], n[2], alpha(), stream, true, t));
+            PAT_TRY(pat::heat3d_tuned(buf[cur], buf[1 - cur], n[0], n[1], n[2], alpha(), stream, t));
             return PAT_OK;
         }
         if (variant == PAT_STENCIL_CUBES) return pat::heat3d_cube_tile(bx, t);

@@ -164,3 +164,40 @@ def test_eigenmode_full_size_384(pa, gpu):
     lam = 1 + alpha * 3 * (2 * np.cos(np.pi / (n + 1)) - 2)
     err = np.max(np.abs(out.numpy() - g0 * lam ** steps))
     assert err < 1e-5
+
+
+STRIPS = [(64, 16), (64, 32), (128, 16), (64, 48), (64, 64)]  # the strip forms' windows
+
+
+def strip_run(pa, g, shape, sweeps, zc):
+    import ctypes
+    f = pa.lib().pat_internal_heat_strip
+    f.restype = ctypes.c_int
+    f.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_float,
+                  ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    nz, ny, nx = (n - 2 for n in g.shape)
+    a = pa.DeviceArray.from_numpy(g)
+    b = pa.DeviceArray.from_numpy(np.zeros_like(g))
+    assert f(a.ptr, b.ptr, nx, ny, nz, 0.1, shape, sweeps, zc, None) == 0, pa.lib().pat_last_error()
+    pa.sync()
+    return b.numpy()
+
+
+@pytest.mark.parametrize("sweeps", [1, 2, 3, 4, 6])
+@pytest.mark.parametrize("shape", range(5))
+def test_strip_windows_vs_oracle(pa, orc, gpu, shape, sweeps):
+    """Every strip form at the edges of its window: narrower than it, as wide,
+    one cell wider (two windows that overlap almost whole), two full windows
+    and one cell more; one plane, fewer planes than sweeps, chunks with a
+    remainder.  The first case's values include infinities and NaN next to the
+    grid's faces, which must stay where the single sweep has them."""
+    wx, wy = STRIPS[shape]
+    two = [2 * w - 2 * sweeps for w in (wx, wy)]
+    cases = [(wx - 1, wy - 3, 5, 2), (wx, wy, 7, 3), (wx + 1, wy + 1, 4, 4), (two[0], two[1], 9, 4),
+             (two[0] + 1, two[1] + 1, 2, 1), (3, 2, 1, 1), (wx, 1, 12, 12), (1, wy + 5, 3, 2)]
+    for i, (nx, ny, nz, zc) in enumerate(cases):
+        g = pa.gen_heat3d(nx, ny, nz, seed=nx + ny)
+        if i == 0:
+            g[1, 1, 1], g[-2, -2, -2], g[2, -2, 3] = np.inf, np.nan, -np.inf
+        got = strip_run(pa, g, shape, sweeps, zc)
+        assert np.array_equal(got, orc.heat3d(g, sweeps), equal_nan=True), (nx, ny, nz, zc)
