@@ -33,7 +33,8 @@
 // is rescored with the plain path's exact FP32 arithmetic, and the exact
 // results decide (same tie rule).  A centre outside the margin provably has a
 // larger reference distance than the best one, so the assignment equals the
-// plain path's bit for bit.
+// plain path's bit for bit.  Shapes whose object is beyond LDS take the same
+// steps with FP16 parts (km_wide).
 #include <algorithm>
 #include <cmath>
 
@@ -320,6 +321,7 @@ __device__ __forceinline__ float exact_dist(const float *__restrict__ xp, const 
 {
     float dist = 0;
     if (vec) {  // D % 4 == 0 and 16-byte aligned rows
+#pragma unroll 4
         for (int d = 0; d < D; d += 4) {
             const float4 cv = *(const float4 *)(ck + d), xv = *(const float4 *)(xp + d);
             float t = cv.x - xv.x;
@@ -818,6 +820,397 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
     }
 }
 
+// ------------------------------------------------------------ wide MFMA path
+//
+// Assignment where the reduction object does not fit in LDS (the bucketed
+// reduction sums it afterwards, and computes min_dist on its way over the
+// rows, so that this kernel only has to find the centre).
+//
+// The bound decides the cost here: with BF16 terms and the norm accumulated
+// first, 58% of the points of a 1,000-centre mixture at D = 128 had another
+// centre inside the margin, and nearly every workgroup went through the
+// centres twice.  So the operands are split into FP16 high and low parts (u =
+// 2^-11, the dropped terms O(u^2)), scaled by a power of two that puts the
+// largest coordinate just below 2^10, and each value is accumulated with the
+// small terms first: lo.hi and hi.lo, then hi.hi, then the norm, so that
+// only 16 KS + 16 of the additions round at the size of the result.  In units
+// of half the scaled squared distance, with x^ = 2^a x, c^ = -2^a c, X = ||x^||,
+// C = max ||c^||, e = 2^-14 (an FP16 subnormal may be taken as zero) and
+// g = 2^-23 per addition (twice the FP32 roundoff, for any rounding inside the
+// MFMA), the value n^ + x^.c^ (n^ = ||c^||^2 / 2) is off by at most
+//     3 u^2 X C + e sqrt(D) (X + C) + D e^2           the split
+//   + g 32 KS (2 u X C + 2 e sqrt(D) (X + C))         the small terms
+//   + g 16 KS (X C (1 + 2 u) + ...)                   hi.hi
+//   + g 16 (X C + C^2 / 2) + u^3 C^2 / 2 + 2          the norm (FP16 parts of n^ / 2^15)
+// (wide_bound, with 2% over it).  A key's packed index costs 2^-16 of its own
+// magnitude, which for every centre that matters is at most max(X^2 / 2, |smallest
+// key|) and not the sum of the largest norms.
+//
+// A wavefront takes TILES tiles of 32 points, so that a centre fragment read
+// from LDS feeds TILES MFMAs, and steps through the centres in chunks of NB
+// blocks of 32 with its workgroup; the next chunk is copied into the other LDS
+// buffer meanwhile (16-byte loads straight to LDS).  Keys carry seven index
+// bits, so eight blocks make a group: the three smallest keys of each group
+// are merged into the lane's three with their places.  At the end every lane
+// finishes one point: it gets the other half's keys of its point, and when
+// only the smallest key lies under the threshold that is the centre.
+// Otherwise its kept keys under the threshold (at most four centres) are left
+// to km_rescore, in the point's assign and mindist words, and the point in a
+// list: rescoring here, by one or two lanes of a wavefront that its whole
+// workgroup waits for at the next barrier, took more than half the time.
+// Only when a half's third key lies under the threshold too does the workgroup
+// go through the centres again and rescore every one under the threshold.
+//
+// Bound by the matrix cores: 3 KS + 1 MFMAs per 32 x 32 values, issued at 1.03
+// PFLOP/s at D = 128 (a large library product reaches 1.18 on this card); the
+// scan takes 4 vector instructions a value.  1 M x 128, K 1,000: 0.84 ms a pass,
+// 0.7% of the points rescored (2.66 ms with BF16 terms and a second pass over
+// the centres in nearly every workgroup).
+typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
+typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2;
+
+constexpr float kWideOne = 32768.0f;  // the norm parts' factor 2^15
+constexpr float kWideFar = 60000.0f;  // first norm part of a row that never wins: above any value (2^28)
+
+struct WideBound {
+    float sx;                        // 2^a
+    float c_dot, c_sum, c_cc, c_abs;  // error: c_dot X C + c_sum (X + C) + c_cc C^2 + c_abs
+    float c_ref, ref_abs;            // the reference's FP32 difference form: relative, and for underflow
+    float far;                       // half squared distances from here on may reach map1's initial minimum
+};
+
+template <int KS, int NB, int TILES, bool TAIL>
+__global__ __launch_bounds__(512) void km_wide(KmArgs a, const _Float16 *__restrict__ cb,
+                                               const float *__restrict__ cnorm, int K_pad, WideBound bd,
+                                               int *__restrict__ list, int *__restrict__ listed,
+                                               unsigned long long *__restrict__ rescored)
+{
+    constexpr int NS = 2 * KS + 1;  // fragments per block: high, low, norm
+    constexpr int BW = 512 / kWave;
+    static_assert(8 % NB == 0, "a group of eight blocks is a whole number of chunks");
+    extern __shared__ __align__(16) unsigned char wide_lds[];  // two chunks of NB x NS KiB
+    __shared__ float red[BW];
+    const int lane = threadIdx.x % kWave, col = lane % 32, half = lane / 32, wv = pat::wave_in_block();
+    float cm = 0.0f;
+    for (int i = threadIdx.x; i < a.K; i += 512) cm = fmaxf(cm, cnorm[i]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) cm = fmaxf(cm, __shfl_xor(cm, o, kWave));
+    if (lane == 0) red[wv] = cm;
+    __syncthreads();
+    float cmax = 0.0f;
+    for (int w = 0; w < BW; w++) cmax = fmaxf(cmax, red[w]);
+    const float C = cmax * bd.sx;
+
+    const int D = a.D, kblocks = K_pad / 32, nchunks = (kblocks + NB - 1) / NB;
+    const bool vec_x = (D % 4) == 0 && ((uintptr_t)a.x % 16) == 0, vec_c = (D % 4) == 0;
+    const int keep = key_mask();
+    unsigned my_rescored = 0;
+
+    // chunk ch into LDS buffer b, one KiB per wavefront instruction
+    auto stage = [&](int ch, int b) {
+        const int n = min(NB, kblocks - ch * NB) * NS;
+        const unsigned char *src = (const unsigned char *)cb + (int64_t)ch * NB * NS * 1024 + lane * 16;
+        unsigned char *dst = wide_lds + b * (NB * NS * 1024);
+        for (int f = wv; f < n; f += BW)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + f * 1024),
+                                             (__attribute__((address_space(3))) void *)(dst + f * 1024), 16, 0, 0);
+    };
+    auto staged = [&] {  // the loads to LDS have landed, for every wavefront
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+    f16x8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; e++) ones[e] = (_Float16)((half == 0 && e < 3) ? kWideOne : 0.0f);
+
+    stage(0, 0);
+    const int64_t per_block = (int64_t)BW * 32 * TILES;
+    for (int64_t base0 = (int64_t)blockIdx.x * per_block; base0 < a.N; base0 += (int64_t)gridDim.x * per_block) {
+        const int64_t base = base0 + (int64_t)wv * 32 * TILES;  // this wavefront's points
+        // operands: point col of each tile, dimensions 16 s + 8 half + e, scaled and split
+        f16x8 xh[TILES][KS], xl[TILES][KS];
+        float xx[TILES];
+#pragma unroll
+        for (int t = 0; t < TILES; t++) {
+            const int64_t p = base + 32 * t + col;
+            const bool live = p < a.N;
+            const float *xp = a.x + (live ? p : a.N - 1) * D;
+            xx[t] = 0.0f;
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const int d0 = 16 * s + 8 * half;
+                float v[8];
+                if (!TAIL || vec_x) {
+                    float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+                    if (!TAIL || d0 < D) lo = *(const float4 *)(xp + d0);
+                    if (!TAIL || d0 + 4 < D) hi = *(const float4 *)(xp + d0 + 4);
+                    v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
+                    v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[e] = d0 + e < D ? xp[d0 + e] : 0.0f;
+                }
+                u32x4 wh, wl;
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    const f32x2 q = {v[e] * bd.sx, v[e + 1] * bd.sx};
+                    xx[t] = __builtin_fmaf(q[0], q[0], xx[t]);
+                    xx[t] = __builtin_fmaf(q[1], q[1], xx[t]);
+                    const f16x2 h = __builtin_convertvector(q, f16x2);
+                    const f32x2 r = {q[0] - (float)h[0], q[1] - (float)h[1]};
+                    wh[e / 2] = __builtin_bit_cast(unsigned, h);
+                    wl[e / 2] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, f16x2));
+                }
+                // the sum of squares follows the operands (left to the end it
+                // would keep every coordinate in a register, and spill)
+                asm volatile("" : "+v"(xx[t]), "+v"(wl[3]));
+                xh[t][s] = __builtin_bit_cast(f16x8, wh);
+                xl[t][s] = __builtin_bit_cast(f16x8, wl);
+            }
+        }
+        // values of block b of LDS buffer 'buf' for every tile: value i of a
+        // lane is centre row 8 (i / 4) + 4 half + i % 4 of the block
+        auto block_values = [&](int buf, int b, f32x16 (&acc)[TILES]) {
+            constexpr int T = 3 * KS + 1, P = 4;
+            int at = (buf * NB + b) * (NS * 1024) + lane * 16, again = at;
+            asm volatile("" : "+v"(again));  // the high parts are read twice: kept, they would spill
+            auto frag = [&](int t) {
+                const int f = t < 2 * KS ? t : (t < 3 * KS ? t - 2 * KS : 2 * KS);
+                return *(const f16x8 *)(wide_lds + (t < 2 * KS ? at : again) + f * 1024);
+            };
+            f16x8 fr[P];
+#pragma unroll
+            for (int t = 0; t < P; t++) fr[t] = frag(t);
+#pragma unroll
+            for (int u = 0; u < TILES; u++) acc[u] = f32x16{};
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                const f16x8 av = fr[t % P];
+                if (t + P < T) fr[t % P] = frag(t + P);
+#pragma unroll
+                for (int u = 0; u < TILES; u++) {
+                    // hi.lo(x), lo.hi(x), hi.hi, norm
+                    const f16x8 bv = t < KS ? xl[u][t < KS ? t : 0]
+                                            : (t < 2 * KS ? xh[u][t < 2 * KS ? (t - KS) & (KS - 1) : 0]
+                                                          : (t < 3 * KS ? xh[u][t & (KS - 1)] : ones));
+                    acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, acc[u], 0, 0, 0);
+                }
+            }
+            // P reads ahead of the MFMAs that use them, all the way (the
+            // scheduler would bunch them, and wait for a read just issued)
+            __builtin_amdgcn_sched_group_barrier(0x100, P, 0);
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, TILES, 0);
+                if (t + P < T) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+        };
+        auto centre_of = [&](int id, int h) {  // id: block << 4 | value
+            const int i = id & 15;
+            return (id >> 4) * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+        };
+
+        // the three smallest keys of this half, sorted, and their places
+        float g[TILES][3];
+        int gi[TILES][3];
+        float k[TILES][3];  // of the group
+#pragma unroll
+        for (int t = 0; t < TILES; t++)
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                g[t][q] = kFar;
+                gi[t][q] = 0;
+                k[t][q] = kFar;
+            }
+        f32x16 acc[TILES];
+        for (int ch = 0; ch < nchunks; ch++) {
+            staged();  // chunk ch is in buffer ch & 1, and every wavefront is done with the other
+            if (ch + 1 < nchunks) stage(ch + 1, (ch + 1) & 1);
+#pragma unroll 1
+            for (int b = 0; b < NB; b++) {
+                const int blk = ch * NB + b;
+                if (blk >= kblocks) break;  // uniform
+                block_values(ch & 1, b, acc);
+                const int at = (blk & 7) * 16;
+#pragma unroll
+                for (int t = 0; t < TILES; t++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const float key = pack_key(acc[t][i], scalar_or(at, i), keep);
+                        k[t][2] = __builtin_amdgcn_fmed3f(k[t][1], k[t][2], key);
+                        k[t][1] = __builtin_amdgcn_fmed3f(k[t][0], k[t][1], key);
+                        k[t][0] = __builtin_amdgcn_fmed3f(k[t][0], key, -kFar);  // min (keys are finite)
+                    }
+                if ((blk & 7) == 7 || blk == kblocks - 1) {  // the group's keys into the lane's
+#pragma unroll
+                    for (int t = 0; t < TILES; t++)
+#pragma unroll
+                        for (int q = 0; q < 3; q++) {
+                            float v = k[t][q];
+                            int id = (blk >> 3) * 128 + (__float_as_int(v) & 127);
+#pragma unroll
+                            for (int r = 0; r < 3; r++) {
+                                const bool less = v < g[t][r];
+                                const float w = g[t][r];
+                                const int wi = gi[t][r];
+                                g[t][r] = less ? v : w;
+                                gi[t][r] = less ? id : wi;
+                                v = less ? w : v;
+                                id = less ? wi : id;
+                            }
+                            k[t][q] = kFar;
+                        }
+                }
+            }
+        }
+
+        // Every lane finishes a point: lane l point l (of the half's tile).
+        // The partner's part of it: what the partner holds of this lane's tile.
+        const int64_t p = base + lane;
+        const bool live = p < a.N && (TILES == 2 || half == 0);
+        auto own = [&](const auto &v0, const auto &v1) { return TILES == 2 && half ? v1 : v0; };
+        auto theirs = [&](const auto &v0, const auto &v1) {
+            return __shfl_xor(TILES == 2 && !half ? v1 : v0, 32, kWave);
+        };
+        constexpr int L = TILES - 1;
+        const float A1 = own(g[0][0], g[L][0]), A2 = own(g[0][1], g[L][1]), A3 = own(g[0][2], g[L][2]);
+        const float B1 = theirs(g[0][0], g[L][0]), B2 = theirs(g[0][1], g[L][1]), B3 = theirs(g[0][2], g[L][2]);
+        const float X2 = own(xx[0], xx[L]) + theirs(xx[0], xx[L]);
+        const int other = 1 - half;
+        const int a1 = centre_of(own(gi[0][0], gi[L][0]), half), a2 = centre_of(own(gi[0][1], gi[L][1]), half);
+        const int b1 = centre_of(theirs(gi[0][0], gi[L][0]), other), b2 = centre_of(theirs(gi[0][1], gi[L][1]), other);
+        const float m1 = fminf(A1, B1), m2 = fminf(fmaxf(A1, B1), fminf(A2, B2));
+        const float X = __builtin_amdgcn_sqrtf(X2) * 1.0001f + 0x1p-40f, H = 0.5f * X2;
+        const float E = bd.c_dot * X * C + bd.c_sum * (X + C) + bd.c_cc * C * C + bd.c_abs;
+        const float dp = 0x1p-16f * 1.02f * (fmaxf(H, fabsf(m1)) * 1.01f + 4.0f * E) + 0x1p-126f;
+        const float dhi = (H + m1 + 4.0f * E + 4.0f * dp) * 1.001f + bd.ref_abs;
+        const float thr = m1 + 2.0f * E + 2.0f * dp + 2.0f * bd.c_ref * dhi;
+        // (comparisons that a value that is not a number fails)
+        const bool multi = !(m2 > thr) || !(dhi < bd.far);
+        const bool full = live && multi && !(A3 > thr && B3 > thr);
+        const bool again = __syncthreads_or(full) != 0;  // and every wavefront is done with the last chunk
+        if (!again) stage(0, 0);                         // the next round's first chunk
+
+        float best_d = kInitMin;
+        int best_k = 0x7fffffff;
+        auto rescore = [&](const float *x, int c, float &bd_, int &bk) {
+            if (c < a.K) {
+                const float dk = exact_dist(x, a.c + (int64_t)c * D, D, vec_c && vec_x);
+                if (dk < bd_ || (dk == bd_ && c < bk)) {
+                    bd_ = dk;
+                    bk = c;
+                }
+            }
+        };
+        if (live && !multi) best_k = A1 < B1 ? a1 : b1;
+        const bool part = live && multi && !full;
+        const unsigned long long parts = __ballot(part);
+        if (parts) {
+            int at = 0;
+            if (lane == 0) at = atomicAdd(listed, __popcll(parts));
+            at = __shfl(at, 0, kWave) + __popcll(parts & ((1ull << lane) - 1ull));
+            if (part) {
+                // up to four places; unused ones hold the smallest key's
+                // centre again (rows past K are never under the threshold:
+                // their keys are above every other's)
+                const int c0 = A1 < B1 ? a1 : b1;
+                const int c1 = A1 < B1 ? (!(B1 > thr) ? b1 : c0) : (!(A1 > thr) ? a1 : c0);
+                const int c2 = !(A2 > thr) ? a2 : c0, c3 = !(B2 > thr) ? b2 : c0;
+                list[at] = (int)p;
+                a.assign[p] = c0 | c1 << 16;
+                a.mindist[p] = __int_as_float(c2 | c3 << 16);
+            }
+        }
+        if (again) {
+            // every value under the threshold of the full points, rescored by
+            // the half that holds it
+            float bdist[TILES], tt[TILES];
+            int bk[TILES], ff[TILES];
+#pragma unroll
+            for (int t = 0; t < TILES; t++) {
+                const int mine = TILES == 2 ? half : 0;
+                const float ot = __shfl_xor(thr, 32, kWave);
+                const int of = __shfl_xor((int)full, 32, kWave);
+                tt[t] = TILES == 1 ? (half ? ot : thr) : (t == mine ? thr : ot);
+                ff[t] = TILES == 1 ? (half ? of : (int)full) : (t == mine ? (int)full : of);
+                bdist[t] = kInitMin;
+                bk[t] = 0x7fffffff;
+            }
+            for (int ch = 0; ch < nchunks; ch++) {
+                stage(ch, 0);
+                staged();
+#pragma unroll 1
+                for (int b = 0; b < NB; b++) {
+                    const int blk = ch * NB + b;
+                    if (blk >= kblocks) break;
+                    block_values(0, b, acc);
+#pragma unroll
+                    for (int t = 0; t < TILES; t++) {
+                        if (!ff[t]) continue;
+                        unsigned w = 0;
+#pragma unroll
+                        for (int i = 0; i < 16; i++)
+                            if (pack_key(acc[t][i], (blk & 7) * 16 + i, keep) <= tt[t]) w |= 1u << i;
+                        const float *x = a.x + min(base + 32 * t + col, a.N - 1) * D;
+                        while (w) {
+                            const int i = __builtin_ctz(w);
+                            w &= w - 1;
+                            rescore(x, centre_of(blk * 16 + i, half), bdist[t], bk[t]);
+                        }
+                    }
+                }
+                __syncthreads();  // the buffer is free
+            }
+            stage(0, 0);
+            const float ad = own(bdist[0], bdist[L]), od = theirs(bdist[0], bdist[L]);
+            const int ak = own(bk[0], bk[L]), ok = theirs(bk[0], bk[L]);
+            if (full) {
+                const bool take = od < ad || (od == ad && ok < ak);
+                best_d = take ? od : ad;
+                best_k = take ? ok : ak;
+            }
+        }
+        if (live && !part) a.assign[p] = best_k == 0x7fffffff ? 0 : best_k;
+        if (live && multi) my_rescored++;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load to LDS outlives the workgroup
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) my_rescored += __shfl_xor(my_rescored, o, kWave);
+    if (lane == 0 && my_rescored) atomicAdd(rescored, (unsigned long long)my_rescored);
+}
+
+// The listed points of km_wide: four lanes a point, one candidate each, with
+// map1's exact arithmetic and tie rule.
+__global__ __launch_bounds__(256) void km_rescore(KmArgs a, const int *__restrict__ list,
+                                                  const int *__restrict__ listed)
+{
+    const int n = *listed, q = threadIdx.x % 4;
+    const bool vec = (a.D % 4) == 0 && ((uintptr_t)a.x % 16) == 0;
+    for (int i = blockIdx.x * 64 + threadIdx.x / 4; i < n; i += gridDim.x * 64) {
+        const int p = list[i];
+        const unsigned w = q < 2 ? (unsigned)a.assign[p] : __float_as_uint(a.mindist[p]);
+        int k = (int)(q & 1 ? w >> 16 : w & 0xffffu);
+        float d = kInitMin;
+        if (k < a.K) {
+            const float v = exact_dist(a.x + (int64_t)p * a.D, a.c + (int64_t)k * a.D, a.D, vec);
+            if (v < d) d = v;
+            else k = 0x7fffffff;
+        } else {
+            k = 0x7fffffff;
+        }
+#pragma unroll
+        for (int o = 1; o < 4; o <<= 1) {
+            const float od = __shfl_xor(d, o, kWave);
+            const int ok = __shfl_xor(k, o, kWave);
+            if (od < d || (od == d && ok < k)) {
+                d = od;
+                k = ok;
+            }
+        }
+        if (q == 0) a.assign[p] = k == 0x7fffffff ? 0 : k;
+    }
+}
+
 // ------------------------------------------------------------ update
 
 // One wavefront per centre: applies the Lloyd update from the reduction
@@ -886,6 +1279,68 @@ __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K,
     }
 }
 
+// The same update with the FP16 rows of the wide path: 2 KS + 1 fragments of 16
+// elements per centre: high parts of c^ = -2^a c, low parts, and n^ / 2^15 in
+// three parts.  A centre with a coordinate that is not finite is never map1's
+// nearest: its row is far, as the padding rows are.
+template <int KS>
+__global__ __launch_bounds__(256) void km_finalize_wide(float *__restrict__ c, int K, int K_pad, int D,
+                                                        unsigned long long *__restrict__ gsum,
+                                                        unsigned long long *__restrict__ gcnt,
+                                                        unsigned long long *__restrict__ gdsum, double inv_scale,
+                                                        int update, _Float16 *__restrict__ cb,
+                                                        float *__restrict__ cnorm, float sx,
+                                                        unsigned long long *__restrict__ csnap)
+{
+    constexpr int NS = 2 * KS + 1;
+    const int k = blockIdx.x * 4 + threadIdx.x / kWave;
+    const int lane = threadIdx.x % kWave;
+    if (k >= K_pad) return;
+    long long n = 0;
+    double ss = 0.0;
+    bool fine = k < K;
+    if (k < K) {
+        n = (long long)gcnt[k];
+        for (int d = lane; d < D; d += kWave) {
+            float v = c[(int64_t)k * D + d];
+            if (update && n > 0) v = (float)(((double)(long long)gsum[(int64_t)k * D + d] * inv_scale) / (double)n);
+            if (update) c[(int64_t)k * D + d] = v;
+            ss += (double)v * (double)v;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
+        fine = isfinite(ss) && isfinite((float)ss);
+    }
+    for (int d = lane; d < 16 * KS; d += kWave) {
+        const float v = fine && d < D ? -(c[(int64_t)k * D + d] * sx) : 0.0f;
+        const _Float16 h = (_Float16)v;
+        cb[frag_index(k, d, NS)] = h;
+        cb[frag_index(k, 16 * KS + d, NS)] = (_Float16)(v - (float)h);
+    }
+    if (lane < 16) {
+        const double nn = fine ? ss * (double)sx * (double)sx * (0.5 / kWideOne) : (double)kWideFar;
+        const _Float16 n1 = (_Float16)(float)nn;
+        const double r1 = nn - (double)(float)n1;
+        const _Float16 n2 = (_Float16)(float)r1;
+        const double r2 = r1 - (double)(float)n2;
+        _Float16 v = (_Float16)0.0f;
+        if (lane == 0) v = n1;
+        if (lane == 1) v = n2;
+        if (lane == 2) v = (_Float16)(float)r2;
+        cb[frag_index(k, 32 * KS + lane, NS)] = v;
+    }
+    if (k >= K) return;
+    if (lane == 0) {
+        cnorm[k] = fine ? (float)sqrt(ss) * 1.0001f : 0.0f;
+        if (csnap) csnap[k] = (unsigned long long)n;
+    }
+    for (int d = lane; d < D; d += kWave) gsum[(int64_t)k * D + d] = 0;
+    if (lane == 0) {
+        gcnt[k] = 0;
+        gdsum[k] = 0;
+    }
+}
+
 // 256 threads per workgroup.  Sixteen-byte loads, four in flight per thread,
 // when x is 16-byte aligned (else one float at a time); the workgroup's
 // maximum reaches *out by one atomic (atomics from every wavefront to one
@@ -923,36 +1378,37 @@ __global__ __launch_bounds__(256) void km_maxabs(const float *__restrict__ x, in
 
 // ------------------------------------------------------------ bucketed reduction
 //
-// For a reduction object too large for LDS the assignment kernels only
-// write assign/mindist, and the object is summed afterwards bucket by
-// bucket: points are counted per centre, the counts scanned, the point
-// indices scattered into their centre's bucket, and wavefronts walk the
-// buckets in runs of kRun positions, summing each centre's rows in
-// registers (the same fixed-point integers as the direct path, so the sums
-// are the same bit for bit) and adding them to the object once per centre
-// run -- about (N / kRun + K) * D atomics instead of N * (D + 2).
+// For a reduction object too large for LDS the assignment kernels only find
+// the centres, and the object is summed afterwards bucket by bucket: points
+// are counted per centre (each workgroup reserving its part of every bucket),
+// the counts scanned, the point indices scattered into their centre's bucket,
+// and wavefronts walk the buckets in runs of kRun positions, summing each
+// centre's rows in registers (the same fixed-point integers as the direct
+// path, so the sums are the same bit for bit) and adding them to the object
+// once per centre run -- about (N / kRun + K) * D atomics instead of
+// N * (D + 2).  The same walk computes min_dist, map1's exact distance to the
+// assigned centre.
 
 constexpr int kRun = 256;
 
-// cnt[k] += points assigned to k (LDS histogram per workgroup when K fits).
-__global__ __launch_bounds__(256) void km_bucket_count(const int32_t *__restrict__ assign, int64_t N, int K,
-                                                       int *__restrict__ cnt, int lds_hist)
+// Points [blockIdx.x * chunk, + chunk) of one workgroup: their number per
+// centre, and (lds_hist) where they start within the centre's bucket.
+__global__ __launch_bounds__(512) void km_bucket_count(const int32_t *__restrict__ assign, int64_t N, int K,
+                                                       int64_t chunk, int *__restrict__ cnt, int *__restrict__ part,
+                                                       int lds_hist)
 {
     extern __shared__ int hist[];
-    if (lds_hist) {
-        for (int k = threadIdx.x; k < K; k += blockDim.x) hist[k] = 0;
-        __syncthreads();
+    const int64_t p0 = (int64_t)blockIdx.x * chunk, p1 = min<int64_t>(N, p0 + chunk);
+    if (!lds_hist) {
+        for (int64_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) atomicAdd(&cnt[assign[p]], 1);
+        return;
     }
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < N; p += (int64_t)gridDim.x * blockDim.x) {
-        const int k = assign[p];
-        if (lds_hist) atomicAdd(&hist[k], 1);
-        else atomicAdd(&cnt[k], 1);
-    }
-    if (lds_hist) {
-        __syncthreads();
-        for (int k = threadIdx.x; k < K; k += blockDim.x)
-            if (hist[k]) atomicAdd(&cnt[k], hist[k]);
-    }
+    for (int k = threadIdx.x; k < K; k += blockDim.x) hist[k] = 0;
+    __syncthreads();
+    for (int64_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) atomicAdd(&hist[assign[p]], 1);
+    __syncthreads();
+    for (int k = threadIdx.x; k < K; k += blockDim.x)
+        part[(int64_t)blockIdx.x * K + k] = hist[k] ? atomicAdd(&cnt[k], hist[k]) : 0;
 }
 
 // One workgroup of 1024 threads: off[k] = exclusive prefix sum of cnt
@@ -983,65 +1439,155 @@ __global__ __launch_bounds__(1024) void km_bucket_scan(const int *__restrict__ c
 }
 
 // idx[slot] = p, each point into its centre's bucket (order within a bucket
-// is arbitrary: the sums are integers).
-__global__ __launch_bounds__(256) void km_bucket_scatter(const int32_t *__restrict__ assign, int64_t N,
-                                                         int *__restrict__ cur, int *__restrict__ idx)
+// is arbitrary: the sums are integers).  With the workgroups' parts the
+// cursors are in LDS; one returning global atomic per point took 0.24 ms for
+// 1 M points of 1,000 centres.
+__global__ __launch_bounds__(512) void km_bucket_scatter(const int32_t *__restrict__ assign, int64_t N, int K,
+                                                         int64_t chunk, const int *__restrict__ off,
+                                                         const int *__restrict__ part, int *__restrict__ cur,
+                                                         int *__restrict__ idx, int lds_hist)
 {
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < N; p += (int64_t)gridDim.x * blockDim.x)
-        idx[atomicAdd(&cur[assign[p]], 1)] = (int)p;
+    extern __shared__ int at[];
+    const int64_t p0 = (int64_t)blockIdx.x * chunk, p1 = min<int64_t>(N, p0 + chunk);
+    if (!lds_hist) {
+        for (int64_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) idx[atomicAdd(&cur[assign[p]], 1)] = (int)p;
+        return;
+    }
+    for (int k = threadIdx.x; k < K; k += blockDim.x) at[k] = off[k] + part[(int64_t)blockIdx.x * K + k];
+    __syncthreads();
+    for (int64_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) idx[atomicAdd(&at[assign[p]], 1)] = (int)p;
 }
 
-// One wavefront per run of kRun bucket positions: lanes hold dimensions
-// lane + 64t; each centre's points in the run are summed in registers and
-// added to the object when the centre changes (and at the run's end).
-template <int DT>
-__global__ __launch_bounds__(256) void km_bucket_sum(const float *__restrict__ x, const int *__restrict__ idx,
-                                                     const int32_t *__restrict__ assign,
-                                                     const float *__restrict__ mindist, int64_t N, int D, float scale,
-                                                     float dscale, unsigned long long *__restrict__ gsum,
-                                                     unsigned long long *__restrict__ gcnt,
-                                                     unsigned long long *__restrict__ gdsum)
+// One wavefront per run of kRun bucket positions, 64 points at a time and 32
+// dimensions of them: the rows go through LDS (eight lanes read 128 bytes of a
+// row), then each lane takes its point's 32 dimensions for the distance (FP32
+// in dimension order, as map1) and each half-wavefront's lane a dimension of
+// every other point for the sums.  The wavefronts of a workgroup do not wait
+// for each other.  One pass over the rows: bound by HBM (128 dimensions,
+// rows in bucket order).  Reading them with the lanes over the dimensions, one
+// point after another, took 0.52 ms for 1 M x 128, and the distances were
+// computed by the assignment kernel.
+constexpr int kRowsStride = 36;  // words per point: 16-byte aligned rows that spread over the banks
+
+template <int DP>
+__global__ __launch_bounds__(256) void km_bucket_rows(const float *__restrict__ x, const int *__restrict__ idx,
+                                                      const int32_t *__restrict__ assign, const float *__restrict__ c,
+                                                      float *__restrict__ mindist, int64_t N, int D, float scale,
+                                                      float dscale, unsigned long long *__restrict__ gsum,
+                                                      unsigned long long *__restrict__ gcnt,
+                                                      unsigned long long *__restrict__ gdsum)
 {
-    const int64_t run = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int lane = threadIdx.x % kWave;
-    const int64_t j0 = run * kRun;
-    if (j0 >= N) return;  // whole wavefronts
+    __shared__ float4 rows_[4][kWave * kRowsStride / 4];
+    const int lane = threadIdx.x % kWave, wv = pat::wave_in_block();
+    float *rows = (float *)rows_[wv];
+    const int64_t j0 = ((int64_t)blockIdx.x * 4 + wv) * kRun;
+    if (j0 >= N) return;  // whole wavefronts, no barrier below
     const int64_t j1 = min<int64_t>(N, j0 + kRun);
-    unsigned long long acc[DT], cnt = 0, dsum = 0;
+    const bool vec = (D % 4) == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)c % 16) == 0;
+    const int half = lane / 32, dim = lane % 32, sub = lane % 8;
+    unsigned long long acc[DP];
 #pragma unroll
-    for (int t = 0; t < DT; t++) acc[t] = 0;
-    int kc = assign[idx[j0]];
-    auto flush = [&](int k) {
-#pragma unroll
-        for (int t = 0; t < DT; t++) {
-            const int d = lane + kWave * t;
-            if (d < D && acc[t]) atomicAdd(&gsum[(int64_t)k * D + d], acc[t]);
-            acc[t] = 0;
-        }
-        if (lane == 0) {
-            atomicAdd(&gcnt[k], cnt);
-            atomicAdd(&gdsum[k], dsum);
-        }
-        cnt = 0;
-        dsum = 0;
+    for (int q = 0; q < DP; q++) acc[q] = 0;
+    auto flush = [&](int k, int q) {  // panel q's sums of centre k
+        const unsigned long long v = acc[q] + __shfl_xor(acc[q], 32, kWave);
+        const int d = 32 * q + dim;
+        if (half == 0 && d < D && v) atomicAdd(&gsum[(int64_t)k * D + d], v);
+        acc[q] = 0;
     };
-    for (int64_t j = j0; j < j1; j++) {
-        const int p = idx[j];
+    int kc = __builtin_amdgcn_readfirstlane(assign[idx[j0]]);  // the centre the sums belong to
+    for (int64_t j = j0; j < j1; j += kWave) {
+        const bool live = j + lane < j1;
+        const int p = idx[live ? j + lane : j1 - 1];
         const int k = assign[p];
-        if (k != kc) {  // uniform: every lane reads the same p
-            flush(kc);
-            kc = k;
-        }
-        const float *xp = x + (int64_t)p * D;
+        const unsigned long long have = __ballot(live);
+        float dist = 0.0f;
+        int kend = kc;
 #pragma unroll
-        for (int t = 0; t < DT; t++) {
-            const int d = lane + kWave * t;
-            if (d < D) acc[t] += to_fixed(xp[d], scale);
+        for (int q = 0; q < DP; q++) {
+            float4 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int64_t r = __shfl(p, 8 * i + lane / 8, kWave);
+                const int d = 32 * q + 4 * sub;
+                const float *xr = x + r * D + d;
+                v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (vec) {
+                    if (d < D) v[i] = *(const float4 *)xr;
+                } else {
+                    if (d < D) v[i].x = xr[0];
+                    if (d + 1 < D) v[i].y = xr[1];
+                    if (d + 2 < D) v[i].z = xr[2];
+                    if (d + 3 < D) v[i].w = xr[3];
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 8; i++) *(float4 *)(rows + (8 * i + lane / 8) * kRowsStride + 4 * sub) = v[i];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            // past D both the row and the centre give 0, and (0 - 0)^2 = +0
+            // changes no bit of the sum
+            const float *ck = c + (int64_t)k * D + 32 * q;
+#pragma unroll
+            for (int e = 0; e < 32; e += 4) {
+                if (32 * q + e < D) {
+                    const float4 xv = *(const float4 *)(rows + lane * kRowsStride + e);
+                    float4 cv = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (vec) {
+                        cv = *(const float4 *)(ck + e);
+                    } else {
+                        cv.x = ck[e];
+                        if (32 * q + e + 1 < D) cv.y = ck[e + 1];
+                        if (32 * q + e + 2 < D) cv.z = ck[e + 2];
+                        if (32 * q + e + 3 < D) cv.w = ck[e + 3];
+                    }
+                    float t = cv.x - xv.x;
+                    dist = dist + t * t;
+                    t = cv.y - xv.y;
+                    dist = dist + t * t;
+                    t = cv.z - xv.z;
+                    dist = dist + t * t;
+                    t = cv.w - xv.w;
+                    dist = dist + t * t;
+                }
+            }
+            // the points of one centre lie together
+            int kcur = kc;
+            for (unsigned long long rem = have; rem;) {
+                const int r0 = __ffsll((long long)rem) - 1;
+                const int kr = __shfl(k, r0, kWave);
+                const unsigned long long m = __ballot(k == kr) & rem;
+                const int r1 = r0 + __popcll(m);
+                if (kr != kcur) {
+                    flush(kcur, q);
+                    kcur = kr;
+                }
+                for (int r = r0 + ((r0 ^ half) & 1); r < r1; r += 2)
+                    acc[q] += to_fixed(rows[r * kRowsStride + dim], scale);
+                rem &= ~m;
+            }
+            kend = kcur;
         }
-        cnt++;
-        if (lane == 0) dsum += to_fixed(mindist[p], dscale);
+        kc = __builtin_amdgcn_readfirstlane(kend);
+        dist = sqrtf(dist);
+        const float md = dist < kInitMin ? dist : kInitMin;  // map1 starts from kInitMin
+        if (live) mindist[p] = md;
+        for (unsigned long long rem = have; rem;) {
+            const int kr = __shfl(k, __ffsll((long long)rem) - 1, kWave);
+            const unsigned long long m = __ballot(k == kr) & rem;
+            unsigned long long v = m >> lane & 1 ? to_fixed(md, dscale) : 0ull;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+            if (lane == 0) {
+                atomicAdd(&gcnt[kr], (unsigned long long)__popcll(m));
+                atomicAdd(&gdsum[kr], v);
+            }
+            rem &= ~m;
+        }
     }
-    flush(kc);
+#pragma unroll
+    for (int q = 0; q < DP; q++) flush(kc, q);
 }
 
 __global__ void km_zero_u64(unsigned long long *__restrict__ p, int64_t n)
@@ -1153,7 +1699,14 @@ int kmeans_prepare_kernels()
         (const void *)km_mfma<1, 8, 3, true, true>, (const void *)km_mfma<2, 8, 3, true, true>,
         (const void *)km_mfma<4, 4, 3, true, true>, (const void *)km_mfma<8, 2, 3, true, true>,
         (const void *)km_mfma<1, 8, 3, false, true>, (const void *)km_mfma<2, 8, 3, false, true>,
-        (const void *)km_mfma<4, 4, 3, false, true>, (const void *)km_mfma<8, 2, 3, false, true>};
+        (const void *)km_mfma<4, 4, 3, false, true>, (const void *)km_mfma<8, 2, 3, false, true>,
+        // FP16 high and low parts, for objects beyond LDS
+        (const void *)km_wide<1, 8, 1, true>, (const void *)km_wide<2, 8, 1, true>, (const void *)km_wide<4, 8, 1, true>,
+        (const void *)km_wide<8, 4, 1, true>, (const void *)km_wide<1, 8, 1, false>, (const void *)km_wide<2, 8, 1, false>,
+        (const void *)km_wide<4, 8, 1, false>, (const void *)km_wide<8, 4, 1, false>, (const void *)km_wide<1, 8, 2, true>,
+        (const void *)km_wide<2, 8, 2, true>, (const void *)km_wide<4, 8, 2, true>, (const void *)km_wide<8, 4, 2, true>,
+        (const void *)km_wide<1, 8, 2, false>, (const void *)km_wide<2, 8, 2, false>, (const void *)km_wide<4, 8, 2, false>,
+        (const void *)km_wide<8, 4, 2, false>};
     for (const void *f : fns)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g_lds_limit) != hipSuccess)
             (void)hipGetLastError();
@@ -1169,32 +1722,45 @@ bool kmeans_object_in_lds(int K, int D)
     return object_bytes(K, D) <= std::min<int64_t>(96 * 1024, g_lds_limit - 32 * 1024);
 }
 
-// The bucketed reduction after an assignment pass (see km_bucket_sum).
+// Largest K counted and placed in LDS by the bucketed reduction (32 KB).
+constexpr int kBucketLdsK = 8192;
+
+// Workgroups that count and place the points: one per 4,096 up to two per CU.
+static int bucket_wgs(int64_t N, int cus)
+{
+    return (int)std::max<int64_t>(1, std::min<int64_t>((N + 4095) / 4096, 2LL * cus));
+}
+
+int64_t kmeans_bucket_part_words(int64_t N, int K, int cus)
+{
+    return K <= kBucketLdsK ? (int64_t)bucket_wgs(N, cus) * K : 1;
+}
+
+// The bucketed reduction after an assignment pass (see km_bucket_rows).
 static int bucket_reduce(const KmDev &d, hipStream_t st)
 {
     const int K = d.K;
-    hipLaunchKernelGGL(km_zero_i32, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, st, d.bcnt, (int64_t)K);
+    // the counts, and km_wide's list for the next pass
+    hipLaunchKernelGGL(km_zero_i32, dim3((unsigned)(K / 256 + 1)), dim3(256), 0, st, d.bcnt, (int64_t)K + 1);
     PAT_LAUNCH_CHECK();
-    const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>((d.N + 255) / 256, 8LL * d.cus));
-    const int lds_hist = K <= 8192;
-    hipLaunchKernelGGL(km_bucket_count, dim3(g), dim3(256), lds_hist ? (size_t)4 * K : 0, st, (const int32_t *)d.assign,
-                       d.N, K, d.bcnt, lds_hist);
+    const int wgs = bucket_wgs(d.N, d.cus);
+    const int64_t chunk = (d.N + wgs - 1) / wgs;
+    const int lds_hist = K <= kBucketLdsK;
+    const size_t lds = lds_hist ? (size_t)4 * K : 0;
+    hipLaunchKernelGGL(km_bucket_count, dim3((unsigned)wgs), dim3(512), lds, st, (const int32_t *)d.assign, d.N, K, chunk,
+                       d.bcnt, d.bpart, lds_hist);
     PAT_LAUNCH_CHECK();
     hipLaunchKernelGGL(km_bucket_scan, dim3(1), dim3(1024), 0, st, (const int *)d.bcnt, K, d.boff, d.bcur);
     PAT_LAUNCH_CHECK();
-    hipLaunchKernelGGL(km_bucket_scatter, dim3(g), dim3(256), 0, st, (const int32_t *)d.assign, d.N, d.bcur, d.bidx);
+    hipLaunchKernelGGL(km_bucket_scatter, dim3((unsigned)wgs), dim3(512), lds, st, (const int32_t *)d.assign, d.N, K,
+                       chunk, (const int *)d.boff, (const int *)d.bpart, d.bcur, d.bidx, lds_hist);
     PAT_LAUNCH_CHECK();
-    const int64_t runs = (d.N + kRun - 1) / kRun;
-    const unsigned gs = (unsigned)((runs + 3) / 4);
+    const unsigned gs = (unsigned)((d.N + 4 * kRun - 1) / (4 * kRun));
     const float scale = ldexpf(1.0f, d.shift), dscale = ldexpf(1.0f, d.dshift);
-    if (d.D <= 64)
-        hipLaunchKernelGGL(km_bucket_sum<1>, dim3(gs), dim3(256), 0, st, d.x, (const int *)d.bidx,
-                           (const int32_t *)d.assign, (const float *)d.mindist, d.N, d.D, scale, dscale, d.gsum, d.gcnt,
-                           d.gdsum);
-    else
-        hipLaunchKernelGGL(km_bucket_sum<2>, dim3(gs), dim3(256), 0, st, d.x, (const int *)d.bidx,
-                           (const int32_t *)d.assign, (const float *)d.mindist, d.N, d.D, scale, dscale, d.gsum, d.gcnt,
-                           d.gdsum);
+    auto rows = d.D <= 32 ? km_bucket_rows<1>
+                          : (d.D <= 64 ? km_bucket_rows<2> : (d.D <= 96 ? km_bucket_rows<3> : km_bucket_rows<4>));
+    hipLaunchKernelGGL(rows, dim3(gs), dim3(256), 0, st, d.x, (const int *)d.bidx, (const int32_t *)d.assign,
+                       (const float *)d.c, d.mindist, d.N, d.D, scale, dscale, d.gsum, d.gcnt, d.gdsum);
     PAT_LAUNCH_CHECK();
     return PAT_OK;
 }
@@ -1210,6 +1776,14 @@ int kmeans_finalize(const KmDev &d, int update, hipStream_t st)
 {
     const double inv = ldexp(1.0, -d.shift);
     const dim3 g((unsigned)((d.K_pad + 3) / 4)), b(256);
+    if (d.wide) {
+        auto f = d.KS == 1 ? km_finalize_wide<1>
+                           : (d.KS == 2 ? km_finalize_wide<2> : (d.KS == 4 ? km_finalize_wide<4> : km_finalize_wide<8>));
+        hipLaunchKernelGGL(f, g, b, 0, st, d.c, d.K, d.K_pad, d.D, d.gsum, d.gcnt, d.gdsum, inv, update,
+                           (_Float16 *)d.cb, d.cnorm, ldexpf(1.0f, d.wexp), d.csnap);
+        PAT_LAUNCH_CHECK();
+        return PAT_OK;
+    }
 #define PAT_KF(KS_, NT_)                                                                                               \
     hipLaunchKernelGGL((km_finalize<KS_, NT_>), g, b, 0, st, d.c, d.K, d.K_pad, d.D, d.gsum, d.gcnt, d.gdsum, inv,    \
                        update, (__bf16 *)d.cb, d.cnorm, d.csnap)
@@ -1290,8 +1864,76 @@ bool kmeans_gc_for(int K, int D) { return kmeans_ks_for(D) != 0 && kmeans_nt_for
 
 bool kmeans_mfma_fits(int K, int D) { return kmeans_ks_for(D) != 0 && K <= 65536; }
 
+// Words (FP16) of the wide path's rows.
+int64_t kmeans_wide_row_words(int K_pad, int D) { return (int64_t)K_pad * 16 * (2 * kmeans_ks_for(D) + 1); }
+
+// Exponent a of the wide path's scale: 2^a times the largest coordinate lies
+// below 2^10 (2^126 is the largest FP32 power of two with an FP32 inverse).
+int kmeans_wide_exp(float maxabs)
+{
+    int e = 0;
+    if (maxabs > 0) (void)frexpf(maxabs, &e);
+    return std::min(126, 10 - e);
+}
+
+// The error bound of km_wide's values (derived there).
+static WideBound wide_bound(const KmDev &d)
+{
+    const double u = ldexp(1.0, -11), e = ldexp(1.0, -14), g = ldexp(1.0, -23), sd = sqrt((double)d.D), KS = d.KS;
+    const double over = 1.02;
+    WideBound b;
+    b.sx = ldexpf(1.0f, d.wexp);
+    b.c_dot = (float)(over * (3 * u * u + g * 32 * KS * 2 * u + g * 16 * KS * (1 + 4 * u) + g * 16 * (1 + 4 * u)));
+    b.c_sum = (float)(over * (e * sd * (1 + 2 * u) * (1 + g * (48 * KS + 16) * 2)));
+    b.c_cc = (float)(over * 0.5 * (u * u * u + g * 16 * (1 + u)));
+    b.c_abs = (float)(over * (d.D * e * e + 2.0));
+    b.c_ref = (float)((3.0 + d.D + 16.0) * ldexp(1.0, -24) * 1.01);
+    b.ref_abs = (float)std::min(1e30, ldexp(1e-30, 2 * d.wexp - 1));
+    b.far = (float)std::min(1e38, ldexp(0.98 * kInitMin * kInitMin, 2 * d.wexp - 1));
+    return b;
+}
+
+// Blocks of 32 centres per LDS chunk of km_wide: two chunks of up to 72 KiB.
+static int wide_nb(int ks) { return ks == 8 ? 4 : 8; }
+
+static int assign_wide(const KmDev &d, hipStream_t st)
+{
+    const KmArgs a = make_args(d);
+    const WideBound bd = wide_bound(d);
+    const size_t lds = 2 * (size_t)wide_nb(d.KS) * (2 * d.KS + 1) * 1024;
+    PAT_REQUIRE((int64_t)lds <= g_lds_limit, PAT_ERR_UNSUPPORTED, "kmeans: %zu bytes of LDS requested, device allows %lld",
+                lds, (long long)g_lds_limit);
+    // two tiles per wavefront (each centre fragment feeds two MFMAs) where
+    // that leaves every CU a workgroup, else one
+    const bool two = d.N >= 512LL * d.cus;
+    const int64_t per = two ? 512 : 256;
+    const unsigned grid = (unsigned)std::min<int64_t>((d.N + per - 1) / per, d.cus);
+    const bool tail = d.D != 16 * d.KS || ((uintptr_t)d.x % 16) != 0;
+#define PAT_KW(KS_, NB_)                                                                                               \
+    do {                                                                                                               \
+        auto k = two ? (tail ? km_wide<KS_, NB_, 2, true> : km_wide<KS_, NB_, 2, false>)                               \
+                     : (tail ? km_wide<KS_, NB_, 1, true> : km_wide<KS_, NB_, 1, false>);                              \
+        hipLaunchKernelGGL(k, dim3(grid), dim3(512), lds, st, a, (const _Float16 *)d.cb, d.cnorm, d.K_pad, bd,        \
+                           d.bidx, d.bcnt + d.K, d.rescored);                                                          \
+    } while (0)
+    switch (d.KS) {
+    case 1: PAT_KW(1, 8); break;
+    case 2: PAT_KW(2, 8); break;
+    case 4: PAT_KW(4, 8); break;
+    case 8: PAT_KW(8, 4); break;
+    default: pat::set_error("kmeans: D too large"); return PAT_ERR_UNSUPPORTED;
+    }
+#undef PAT_KW
+    PAT_LAUNCH_CHECK();
+    hipLaunchKernelGGL(km_rescore, dim3((unsigned)std::min<int64_t>((d.N + 63) / 64, 4LL * d.cus)), dim3(256), 0, st, a,
+                       (const int *)d.bidx, (const int *)(d.bcnt + d.K));
+    PAT_LAUNCH_CHECK();
+    return bucket_reduce(d, st);
+}
+
 int kmeans_assign_mfma(const KmDev &d, hipStream_t st)
 {
+    if (d.wide) return assign_wide(d, st);
     KmArgs a = make_args(d);
     PAT_REQUIRE(d.NT == 1 || d.NT == 3, PAT_ERR_UNSUPPORTED, "kmeans: K=%d, D=%d too large for the MFMA path", d.K,
                 d.D);

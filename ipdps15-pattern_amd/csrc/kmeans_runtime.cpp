@@ -28,7 +28,8 @@ struct pat_kmeans {
     int mode = PAT_KM_MFMA;
     bool own_x = false;
     float *xbuf = nullptr;
-    void *rowbuf = nullptr;  // BF16 rows
+    void *rowbuf = nullptr;   // BF16 rows
+    void *widebuf = nullptr;  // FP16 rows (wide path)
     unsigned long long *maxbits = nullptr;
     unsigned long long *snap = nullptr;  // last pass's reduction object (K*D + 2K)
     hipStream_t stream = nullptr;
@@ -64,7 +65,7 @@ struct pat_kmeans {
         for (void *p : {(void *)xbuf, (void *)d.c, (void *)d.assign, (void *)d.mindist, (void *)d.gsum, (void *)d.gcnt,
                         (void *)d.gdsum, (void *)d.csnap, rowbuf, (void *)d.cnorm, (void *)d.rescored,
                         (void *)maxbits, (void *)snap, (void *)d.bidx, (void *)d.bcnt, (void *)d.boff,
-                        (void *)d.bcur})
+                        (void *)d.bcur, (void *)d.bpart, widebuf})
             if (p) (void)pat::dev_free(p);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -179,9 +180,16 @@ int setup(pat_kmeans *h, const float *x, int64_t n, int d, int k, int mode, int 
     D.bucketed = !pat::kmeans_object_in_lds(k, d) && n < (1LL << 31);
     if (D.bucketed) {
         PAT_TRY(amalloc((void **)&D.bidx, sizeof(int) * (size_t)n));
-        PAT_TRY(amalloc((void **)&D.bcnt, sizeof(int) * (size_t)k));
+        PAT_TRY(amalloc((void **)&D.bcnt, sizeof(int) * ((size_t)k + 1)));
+        PAT_HIP(hipMemsetAsync(D.bcnt, 0, sizeof(int) * ((size_t)k + 1), h->stream));
         PAT_TRY(amalloc((void **)&D.boff, sizeof(int) * ((size_t)k + 1)));
         PAT_TRY(amalloc((void **)&D.bcur, sizeof(int) * (size_t)k));
+        PAT_TRY(amalloc((void **)&D.bpart, sizeof(int) * (size_t)pat::kmeans_bucket_part_words(n, k, D.cus)));
+        // the assignment then leaves min_dist to the reduction, and its FP16
+        // form is the faster one for every such shape
+        PAT_TRY(amalloc(&h->widebuf, 2 * (size_t)pat::kmeans_wide_row_words(D.K_pad, d)));
+        D.wide = 1;
+        D.cb = h->widebuf;
     }
     PAT_TRY(amalloc((void **)&D.rescored, 8));
     PAT_TRY(amalloc((void **)&h->maxbits, 8));
@@ -195,6 +203,7 @@ int setup(pat_kmeans *h, const float *x, int64_t n, int d, int k, int mode, int 
     PAT_HIP(hipStreamSynchronize(h->stream));
     unsigned int bits = (unsigned int)mb;
     memcpy(&h->maxabs, &bits, 4);
+    D.wexp = pat::kmeans_wide_exp(h->maxabs);
     D.shift = pat::kmeans_fixed_shift(n, h->maxabs);
     D.dshift = pat::kmeans_fixed_shift(n, (float)(2.0 * (double)h->maxabs * std::sqrt((double)d)));
     // the kernels scale by 2^shift in FP32
@@ -208,7 +217,7 @@ int setup(pat_kmeans *h, const float *x, int64_t n, int d, int k, int mode, int 
     PAT_TRY(pat::kmeans_finalize(D, 0, h->stream));
     PAT_HIP(hipStreamSynchronize(h->stream));
     // timed only where a pass is long enough to pay for six trial passes
-    if (mode == PAT_KM_MFMA && !D.gc && D.NT == 3 && n >= (1 << 20) && pat::tuning_enabled()) PAT_TRY(tune_terms(h));
+    if (mode == PAT_KM_MFMA && !D.wide && !D.gc && D.NT == 3 && n >= (1 << 20) && pat::tuning_enabled()) PAT_TRY(tune_terms(h));
     return PAT_OK;
 }
 
@@ -267,8 +276,10 @@ int pat_kmeans_set_terms(pat_kmeans *h, int terms)
     const int fits = pat::kmeans_nt_for(D.K, D.D);  // 3: both forms fit, 1: only one term, 0: neither
     PAT_REQUIRE(!D.gc && (fits == 3 || (fits == 1 && terms == 1)), PAT_ERR_UNSUPPORTED,
                 "pat_kmeans_set_terms: %d-term rows for K = %d, D = %d do not fit in LDS", terms, D.K, D.D);
-    if (D.NT != terms) {
+    if (D.NT != terms || D.wide) {
         D.NT = terms;
+        D.wide = 0;
+        D.cb = h->rowbuf;
         PAT_TRY(pat::kmeans_finalize(D, 0, h->stream));
         PAT_HIP(hipStreamSynchronize(h->stream));
         h->drop_graphs();
@@ -286,6 +297,16 @@ int pat_kmeans_get_terms(pat_kmeans *h, int *terms)
 int pat_kmeans_set_centroids(pat_kmeans *h, const float *c)
 {
     PAT_REQUIRE(h && c, PAT_ERR_INVALID, "pat_kmeans_set_centroids: null argument");
+    if (h->d.wide) {  // the rows' scale covers the points and the centres
+        float m = h->maxabs;
+        for (int64_t i = 0; i < (int64_t)h->d.K * h->d.D; i++)
+            if (std::isfinite(c[i])) m = std::max(m, std::fabs(c[i]));
+        const int e = pat::kmeans_wide_exp(m);
+        if (e != h->d.wexp) {
+            h->d.wexp = e;
+            h->drop_graphs();
+        }
+    }
     PAT_HIP(hipMemcpyAsync(h->d.c, c, sizeof(float) * (size_t)h->d.K * h->d.D, hipMemcpyHostToDevice, h->stream));
     PAT_TRY(pat::kmeans_finalize(h->d, 0, h->stream));
     PAT_HIP(hipStreamSynchronize(h->stream));

@@ -139,8 +139,11 @@ struct pat_serve {
         case PAT_JOB_KMEANS: {
             const int64_t kd = (int64_t)j.k * j.dim;
             // points, assignments and distances, bucket indices (bucketed
-            // reduction), rows and the reduction object, per-centre arrays
-            return j.size * j.dim * 4 + 12 * j.size + 40 * kd + 80 * (int64_t)j.k + MB;
+            // reduction), rows and the reduction object, per-centre arrays,
+            // bucket starts per workgroup of the bucketed reduction
+            const int64_t parts =
+                pat::kmeans_object_in_lds(j.k, j.dim) ? 0 : 4 * pat::kmeans_bucket_part_words(j.size, j.k, 256);
+            return j.size * j.dim * 4 + 12 * j.size + 40 * kd + 80 * (int64_t)j.k + parts + MB;
         }
         default: return 0;
         }

@@ -219,3 +219,51 @@ def test_kmeans_workload_full_size(pa, orc, gpu):
     kp.run(20)
     assert np.array_equal(kp.centroids(), c)
     kp.close()
+
+
+@pytest.mark.parametrize("n,d,k", [(700, 128, 97), (513, 128, 200), (2000, 128, 289), (5000, 65, 257), (4100, 32, 385),
+                                   (3000, 16, 700), (4000, 8, 2049), (1500, 5, 1500), (9000, 97, 260)])
+@pytest.mark.parametrize("scale", [1.0, 1e-12, 3e15])
+def test_wide_path_bitexact(pa, orc, gpu, n, d, k, scale):
+    """Objects beyond LDS (FP16 high and low parts): partial blocks, chunks and
+    groups of centres, one and two tiles a wavefront, rows with a tail, points
+    of small and large magnitude; then centres far outside the points' range
+    and one that is not finite, which no point may choose."""
+    x = (pa.gen_gmm(n, d, max(1, k // 2), sigma=1.0, seed=n + d + k) * np.float32(scale)).astype(np.float32)
+    km = pa.KMeans(x, k, mode=1)
+    km.run(2)
+    c, a, md = km.get()
+    sums, counts, dsums, s, ds = km.get_object()
+    *_, (c1, ra, rmd, rsums, rcounts, rdsum) = oracle_iters(orc, pa, x, k, 2)
+    assert np.array_equal(a, ra) and np.array_equal(md, rmd)
+    assert np.array_equal(sums, rsums) and np.array_equal(counts, rcounts) and np.array_equal(dsums, rdsum)
+    assert np.array_equal(c, orc.kmeans_update(rsums, rcounts, s, c1))
+    if scale == 1.0:
+        far = x[:k].copy()
+        far[0] *= 4096.0
+        far[1, 0] = np.inf
+        far[2, -1] = np.nan
+        km.set_centroids(far)
+        km.run(1)
+        _, a, md = km.get()
+        ra, rmd = orc.kmeans_assign(x, far)
+        assert np.array_equal(a, ra) and np.array_equal(md, rmd)
+    km.close()
+
+
+def test_wide_path_two_tiles(pa, orc, gpu):
+    """Enough points for two tiles per wavefront, the last workgroups ragged,
+    and centres that repeat: three equal keys, so the second pass."""
+    x = pa.gen_gmm(512 * 256 + 333, 33, 150, sigma=1.0, seed=3)
+    k = 300
+    for repeat in (False, True):
+        c = x[:k].copy()
+        if repeat:
+            c[100:140] = c[5]
+        km = pa.KMeans(x, k, mode=1)
+        km.set_centroids(c)
+        km.run(1)
+        _, a, md = km.get()
+        km.close()
+        ra, rmd = orc.kmeans_assign(x, c)
+        assert np.array_equal(a, ra) and np.array_equal(md, rmd)
