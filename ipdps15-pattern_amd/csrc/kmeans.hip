@@ -1213,6 +1213,32 @@ __global__ __launch_bounds__(256) void km_rescore(KmArgs a, const int *__restric
 
 // ------------------------------------------------------------ update
 
+// Centre k's part of the reduction object, by its wavefront: an update keeps
+// it in snap (K x D sums, K counts, K distance sums), then it is cleared for
+// the next pass (a fill, not a memset, so that the sequence can be captured).
+// Ten iterations of 20,000 x 8, K 16: 256 us, 281 with three copies (a graph
+// node each) before the update kernel.
+__device__ __forceinline__ void retire_object(int k, int lane, int K, int D, unsigned long long *__restrict__ gsum,
+                                              unsigned long long *__restrict__ gcnt,
+                                              unsigned long long *__restrict__ gdsum, int update,
+                                              unsigned long long *__restrict__ snap)
+{
+    const int64_t KD = (int64_t)K * D;
+    for (int d = lane; d < D; d += kWave) {
+        const int64_t i = (int64_t)k * D + d;
+        if (update) snap[i] = gsum[i];
+        gsum[i] = 0;
+    }
+    if (lane == 0) {
+        if (update) {
+            snap[KD + k] = gcnt[k];
+            snap[KD + K + k] = gdsum[k];
+        }
+        gcnt[k] = 0;
+        gdsum[k] = 0;
+    }
+}
+
 // One wavefront per centre: applies the Lloyd update from the reduction
 // object (c = (sum * 2^-s) / count in FP64, rounded to FP32; empty clusters
 // keep their centre), writes the BF16 MFMA row and the norm, and clears the
@@ -1223,7 +1249,7 @@ __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K,
                                                    unsigned long long *__restrict__ gcnt,
                                                    unsigned long long *__restrict__ gdsum, double inv_scale,
                                                    int update, __bf16 *__restrict__ cb, float *__restrict__ cnorm,
-                                                   unsigned long long *__restrict__ csnap)
+                                                   unsigned long long *__restrict__ snap)
 {
     constexpr int KW = 16 * (NT * KS + 1);
     constexpr int NB = 16 * NT * KS;  // first norm column
@@ -1266,17 +1292,8 @@ __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K,
         if (lane == 2) v = n3;
         cb[frag_index(k, NB + lane, KW / 16)] = v;
     }
-    if (lane == 0) {
-        cnorm[k] = (float)sqrt(ss) * 1.0001f;
-        if (csnap) csnap[k] = (unsigned long long)n;
-    }
-    // clear the reduction object for the next pass (a fill, not a memset, so
-    // the sequence can be captured in a graph)
-    for (int d = lane; d < D; d += kWave) gsum[(int64_t)k * D + d] = 0;
-    if (lane == 0) {
-        gcnt[k] = 0;
-        gdsum[k] = 0;
-    }
+    if (lane == 0) cnorm[k] = (float)sqrt(ss) * 1.0001f;
+    retire_object(k, lane, K, D, gsum, gcnt, gdsum, update, snap);
 }
 
 // The same update with the FP16 rows of the wide path: 2 KS + 1 fragments of 16
@@ -1290,7 +1307,7 @@ __global__ __launch_bounds__(256) void km_finalize_wide(float *__restrict__ c, i
                                                         unsigned long long *__restrict__ gdsum, double inv_scale,
                                                         int update, _Float16 *__restrict__ cb,
                                                         float *__restrict__ cnorm, float sx,
-                                                        unsigned long long *__restrict__ csnap)
+                                                        unsigned long long *__restrict__ snap)
 {
     constexpr int NS = 2 * KS + 1;
     const int k = blockIdx.x * 4 + threadIdx.x / kWave;
@@ -1330,15 +1347,8 @@ __global__ __launch_bounds__(256) void km_finalize_wide(float *__restrict__ c, i
         cb[frag_index(k, 32 * KS + lane, NS)] = v;
     }
     if (k >= K) return;
-    if (lane == 0) {
-        cnorm[k] = fine ? (float)sqrt(ss) * 1.0001f : 0.0f;
-        if (csnap) csnap[k] = (unsigned long long)n;
-    }
-    for (int d = lane; d < D; d += kWave) gsum[(int64_t)k * D + d] = 0;
-    if (lane == 0) {
-        gcnt[k] = 0;
-        gdsum[k] = 0;
-    }
+    if (lane == 0) cnorm[k] = fine ? (float)sqrt(ss) * 1.0001f : 0.0f;
+    retire_object(k, lane, K, D, gsum, gcnt, gdsum, update, snap);
 }
 
 // 256 threads per workgroup.  Sixteen-byte loads, four in flight per thread,
@@ -1780,13 +1790,13 @@ int kmeans_finalize(const KmDev &d, int update, hipStream_t st)
         auto f = d.KS == 1 ? km_finalize_wide<1>
                            : (d.KS == 2 ? km_finalize_wide<2> : (d.KS == 4 ? km_finalize_wide<4> : km_finalize_wide<8>));
         hipLaunchKernelGGL(f, g, b, 0, st, d.c, d.K, d.K_pad, d.D, d.gsum, d.gcnt, d.gdsum, inv, update,
-                           (_Float16 *)d.cb, d.cnorm, ldexpf(1.0f, d.wexp), d.csnap);
+                           (_Float16 *)d.cb, d.cnorm, ldexpf(1.0f, d.wexp), d.snap);
         PAT_LAUNCH_CHECK();
         return PAT_OK;
     }
 #define PAT_KF(KS_, NT_)                                                                                               \
     hipLaunchKernelGGL((km_finalize<KS_, NT_>), g, b, 0, st, d.c, d.K, d.K_pad, d.D, d.gsum, d.gcnt, d.gdsum, inv,    \
-                       update, (__bf16 *)d.cb, d.cnorm, d.csnap)
+                       update, (__bf16 *)d.cb, d.cnorm, d.snap)
     const int code = d.KS * 4 + d.NT;
     switch (code) {
     case 1 * 4 + 1: PAT_KF(1, 1); break;

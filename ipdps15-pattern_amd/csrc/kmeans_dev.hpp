@@ -19,7 +19,8 @@ struct KmDev {
     int shift, dshift;    // fixed-point scales 2^shift (coordinates), 2^dshift (distances)
     int32_t *assign;      // N
     float *mindist;       // N
-    unsigned long long *gsum, *gcnt, *gdsum, *csnap;  // reduction object (K x D, K, K), count snapshot
+    unsigned long long *gsum, *gcnt, *gdsum;  // reduction object (K x D, K, K)
+    unsigned long long *snap;                 // last pass's reduction object (K x D + 2 K)
     void *cb;             // MFMA rows: BF16, K_pad x 16*(NT*KS+1), or FP16, K_pad x 16*(2*KS+1) (wide)
     float *cnorm;         // ||c_k|| (rounded up)
     unsigned long long *rescored;  // points with more than one candidate

@@ -31,7 +31,6 @@ struct pat_kmeans {
     void *rowbuf = nullptr;   // BF16 rows
     void *widebuf = nullptr;  // FP16 rows (wide path)
     unsigned long long *maxbits = nullptr;
-    unsigned long long *snap = nullptr;  // last pass's reduction object (K*D + 2K)
     hipStream_t stream = nullptr;
     float maxabs = 0.0f;
     int iters_done = 0;
@@ -44,16 +43,12 @@ struct pat_kmeans {
         graphs.clear();
     }
 
-    // One Lloyd iteration: assignment + accumulation, snapshot of the
-    // reduction object, centre update (which also clears the object).
+    // One Lloyd iteration: assignment + accumulation, centre update (which
+    // also keeps and clears the reduction object).
     int enqueue_iter(hipStream_t s)
     {
         if (mode == PAT_KM_MFMA) PAT_TRY(pat::kmeans_assign_mfma(d, s));
         else PAT_TRY(pat::kmeans_assign_plain(d, s));
-        const int64_t KD = (int64_t)d.K * d.D;
-        PAT_HIP(hipMemcpyAsync(snap, d.gsum, 8 * KD, hipMemcpyDeviceToDevice, s));
-        PAT_HIP(hipMemcpyAsync(snap + KD, d.gcnt, 8 * (size_t)d.K, hipMemcpyDeviceToDevice, s));
-        PAT_HIP(hipMemcpyAsync(snap + KD + d.K, d.gdsum, 8 * (size_t)d.K, hipMemcpyDeviceToDevice, s));
         PAT_TRY(pat::kmeans_finalize(d, 1, s));
         return PAT_OK;
     }
@@ -63,8 +58,8 @@ struct pat_kmeans {
         if (stream) (void)hipStreamSynchronize(stream);
         drop_graphs();
         for (void *p : {(void *)xbuf, (void *)d.c, (void *)d.assign, (void *)d.mindist, (void *)d.gsum, (void *)d.gcnt,
-                        (void *)d.gdsum, (void *)d.csnap, rowbuf, (void *)d.cnorm, (void *)d.rescored,
-                        (void *)maxbits, (void *)snap, (void *)d.bidx, (void *)d.bcnt, (void *)d.boff,
+                        (void *)d.gdsum, rowbuf, (void *)d.cnorm, (void *)d.rescored,
+                        (void *)maxbits, (void *)d.snap, (void *)d.bidx, (void *)d.bcnt, (void *)d.boff,
                         (void *)d.bcur, (void *)d.bpart, widebuf})
             if (p) (void)pat::dev_free(p);
         if (stream) (void)hipStreamDestroy(stream);
@@ -172,7 +167,6 @@ int setup(pat_kmeans *h, const float *x, int64_t n, int d, int k, int mode, int 
     PAT_TRY(amalloc((void **)&D.gsum, 8 * (size_t)k * d));
     PAT_TRY(amalloc((void **)&D.gcnt, 8 * (size_t)k));
     PAT_TRY(amalloc((void **)&D.gdsum, 8 * (size_t)k));
-    PAT_TRY(amalloc((void **)&D.csnap, 8 * (size_t)k));
     PAT_TRY(amalloc(&h->rowbuf, 2 * (size_t)D.K_pad * 16 * (D.NT * D.KS + 1)));
     D.cb = h->rowbuf;
     PAT_TRY(amalloc((void **)&D.cnorm, sizeof(float) * (size_t)k));
@@ -193,7 +187,7 @@ int setup(pat_kmeans *h, const float *x, int64_t n, int d, int k, int mode, int 
     }
     PAT_TRY(amalloc((void **)&D.rescored, 8));
     PAT_TRY(amalloc((void **)&h->maxbits, 8));
-    PAT_TRY(amalloc((void **)&h->snap, 8 * ((size_t)k * d + 2 * (size_t)k)));
+    PAT_TRY(amalloc((void **)&D.snap, 8 * ((size_t)k * d + 2 * (size_t)k)));
     // centres start as the first k points
     PAT_HIP(hipMemcpyAsync(D.c, D.x, sizeof(float) * (size_t)k * d, hipMemcpyDeviceToDevice, h->stream));
     // fixed-point scales from max |x|
@@ -372,14 +366,6 @@ int pat_kmeans_run_timed(pat_kmeans *h, int iters, float *total_ms, float *assig
         (void)hipEventRecord(ev[1 + 2 * i], h->stream);
         rc = h->mode == PAT_KM_MFMA ? pat::kmeans_assign_mfma(h->d, h->stream) : pat::kmeans_assign_plain(h->d, h->stream);
         (void)hipEventRecord(ev[2 + 2 * i], h->stream);
-        if (rc != PAT_OK) break;
-        const int64_t KD = (int64_t)h->d.K * h->d.D;
-        if (hipMemcpyAsync(h->snap, h->d.gsum, 8 * KD, hipMemcpyDeviceToDevice, h->stream) != hipSuccess ||
-            hipMemcpyAsync(h->snap + KD, h->d.gcnt, 8 * (size_t)h->d.K, hipMemcpyDeviceToDevice, h->stream) !=
-                hipSuccess ||
-            hipMemcpyAsync(h->snap + KD + h->d.K, h->d.gdsum, 8 * (size_t)h->d.K, hipMemcpyDeviceToDevice,
-                           h->stream) != hipSuccess)
-            rc = PAT_ERR_HIP;
         if (rc == PAT_OK) rc = pat::kmeans_finalize(h->d, 1, h->stream);
     }
     (void)hipEventRecord(ev[2 * (size_t)iters + 1], h->stream);
@@ -412,9 +398,9 @@ int pat_kmeans_get_object(pat_kmeans *h, int64_t *sums, int64_t *counts, int64_t
     PAT_REQUIRE(h, PAT_ERR_INVALID, "pat_kmeans_get_object: null handle");
     PAT_REQUIRE(h->iters_done > 0, PAT_ERR_STATE, "pat_kmeans_get_object: no pass has run");
     const int64_t KD = (int64_t)h->d.K * h->d.D;
-    if (sums) PAT_HIP(hipMemcpyAsync(sums, h->snap, 8 * KD, hipMemcpyDeviceToHost, h->stream));
-    if (counts) PAT_HIP(hipMemcpyAsync(counts, h->snap + KD, 8 * (size_t)h->d.K, hipMemcpyDeviceToHost, h->stream));
-    if (dsums) PAT_HIP(hipMemcpyAsync(dsums, h->snap + KD + h->d.K, 8 * (size_t)h->d.K, hipMemcpyDeviceToHost, h->stream));
+    if (sums) PAT_HIP(hipMemcpyAsync(sums, h->d.snap, 8 * KD, hipMemcpyDeviceToHost, h->stream));
+    if (counts) PAT_HIP(hipMemcpyAsync(counts, h->d.snap + KD, 8 * (size_t)h->d.K, hipMemcpyDeviceToHost, h->stream));
+    if (dsums) PAT_HIP(hipMemcpyAsync(dsums, h->d.snap + KD + h->d.K, 8 * (size_t)h->d.K, hipMemcpyDeviceToHost, h->stream));
     PAT_HIP(hipStreamSynchronize(h->stream));
     if (shift) *shift = h->d.shift;
     if (dshift) *dshift = h->d.dshift;
