@@ -1967,9 +1967,14 @@ int kmeans_assign_mfma(const KmDev &d, hipStream_t st)
         bd.c_dot = (float)((4 * u + 2 * u * u + 4 * g * (1 + u) * (1 + u)) * 1.01);
     bd.c_norm = (float)((u * u * u + 2 * g * (1 + 2 * u)) * 1.01);
     bd.c_ref = (float)((3.0 + d.D + 16.0) * ldexp(1.0, -24) * 1.01);
-    // one workgroup per CU (the LDS holds one), BS_ / 64 wavefronts each
+    // one workgroup per CU (the LDS holds one), BS_ / 64 wavefronts each.  While
+    // the points do not fill the chip every wavefront takes one tile (rounded
+    // down, a few took two, and 10 iterations of 3,000 x 4, K 8 took 165 us, not 137).  Smaller
+    // workgroups on more CUs are slower: each stages the rows and flushes its
+    // object (10 iterations of 20,000 x 8, K 16: 158 us with 256 threads, 149
+    // with 768; of 100,000 x 16, K 32: 275 and 253).
     auto grid_for = [&](int bs) {
-        const int64_t want = (d.N + 31) / 32 / (bs / 64);
+        const int64_t want = ((d.N + 31) / 32 + bs / 64 - 1) / (bs / 64);
         return (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)d.cus));
     };
     // no tail: every K-step full and 16-byte aligned rows
