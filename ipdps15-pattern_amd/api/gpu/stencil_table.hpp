@@ -15,15 +15,15 @@
 //
 // With CONSTANT = __device__ constexpr (pattern_api.h) the table is a
 // compile-time array, so each index becomes its own kernel with the functor
-// called directly and inlined.  One thread per interior cell, 64 consecutive
-// x cells per wavefront (coalesced rows), 64 x 4 cells per workgroup, one
-// z-plane per grid row.  The library's stencil handle calls the table's
+// called directly and inlined.  A workgroup takes 256 consecutive cells of the
+// interior's rows and 1 to 4 planes.  The library's stencil handle calls the table's
 // sweep() once per step on its two halo-inclusive grids (pat_stencil_set_table).
 #ifndef PAT_GPU_STENCIL_TABLE_HPP_
 #define PAT_GPU_STENCIL_TABLE_HPP_
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 #include <utility>
@@ -48,29 +48,85 @@ __device__ __forceinline__ void call_stencil(F f, void *in, void *out, int *offs
         f(in, out, offset, size);
 }
 
-template <class Tab, int I>
-__global__ __launch_bounds__(256) void stencil_sweep(const void *in, void *out, StencilGrid g, const void *param)
+// t / d for 0 <= t < 2^31: the product with the reciprocal, rounded down, is
+// short by one at most.  (The compiler's division of two numbers known only at
+// run time took half of a sweep.)
+struct Divisor {
+    int d;
+    unsigned m;
+};
+inline Divisor divisor(int d) { return {d, 0xffffffffu / (unsigned)d}; }
+__device__ __forceinline__ int divide(int t, Divisor v)
 {
-    const int x = g.lo[0] + (int)blockIdx.x * 64 + (int)threadIdx.x;
-    const int y = g.lo[1] + (int)blockIdx.y * 4 + (int)threadIdx.y;
-    const int z = g.lo[2] + (int)blockIdx.z;
-    if (x >= g.hi[0] || y >= g.hi[1]) return;
-    int offset[3] = {x, y, z};
-    int size[3] = {g.size[0], g.size[1], g.size[2]};
-    Tab::template call<I>(const_cast<void *>(in), out, offset, size, const_cast<void *>(param));
+    const int q = (int)__umulhi((unsigned)t, v.m);
+    return t - q * v.d >= v.d ? q + 1 : q;
+}
+
+// A thread takes P planes of one column: the functor inlined P times, with the
+// grids known not to overlap, lets the compiler load a neighbour once for all
+// of them.  Bound by loads and their misses in L2: 200 x 186 x 210, W = 3 star,
+// 17.0 us a sweep against 26.5 with one cell a thread in 64 x 4 blocks dealt to
+// the XCDs in turn (every XCD then fetches every plane); 300^3 FP32 heat 37.0
+// against 87.8, 300 x 280 x 290 FP64 heat 112 against 138 (3.5 TB/s).  Without
+// the XCDs' chunks: 23.8, 65.4 and 111; in 64 x 4 blocks, whose last column of
+// blocks is nearly empty at 200 and 300: 19.5, 35.8 and 119.
+template <class Tab, int I, int P>
+__global__ __launch_bounds__(256) void stencil_sweep(const void *__restrict__ in, void *__restrict__ out,
+                                                     StencilGrid g, const void *param, Divisor blocks, Divisor nx,
+                                                     int plane)
+{
+    // workgroups are dealt to the 8 XCDs in turn: each takes a run of planes
+    const int per = (int)gridDim.x / 8, bid = (int)blockIdx.x;
+    const int t = bid < per * 8 ? bid % 8 * per + bid / 8 : bid;
+    const int tz = divide(t, blocks), i = (t - tz * blocks.d) * 256 + (int)threadIdx.x;
+    const int z = g.lo[2] + tz * P;
+    if (i >= plane) return;
+    const int row = divide(i, nx);
+    const int x = g.lo[0] + i - row * nx.d, y = g.lo[1] + row;
+    auto cell = [&](int zz) {
+        int offset[3] = {x, y, zz};
+        int size[3] = {g.size[0], g.size[1], g.size[2]};
+        Tab::template call<I>(const_cast<void *>(in), out, offset, size, const_cast<void *>(param));
+    };
+    if (z + P <= g.hi[2]) {
+#pragma unroll
+        for (int p = 0; p < P; p++) cell(z + p);
+    } else {
+        for (int zz = z; zz < g.hi[2]; zz++) cell(zz);
+    }
 }
 
 template <class Tab, int I>
-int stencil_launch(const void *in, void *out, const StencilGrid &g, const void *param, hipStream_t st)
+int stencil_launch(const void *in, void *out, const StencilGrid &grid, const void *param, hipStream_t st)
 {
     if constexpr (!Tab::template valid<I>()) {
         return PAT_ERR_UNSUPPORTED;
     } else {
-        const dim3 block(64, 4, 1);
-        const dim3 grid((unsigned)((g.hi[0] - g.lo[0] + 63) / 64), (unsigned)((g.hi[1] - g.lo[1] + 3) / 4),
-                        (unsigned)(g.hi[2] - g.lo[2]));
-        hipLaunchKernelGGL((stencil_sweep<Tab, I>), grid, block, 0, st, in, out, g, param);
-        return hipGetLastError() == hipSuccess ? PAT_OK : PAT_ERR_HIP;
+        const int nx = grid.hi[0] - grid.lo[0], ny = grid.hi[1] - grid.lo[1], nz = grid.hi[2] - grid.lo[2];
+        // More planes a thread save loads, fewer leave more wavefronts: 4
+        // planes from 8 workgroups per CU (128^3 FP32 heat 5.8 us a sweep, 6.2
+        // with 2; 64^3 star 3.4 and 3.4), 2 from 1 per CU (100^3 star 4.9, 5.6
+        // with 1; at 32^3 star 3.1, 3.0 with 1).
+        const int64_t b256 = ((int64_t)nx * ny + 255) / 256;
+        const int P = b256 * ((nz + 3) / 4) >= 2048 ? (nz >= 4 ? 4 : 1) : (b256 * ((nz + 1) / 2) >= 256 && nz >= 2 ? 2 : 1);
+        const int chunks = (nz + P - 1) / P;
+        // rows per launch: indexes within a plane and workgroups below 2^31
+        const int rows = (int)std::max<int64_t>(1, std::min<int64_t>(ny, (1LL << 30) / ((int64_t)nx * chunks)));
+        for (int y0 = 0; y0 < ny; y0 += rows) {
+            StencilGrid g = grid;
+            g.lo[1] = grid.lo[1] + y0;
+            g.hi[1] = std::min(grid.hi[1], g.lo[1] + rows);
+            const int plane = nx * (g.hi[1] - g.lo[1]), blocks = (plane + 255) / 256;
+            auto launch = [&](auto planes) {
+                hipLaunchKernelGGL((stencil_sweep<Tab, I, decltype(planes)::value>), dim3((unsigned)(blocks * chunks)),
+                                   dim3(256), 0, st, in, out, g, param, divisor(blocks), divisor(nx), plane);
+            };
+            if (P == 4) launch(std::integral_constant<int, 4>{});
+            else if (P == 2) launch(std::integral_constant<int, 2>{});
+            else launch(std::integral_constant<int, 1>{});
+            if (hipGetLastError() != hipSuccess) return PAT_ERR_HIP;
+        }
+        return PAT_OK;
     }
 }
 

@@ -92,6 +92,50 @@ def test_cross2d_on_a_2d_grid(pa, gpu, shape, steps):
     assert got.shape == ref.shape and np.array_equal(got, ref)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 300, 2), (257, 1, 9), (64, 64, 31), (63, 65, 33), (128, 129, 130),
+                                   (509, 3, 700), (255, 257, 65), (2, 2, 40000)])
+def test_sweep_planes_and_blocks(pa, orc, gpu, shape):
+    """One, two and four planes a thread, with and without a remainder, runs
+    of cells that end inside a row, numbers of workgroups that 8 does not
+    divide: the W = 3 star and the FP64 functor, bit for bit."""
+    nx, ny, nz = shape
+    for w, dtype, param, app, idx, ref in ((3, np.float32, np.zeros(0, np.float32), "stencil2", 0, orc.star),
+                                           (1, np.float64, np.zeros(5), "heat3d", 1, orc.heat_ref)):
+        g = seeded(pa, nx, ny, nz, w, dtype, nx + ny + nz)
+        st = pa.Stencil(nx, ny, nz, width=w, dtype=dtype, param=param, table=pa.app_table(app), idx=idx)
+        st.upload(g)
+        st.run(2)
+        got = st.download()
+        st.close()
+        assert np.array_equal(got, ref(g, 2, w=3) if app == "stencil2" else ref(g, 2))
+
+
+def test_sweep_of_a_plane_beyond_2_30_cells(pa, gpu):
+    """A plane that takes more than one launch: the rows on both sides of the
+    cut, the first and the last, against the same operations in NumPy."""
+    nx, ny = 40000, 27000
+    cut = (1 << 30) // nx
+    assert cut < ny
+    st = pa.Stencil(nx, ny, None, width=1, param=np.zeros(0, np.float32), table=pa.app_table("stencil2"), idx=1)
+    rng = np.random.default_rng(4)
+    grid = np.zeros((ny + 2, nx + 2), np.float32)
+    picks = (0, cut - 1, cut, ny - 1)
+    for r in sorted({q for r in picks for q in (r, r + 1, r + 2)} - {0, ny + 1}):
+        grid[r, 1:-1] = rng.standard_normal(nx).astype(np.float32)
+    st.upload(grid)
+    st.run(1)
+    ptr = pa.c_vp()
+    pa.call("pat_stencil_device_ptr", st.h, pa.ctypes.byref(ptr))
+    for r in picks:
+        b = grid[r:r + 3]
+        got = np.empty(nx + 2, np.float32)
+        pa.call("pat_memcpy_d2h", pa.ptr(got), pa.c_vp(ptr.value + 4 * (r + 1) * (nx + 2)), got.nbytes, None)
+        pa.sync()
+        want = ((b[1, 2:] + b[1, :-2]) + (b[2, 1:-1] + b[0, 1:-1])) * np.float32(0.25)
+        assert np.array_equal(got[1:-1], want), r
+    st.close()
+
+
 def test_table_errors(pa, gpu):
     # an index outside the table, a functor of another element type, and a
     # width the tuned engine cannot run without a table are refused
