@@ -21,11 +21,11 @@
 // Compiled with -ffp-contract=off so no multiply-add is fused.
 //
 // Assignment, MFMA path: a wavefront takes 32 points and computes
-// ||c||^2 - 2 x.c for every centre with v_mfma_f32_32x32x16_bf16 (FP32
-// accumulation, ||c||^2 split into three BF16 terms on an extra K step).
-// With NT = 3 terms, x and -2c are each split into BF16 high and low parts
-// and the product is xh.ch + xh.cl + xl.ch (the dropped terms are O(2^-16)
-// relative); with NT = 1 both are rounded to BF16 once (O(2^-8)).  A
+// ||c||^2 - 2 x.c (up to a scale) for every centre with 32x32x16 MFMAs (FP32
+// accumulation, the norm split into three terms on an extra K step).
+// With NT = 3 terms, x and c are each split into FP16 high and low parts and
+// the product is xl.ch + xh.cl + xh.ch (the dropped terms are O(2^-22)
+// relative); with NT = 1 x and -2c are rounded to BF16 once (O(2^-8)).  A
 // per-point bound E on the error of that value (operand rounding, the norm
 // split, FP32 accumulation) plus the FP32 rounding of the reference's own
 // difference form gives a margin:
@@ -34,7 +34,7 @@
 // results decide (same tie rule).  A centre outside the margin provably has a
 // larger reference distance than the best one, so the assignment equals the
 // plain path's bit for bit.  Shapes whose object is beyond LDS take the same
-// steps with FP16 parts (km_wide).
+// steps against rows in global memory (km_wide).
 #include <algorithm>
 #include <cmath>
 
@@ -305,8 +305,14 @@ __global__ __launch_bounds__(BS) void km_plain(KmArgs a, int centres_in_lds)
 
 // ------------------------------------------------------------ MFMA path
 
-// Per-point bound inputs: u = 2^-8 (BF16 unit roundoff), g = FP32
-// accumulation over the MFMA's terms with a factor 2 of slack for any
+typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
+typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2;
+
+constexpr float kWideOne = 32768.0f;  // the norm parts' factor 2^15
+constexpr float kWideFar = 60000.0f;  // first norm part of a row that never wins: above any value (2^28)
+
+// Per-point bound inputs of the one-term form: u = 2^-8 (BF16 unit roundoff),
+// g = FP32 accumulation over the MFMA's terms with a factor 2 of slack for any
 // intermediate rounding mode.
 struct MfmaBound {
     float c_dot;   // multiplies ||x|| * max||c||
@@ -314,30 +320,53 @@ struct MfmaBound {
     float c_ref;   // relative error of the reference's FP32 difference form
 };
 
+// Those of the FP16 parts (km_wide has the proof).
+struct WideBound {
+    float sx;                        // 2^a
+    float c_dot, c_sum, c_cc, c_abs;  // error: c_dot X C + c_sum (X + C) + c_cc C^2 + c_abs
+    float c_ref, ref_abs;            // the reference's FP32 difference form: relative, and for underflow
+    float far;                       // half squared distances from here on may reach map1's initial minimum
+};
+
+// Four floats at any float's address (a 16-byte global load needs no more).
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// x[d .. d+3] of a row of D, zeros past its end.
+__device__ __forceinline__ float4u ragged_4(const float *__restrict__ x, int d, int D)
+{
+    float4u q = {0.f, 0.f, 0.f, 0.f};
+    if (d + 4 <= D) {
+        q = *(const float4u *)(x + d);
+    } else {
+        if (d < D) q.x = x[d];
+        if (d + 1 < D) q.y = x[d + 1];
+        if (d + 2 < D) q.z = x[d + 2];
+    }
+    return q;
+}
+
 // Exact plain-path distance (sqrt of the FP32 difference form, dimensions in
 // order) of point row xp to centre row ck, both read from memory (the point
 // row was just loaded by the wavefront, so it is in cache).
-__device__ __forceinline__ float exact_dist(const float *__restrict__ xp, const float *__restrict__ ck, int D, bool vec)
+__device__ __forceinline__ float exact_dist(const float *__restrict__ xp, const float *__restrict__ ck, int D)
 {
     float dist = 0;
-    if (vec) {  // D % 4 == 0 and 16-byte aligned rows
+    int d = 0;
 #pragma unroll 4
-        for (int d = 0; d < D; d += 4) {
-            const float4 cv = *(const float4 *)(ck + d), xv = *(const float4 *)(xp + d);
-            float t = cv.x - xv.x;
-            dist = dist + t * t;
-            t = cv.y - xv.y;
-            dist = dist + t * t;
-            t = cv.z - xv.z;
-            dist = dist + t * t;
-            t = cv.w - xv.w;
-            dist = dist + t * t;
-        }
-    } else {
-        for (int d = 0; d < D; d++) {
-            const float t = ck[d] - xp[d];
-            dist = dist + t * t;
-        }
+    for (; d + 4 <= D; d += 4) {
+        const float4u cv = *(const float4u *)(ck + d), xv = *(const float4u *)(xp + d);
+        float t = cv.x - xv.x;
+        dist = dist + t * t;
+        t = cv.y - xv.y;
+        dist = dist + t * t;
+        t = cv.z - xv.z;
+        dist = dist + t * t;
+        t = cv.w - xv.w;
+        dist = dist + t * t;
+    }
+    for (; d < D; d++) {
+        const float t = ck[d] - xp[d];
+        dist = dist + t * t;
     }
     return sqrtf(dist);
 }
@@ -416,23 +445,31 @@ constexpr float kFar = 3.0e38f;
 
 // KS: K-steps of 16 dimensions holding the data (D <= 16*KS); NT: terms
 // (1 or 3), each KS steps; one more K-step holds the norm terms.  KB:
-// 32-centre blocks per chunk.  cb: K_pad x (16*(NT*KS+1)) BF16 centre rows
-// [-2c | n1 n2 n3 0...] (NT = 1) or [hi(-2c) | lo(-2c) | hi(-2c) | n1 n2 n3
-// 0...] (NT = 3), data zero-padded to 16*KS, stored in fragment order
-// (frag_index); padded rows have n1 = 1e30 (far, but finite so that their
-// keys are numbers).  cnorm: ||c_k|| (K entries).
+// 32-centre blocks per chunk.  cb: NT = 1: K_pad x 16 (KS + 1) BF16 rows
+// [-2c | n1 n2 n3 0...]; padded rows have n1 = 1e30 (far, but finite so that
+// their keys are numbers).  NT = 3: K_pad x 16 (2 KS + 1) FP16 rows (km_wide
+// has their form, the value they give and its bound).  Data zero-padded to
+// 16*KS, fragment order (frag_index).  cnorm: ||c_k|| (K entries).
 //
 // Per 32-point tile a wavefront (lanes l and l+32 hold halves of point l):
-// computes the approximate values of every centre with MFMAs, packs each
-// with its index (pack_key) and keeps the three smallest keys of each half
-// (the two smallest per chunk when the index bits cannot tell the chunks
-// apart).  The threshold is the minimum plus the error bound plus the
-// packing error; when only the smallest key is under it (the usual case)
-// that one centre is rescored, when a half's third key lies above it its
-// kept keys under it are, and otherwise every centre under it is (the
-// values recomputed chunk by chunk).  The exact FP32 results
-// decide with map1's rule, and the point is added to the LDS reduction object
-// from the registers holding its half rows.
+// computes the approximate values of every centre with MFMAs, packs the
+// smaller of every two with their index (pack_key) and keeps the three
+// smallest keys of each half (the two smallest values per chunk when the index
+// bits cannot tell the chunks apart).  The threshold is the minimum plus the
+// error bound plus the packing error; when only the smallest key is under it
+// (the usual case) its two centres are rescored, one by each half, when a
+// half's third key lies above it the kept keys under it are, and otherwise
+// every centre under it is (the values recomputed chunk by chunk).  The exact
+// FP32 results decide with map1's rule, and the point is added to the LDS
+// reduction object from the registers holding its half rows.
+//
+// Bound by instruction issue, vector and matrix together: 2^24 x 32, K 256,
+// 1.16 ms a pass (1.31 with BF16 parts and a key for every value; the wider
+// bound of those left 2.3% of the points several candidates, of every second
+// tile one).  One block of centres per chunk at every KS: its two accumulators
+// and the registers around them fit without spills (1 M x 8, K 16: 41 us with
+// one, 54 with four; 1 M x 16, K 128: 55 and 64), and the matrix cores work on
+// the next block during a scan.
 // TAIL = false: D == 16*KS and the rows are 16-byte aligned, so every
 // K-step is full and the loads need no per-element guard.
 // GC: the form for K x D too large for LDS.  The workgroup's wavefronts
@@ -447,27 +484,27 @@ constexpr float kFar = 3.0e38f;
 // object are shared by all its wavefronts, so larger workgroups raise the
 // occupancy the LDS allows when the registers permit).
 template <int KS, int KB, int NT, bool TAIL, bool GC, int BS = 512>
-__global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict__ cb, const float *__restrict__ cnorm,
-                                               int K_pad, MfmaBound bd, unsigned long long *__restrict__ rescored)
+__global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const void *__restrict__ cb, const float *__restrict__ cnorm,
+                                               int K_pad, MfmaBound bd, WideBound wb,
+                                               unsigned long long *__restrict__ rescored)
 {
-    constexpr int NS = NT * KS + 1;  // K-steps per centre row
-    constexpr int KW = 16 * NS;      // BF16 row width of cb
+    constexpr bool F16 = NT == 3;
+    constexpr int NS = NT * KS + 1;               // MFMAs per block of 32 centres
+    constexpr int NF = F16 ? 2 * KS + 1 : NS;     // fragments per block in cb (1 KiB each)
     static_assert(KB * 16 <= 128, "pack_key indexes at most 128 values per chunk");
     extern __shared__ unsigned long long smem[];
     unsigned long long *acc_o, *cnt_o, *dsum_o;
     lds_object(a, smem, acc_o, cnt_o, dsum_o);
-    __bf16 *cbs = (__bf16 *)(smem + (a.use_lds_acc ? object_words(a.K, a.D) : 0));
+    u32x4 *cbs = (u32x4 *)(smem + (a.use_lds_acc ? object_words(a.K, a.D) : 0));
     __shared__ float red[16];
     if (a.use_lds_acc) zero_lds_object(a, acc_o, cnt_o, dsum_o);
-    // stage the BF16 centre matrix in LDS (16-byte copies); the GC form
-    // stages one chunk at a time (stage_chunk)
+    // stage the centre rows in LDS (16-byte copies); the GC form stages one
+    // chunk at a time (stage_chunk)
     if (!GC) {
-        const int n16 = K_pad * KW / 8;
-        const bf16x8 *src = (const bf16x8 *)cb;
-        bf16x8 *dst = (bf16x8 *)cbs;
-        for (int i = threadIdx.x; i < n16; i += blockDim.x) dst[i] = src[i];
+        const int n16 = K_pad * NF * 2;
+        const u32x4 *src = (const u32x4 *)cb;
+        for (int i = threadIdx.x; i < n16; i += blockDim.x) cbs[i] = src[i];
     }
-    const __bf16 *__restrict__ cfr = cbs;
     // max ||c|| over the centres (for the bound)
     float cm = 0.0f;
     for (int i = threadIdx.x; i < a.K; i += blockDim.x) cm = fmaxf(cm, cnorm[i]);
@@ -477,11 +514,9 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
     __syncthreads();
     float cmax = 0.0f;
     for (int w = 0; w < (int)(blockDim.x / kWave); w++) cmax = fmaxf(cmax, red[w]);
-    const float cc_max = cmax * cmax;
+    const float cc_max = cmax * cmax, C = cmax * wb.sx;
 
     const int D = a.D;
-    const bool vec_x = (D % 4) == 0 && ((uintptr_t)a.x % 16) == 0;  // rows start 16-byte aligned
-    const bool vec_c = (D % 4) == 0 && ((uintptr_t)a.c % 16) == 0;
     const int lane = threadIdx.x % kWave;
     const int col = lane % 32;   // point within the tile
     const int half = lane / 32;  // which 8 of each 16 K elements this lane holds
@@ -497,24 +532,36 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
     // on the scalar unit -- and skipped by the scans.
     const int kblocks = K_pad / 32;
     const int keep = key_mask();
-    auto chunk_values = [&](int ch, const bf16x8 (&bx)[NS], f32x16 (&acc)[KB]) {
+    auto chunk_values = [&](int ch, const u32x4 (&bx)[NF], f32x16 (&acc)[KB]) {
         constexpr int T = KB * NS, P = 3;
-        const bf16x8 *ab = (const bf16x8 *)cfr + lane;
+        const u32x4 *ab = cbs + lane;
+        int again = 0;  // where the high parts, read twice, would not fit in registers
+        if (F16 && KS > 2) asm volatile("" : "+s"(again));
         auto frag = [&](int t) {
-            if (GC) return ab[t * kWave];  // the staged chunk: block t / NS, K-step t % NS
+            // F16: high, low, high parts, norm
+            const int st = t % NS, f = !F16 || st < 2 * KS ? st : (st < 3 * KS ? st - 2 * KS : 2 * KS);
+            const int at = (F16 && st >= 2 * KS ? again : 0) + f * kWave;
+            if (GC) return ab[t / NS * NF * kWave + at];  // the staged chunk
             const int blk = ch * KB + t / NS;
-            return ab[((int64_t)(blk < kblocks ? blk : 0) * NS + t % NS) * kWave];
+            return ab[(blk < kblocks ? blk : 0) * NF * kWave + at];
         };
-        bf16x8 fr[P];
+        u32x4 fr[P];
 #pragma unroll
         for (int t = 0; t < P; t++) fr[t] = frag(t);
 #pragma unroll
         for (int t = 0; t < T; t++) {
             const int b = t / NS, st = t % NS;
-            const bf16x8 av = fr[t % P];
+            const u32x4 av = fr[t % P];
             if (t + P < T) fr[t % P] = frag(t + P);
             if (st == 0) acc[b] = f32x16{};
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bx[st], acc[b], 0, 0, 0);
+            // F16: high.low(x), low.high(x), high.high, norm: the small terms first
+            const u32x4 bv = bx[!F16 ? st : (st < KS ? KS + st : (st < 3 * KS ? (st - KS) % KS : 2 * KS))];
+            if constexpr (F16)
+                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, av),
+                                                                __builtin_bit_cast(f16x8, bv), acc[b], 0, 0, 0);
+            else
+                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av),
+                                                                 __builtin_bit_cast(bf16x8, bv), acc[b], 0, 0, 0);
         }
     };
     auto centre_of = [&](int ch, int idx) {
@@ -527,10 +574,9 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
     auto stage_chunk = [&](int ch) {
         __syncthreads();  // every wavefront is done with the previous chunk
         const int nblk = min(KB, kblocks - ch * KB);
-        const int n16 = nblk * NS * kWave;
-        const bf16x8 *src = (const bf16x8 *)cb + (int64_t)ch * KB * NS * kWave;
-        bf16x8 *dst = (bf16x8 *)cbs;
-        for (int i = threadIdx.x; i < n16; i += blockDim.x) dst[i] = src[i];
+        const int n16 = nblk * NF * kWave;
+        const u32x4 *src = (const u32x4 *)cb + (int64_t)ch * KB * NF * kWave;
+        for (int i = threadIdx.x; i < n16; i += blockDim.x) cbs[i] = src[i];
         __syncthreads();
     };
 
@@ -549,15 +595,12 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
                 const float4 lo = *(const float4 *)(xp + d0), hi = *(const float4 *)(xp + d0 + 4);
                 xo[8 * s] = lo.x; xo[8 * s + 1] = lo.y; xo[8 * s + 2] = lo.z; xo[8 * s + 3] = lo.w;
                 xo[8 * s + 4] = hi.x; xo[8 * s + 5] = hi.y; xo[8 * s + 6] = hi.z; xo[8 * s + 7] = hi.w;
-            } else if (vec_x) {
-                float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
-                if (live && d0 < D) lo = *(const float4 *)(xp + d0);
-                if (live && d0 + 4 < D) hi = *(const float4 *)(xp + d0 + 4);
-                xo[8 * s] = lo.x; xo[8 * s + 1] = lo.y; xo[8 * s + 2] = lo.z; xo[8 * s + 3] = lo.w;
-                xo[8 * s + 4] = hi.x; xo[8 * s + 5] = hi.y; xo[8 * s + 6] = hi.z; xo[8 * s + 7] = hi.w;
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; e++) xo[8 * s + e] = (live && d0 + e < D) ? xp[d0 + e] : 0.0f;
+                for (int e = 0; e < 8; e += 4) {
+                    const float4u q = ragged_4(xp, d0 + e, D);
+                    xo[8 * s + e] = q.x; xo[8 * s + e + 1] = q.y; xo[8 * s + e + 2] = q.z; xo[8 * s + e + 3] = q.w;
+                }
             }
         }
     };
@@ -588,51 +631,51 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
             for (int i = 0; i < 8 * KS; i++) xo[i] = xnext[i];
             if (tile + nw < ntiles) load_half_row(tile + nw, xnext);
         }
-        // B operand: point p, K elements [16s + 8*half, +8) of
-        // [x, 1, 1, 1, 0...] or [xh, xh, xl, 1, 1, 1, 0...]
-        bf16x8 bx[NS];
+        // B operand: point p, K elements [16s + 8*half, +8): x and ones for the
+        // norm's three parts, or high and low parts of 2^a x and its ones;
+        // pairs of elements, one packed conversion each
+        u32x4 bx[NF];
         float xx = 0.0f;
-        // pairs of elements, one packed conversion each, straight into the
-        // operand's 32-bit words (xh = bf16(x), xl = bf16(x - xh))
 #pragma unroll
         for (int s = 0; s < KS; s++) {
-            u32x4 wh, wl;
 #pragma unroll
             for (int e = 0; e < 8; e += 2) {
-                const float v0 = xo[8 * s + e], v1 = xo[8 * s + e + 1];
-                xx = __builtin_fmaf(v0, v0, xx);  // a bound input only (used with slack)
-                xx = __builtin_fmaf(v1, v1, xx);
-                const unsigned h = bf16_pair(v0, v1);
-                wh[e / 2] = h;
-                if (NT == 3)
-                    wl[e / 2] = bf16_pair(v0 - __uint_as_float(h << 16), v1 - __uint_as_float(h & 0xffff0000u));
-            }
-            bx[s] = __builtin_bit_cast(bf16x8, wh);
-            if (NT == 3) {
-                bx[KS + s] = bx[s];
-                bx[2 * KS + s] = __builtin_bit_cast(bf16x8, wl);
+                const f32x2 q = F16 ? (f32x2){xo[8 * s + e] * wb.sx, xo[8 * s + e + 1] * wb.sx}
+                                    : (f32x2){xo[8 * s + e], xo[8 * s + e + 1]};
+                xx = __builtin_fmaf(q[0], q[0], xx);  // a bound input only (used with slack)
+                xx = __builtin_fmaf(q[1], q[1], xx);
+                if constexpr (F16) {
+                    const f16x2 h = __builtin_convertvector(q, f16x2);
+                    const f32x2 r = {q[0] - (float)h[0], q[1] - (float)h[1]};
+                    bx[s][e / 2] = __builtin_bit_cast(unsigned, h);
+                    bx[KS + s][e / 2] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, f16x2));
+                } else {
+                    bx[s][e / 2] = bf16_pair(q[0], q[1]);
+                }
             }
         }
-#pragma unroll
-        for (int e = 0; e < 8; e++) bx[NT * KS][e] = (__bf16)((half == 0 && e < 3) ? 1.0f : 0.0f);
+        // 2^15 or 1 three times
+        bx[NF - 1] = half == 0 ? (F16 ? (u32x4){0x78007800u, 0x7800u, 0u, 0u} : (u32x4){0x3f803f80u, 0x3f80u, 0u, 0u})
+                               : (u32x4){0u, 0u, 0u, 0u};
         xx = xx + __shfl_xor(xx, 32, kWave);  // ||x||^2 of point p (both halves)
         // an upper bound of ||x|| only: the hardware square root (within an
         // ulp or two for normal inputs, 0 for flushed subnormals, whose
         // root lies below 2^-63) with relative and absolute slack, in place
         // of the correctly rounded sequence
         const float xn = __builtin_amdgcn_sqrtf(xx) * 1.0001f + 0x1p-40f;
-        const float E = bd.c_dot * xn * cmax + bd.c_norm * (cc_max + xx);
-        // packing error bound: |values| <= ||c||^2 + 2 ||x|| ||c||
-        const float dp = 0x1p-16f * (cc_max + 2.0f * xn * cmax) * 1.01f + 0x1p-126f;
+        const float E = F16 ? wb.c_dot * xn * C + wb.c_sum * (xn + C) + wb.c_cc * C * C + wb.c_abs
+                            : bd.c_dot * xn * cmax + bd.c_norm * (cc_max + xx);
 
         f32x16 acc[KB];
-        // The three smallest keys of this half.  When the lane's values of all
-        // chunks fit the 7 index bits (gidx: at most 128 per lane), every key
-        // carries the lane's global value index (value i of block blk ->
-        // 16 blk + i) and one sorted triple runs over all chunks; otherwise
-        // each chunk's two smallest are merged with their chunk recorded and
-        // k3 stays unknown (kFar, never used).
-        const bool gidx = nchunks * KB <= 8;  // uniform
+        // The three smallest keys of this half.  When the pairs of a lane's
+        // values in all chunks fit the 7 index bits (gidx: at most 128), a key
+        // is the smaller of two adjacent centres' values with the pair's index
+        // (values i and i + 1 of block blk -> 8 blk + i / 2): five instructions
+        // for two values, and the halves rescore one centre of a pair each.
+        // One sorted triple runs over all chunks.  Otherwise the keys are
+        // single values, each chunk's two smallest are merged with their
+        // chunk recorded and k3 stays unknown (kFar, never used).
+        const bool gidx = nchunks * KB <= 16;  // uniform
         float k1 = kFar, k2 = kFar, k3 = kFar;
         int ch1 = 0;
         auto scan3 = [&](int ch, const f32x16 (&v)[KB]) {
@@ -640,11 +683,12 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
             for (int b = 0; b < KB; b++) {
                 if (b > 0 && ch * KB + b >= kblocks) break;  // uniform; block 0 of a chunk always exists
 #pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const float key = pack_key(v[b][i], scalar_or((ch * KB + b) * 16, i), keep);
+                for (int i = 0; i < 16; i += 2) {
+                    const float lo = __builtin_amdgcn_fmed3f(v[b][i], v[b][i + 1], -kFar);  // min (finite)
+                    const float key = pack_key(lo, scalar_or((ch * KB + b) * 8, i / 2), keep);
                     k3 = __builtin_amdgcn_fmed3f(k2, k3, key);
                     k2 = __builtin_amdgcn_fmed3f(k1, k2, key);
-                    k1 = __builtin_amdgcn_fmed3f(k1, key, -kFar);  // min (keys are finite)
+                    k1 = __builtin_amdgcn_fmed3f(k1, key, -kFar);
                 }
             }
         };
@@ -698,43 +742,67 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
             }
         }
         // both halves: overall smallest and second smallest
-        const float o1 = __shfl_xor(k1, 32, kWave), o2 = __shfl_xor(k2, 32, kWave);
+        const float o1 = __shfl_xor(k1, 32, kWave), o2 = __shfl_xor(k2, 32, kWave), o3 = __shfl_xor(k3, 32, kWave);
         const float m1 = fminf(k1, o1);
         const float m2 = fminf(fmaxf(k1, o1), fminf(k2, o2));
-        // candidates: keys within the margin of the minimum
-        const float dhi = (xx + m1 + 4.0f * E + 4.0f * dp) * 1.001f + 1e-30f;
-        const float thr = m1 + 2.0f * E + 2.0f * dp + 2.0f * bd.c_ref * dhi;
+        // candidates: keys within the margin of the minimum.  The packing
+        // moves a value by 2^-16 of itself: at most ||c||^2 + 2 ||x|| ||c||,
+        // or (F16) at most the larger of ||x||^2 / 2 and the smallest key, for
+        // every centre that matters
+        float dp, dhi;
+        if (F16) {
+            const float H = 0.5f * xx;
+            dp = 0x1p-16f * 1.02f * (fmaxf(H, fabsf(m1)) * 1.01f + 4.0f * E) + 0x1p-126f;
+            dhi = (H + m1 + 4.0f * E + 4.0f * dp) * 1.001f + wb.ref_abs;
+        } else {
+            dp = 0x1p-16f * (cc_max + 2.0f * xn * cmax) * 1.01f + 0x1p-126f;
+            dhi = (xx + m1 + 4.0f * E + 4.0f * dp) * 1.001f + 1e-30f;
+        }
+        const float thr = m1 + 2.0f * E + 2.0f * dp + 2.0f * (F16 ? wb.c_ref : bd.c_ref) * dhi;
         const bool multi = !(m2 > thr);
-        // lanes whose candidates may lie beyond the keys they kept: every
+        // points whose candidates may lie beyond the keys they kept: every
         // value under the threshold is then visited again (full)
-        const bool full = multi && (!gidx || !(k3 > thr));
+        const bool full = multi && (!gidx || !(fminf(k3, o3) > thr));
         // the whole point row in registers (full K-steps) where the form has
         // the registers to spare (the others would spill: they reload it)
-        constexpr bool ROW = !TAIL && !GC && KS == 2 && KB == 1;
+        constexpr bool ROW = !TAIL && !GC && KB == 1 && (KS <= 2 || (KS == 4 && BS <= 512));
         float row[16 * KS];
         if (ROW) point_row<KS>(xo, row);
 
         float best_d = kInitMin;
         int best_k = 0x7fffffff;
-        // exact distance to value idx of chunk ch (the pack_key index)
-        auto rescore = [&](int ch, int idx) {
-            const int k = centre_of(ch, idx);
+        // exact distance to centre k
+        auto rescore = [&](int k) {
             if (k < a.K) {
                 const float *ck = a.c + (int64_t)k * D;
-                const float dk = ROW && vec_c ? exact_dist_row<KS>(row, ck) : exact_dist(xp, ck, D, vec_c && vec_x);
+                const float dk = ROW ? exact_dist_row<KS>(row, ck) : exact_dist(xp, ck, D);
                 if (dk < best_d || (dk == best_d && k < best_k)) {
                     best_d = dk;
                     best_k = k;
                 }
             }
         };
-        if (live && !full) {
-            // one candidate: rescored by the half that holds it; several
-            // (gidx only): each half rescores its kept keys under the
-            // threshold, which are all of its candidates since its third
-            // smallest lies above it
-            if (multi ? !(k1 > thr) : k1 < o1) rescore(gidx ? 0 : ch1, __float_as_int(k1) & 127);
-            if (multi && !(k2 > thr)) rescore(0, __float_as_int(k2) & 127);
+        // this half's centre of the pair that key stands for, held by half h
+        auto pair_centre = [&](float key, int h) {
+            const int id = __float_as_int(key) & 127, i = 2 * (id & 7);
+            return (id >> 3) * 32 + 8 * (i >> 2) + 4 * h + (i & 3) + half;
+        };
+        if (gidx) {
+            // the kept pairs under the threshold are all of its candidates
+            // (the third smallest of each half lies above it): the smallest,
+            // and of several the other three as far as they are under it
+            const bool first = half ? k1 < o1 : k1 <= o1;  // the halves agree on ties
+            const bool second = half ? k2 < o2 : k2 <= o2;
+            if (live && !full) rescore(pair_centre(m1, first ? half : 1 - half));
+            const bool more = live && multi && !full;
+            if (__any(more)) {
+                const float t = fmaxf(k1, o1), u = fminf(k2, o2), w = fmaxf(k2, o2);
+                if (more && !(t > thr)) rescore(pair_centre(t, first ? 1 - half : half));
+                if (more && !(u > thr)) rescore(pair_centre(u, second ? half : 1 - half));
+                if (more && !(w > thr)) rescore(pair_centre(w, second ? 1 - half : half));
+            }
+        } else if (live && !multi && k1 < o1) {
+            rescore(centre_of(ch1, __float_as_int(k1) & 127));
         }
         // Every value under the threshold for the full lanes.  Taken by the
         // whole wavefront (a vote), because recomputing a chunk's values
@@ -764,7 +832,7 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
                     while (mw) {
                         const int bit = __builtin_ctzll(mw);
                         mw &= mw - 1;
-                        if (live) rescore(ch, 64 * w + bit);
+                        if (live) rescore(centre_of(ch, 64 * w + bit));
                     }
                 }
             }
@@ -866,19 +934,6 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const __bf16 *__restrict
 // scan takes 4 vector instructions a value.  1 M x 128, K 1,000: 0.84 ms a pass,
 // 0.7% of the points rescored (2.66 ms with BF16 terms and a second pass over
 // the centres in nearly every workgroup).
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
-typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2;
-
-constexpr float kWideOne = 32768.0f;  // the norm parts' factor 2^15
-constexpr float kWideFar = 60000.0f;  // first norm part of a row that never wins: above any value (2^28)
-
-struct WideBound {
-    float sx;                        // 2^a
-    float c_dot, c_sum, c_cc, c_abs;  // error: c_dot X C + c_sum (X + C) + c_cc C^2 + c_abs
-    float c_ref, ref_abs;            // the reference's FP32 difference form: relative, and for underflow
-    float far;                       // half squared distances from here on may reach map1's initial minimum
-};
-
 template <int KS, int NB, int TILES, bool TAIL>
 __global__ __launch_bounds__(512) void km_wide(KmArgs a, const _Float16 *__restrict__ cb,
                                                const float *__restrict__ cnorm, int K_pad, WideBound bd,
@@ -902,7 +957,6 @@ __global__ __launch_bounds__(512) void km_wide(KmArgs a, const _Float16 *__restr
     const float C = cmax * bd.sx;
 
     const int D = a.D, kblocks = K_pad / 32, nchunks = (kblocks + NB - 1) / NB;
-    const bool vec_x = (D % 4) == 0 && ((uintptr_t)a.x % 16) == 0, vec_c = (D % 4) == 0;
     const int keep = key_mask();
     unsigned my_rescored = 0;
 
@@ -940,15 +994,16 @@ __global__ __launch_bounds__(512) void km_wide(KmArgs a, const _Float16 *__restr
             for (int s = 0; s < KS; s++) {
                 const int d0 = 16 * s + 8 * half;
                 float v[8];
-                if (!TAIL || vec_x) {
-                    float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
-                    if (!TAIL || d0 < D) lo = *(const float4 *)(xp + d0);
-                    if (!TAIL || d0 + 4 < D) hi = *(const float4 *)(xp + d0 + 4);
+                if (!TAIL) {
+                    const float4 lo = *(const float4 *)(xp + d0), hi = *(const float4 *)(xp + d0 + 4);
                     v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
                     v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
                 } else {
 #pragma unroll
-                    for (int e = 0; e < 8; e++) v[e] = d0 + e < D ? xp[d0 + e] : 0.0f;
+                    for (int e = 0; e < 8; e += 4) {
+                        const float4u q = ragged_4(xp, d0 + e, D);
+                        v[e] = q.x; v[e + 1] = q.y; v[e + 2] = q.z; v[e + 3] = q.w;
+                    }
                 }
                 u32x4 wh, wl;
 #pragma unroll
@@ -1095,7 +1150,7 @@ __global__ __launch_bounds__(512) void km_wide(KmArgs a, const _Float16 *__restr
         int best_k = 0x7fffffff;
         auto rescore = [&](const float *x, int c, float &bd_, int &bk) {
             if (c < a.K) {
-                const float dk = exact_dist(x, a.c + (int64_t)c * D, D, vec_c && vec_x);
+                const float dk = exact_dist(x, a.c + (int64_t)c * D, D);
                 if (dk < bd_ || (dk == bd_ && c < bk)) {
                     bd_ = dk;
                     bk = c;
@@ -1185,14 +1240,13 @@ __global__ __launch_bounds__(256) void km_rescore(KmArgs a, const int *__restric
                                                   const int *__restrict__ listed)
 {
     const int n = *listed, q = threadIdx.x % 4;
-    const bool vec = (a.D % 4) == 0 && ((uintptr_t)a.x % 16) == 0;
     for (int i = blockIdx.x * 64 + threadIdx.x / 4; i < n; i += gridDim.x * 64) {
         const int p = list[i];
         const unsigned w = q < 2 ? (unsigned)a.assign[p] : __float_as_uint(a.mindist[p]);
         int k = (int)(q & 1 ? w >> 16 : w & 0xffffu);
         float d = kInitMin;
         if (k < a.K) {
-            const float v = exact_dist(a.x + (int64_t)p * a.D, a.c + (int64_t)k * a.D, a.D, vec);
+            const float v = exact_dist(a.x + (int64_t)p * a.D, a.c + (int64_t)k * a.D, a.D);
             if (v < d) d = v;
             else k = 0x7fffffff;
         } else {
@@ -1243,7 +1297,7 @@ __device__ __forceinline__ void retire_object(int k, int lane, int K, int D, uns
 // object (c = (sum * 2^-s) / count in FP64, rounded to FP32; empty clusters
 // keep their centre), writes the BF16 MFMA row and the norm, and clears the
 // object for the next pass.  With update == 0 only the rows are prepared.
-template <int KS, int NT>
+template <int KS>
 __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K, int K_pad, int D,
                                                    unsigned long long *__restrict__ gsum,
                                                    unsigned long long *__restrict__ gcnt,
@@ -1251,8 +1305,8 @@ __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K,
                                                    int update, __bf16 *__restrict__ cb, float *__restrict__ cnorm,
                                                    unsigned long long *__restrict__ snap)
 {
-    constexpr int KW = 16 * (NT * KS + 1);
-    constexpr int NB = 16 * NT * KS;  // first norm column
+    constexpr int KW = 16 * (KS + 1);
+    constexpr int NB = 16 * KS;  // first norm column
     const int k = blockIdx.x * 4 + threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
     if (k >= K_pad) return;
@@ -1273,12 +1327,7 @@ __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K,
     for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
     for (int d = lane; d < 16 * KS; d += kWave) {
         const float v = d < D ? -2.0f * c[(int64_t)k * D + d] : 0.0f;  // exact
-        const __bf16 h = (__bf16)v;
-        cb[frag_index(k, d, KW / 16)] = h;
-        if (NT == 3) {
-            cb[frag_index(k, 16 * KS + d, KW / 16)] = (__bf16)(v - (float)h);
-            cb[frag_index(k, 32 * KS + d, KW / 16)] = h;
-        }
+        cb[frag_index(k, d, KW / 16)] = (__bf16)v;
     }
     if (lane < 16) {
         const __bf16 n1 = (__bf16)(float)ss;
@@ -1296,7 +1345,7 @@ __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K,
     retire_object(k, lane, K, D, gsum, gcnt, gdsum, update, snap);
 }
 
-// The same update with the FP16 rows of the wide path: 2 KS + 1 fragments of 16
+// The same update with FP16 rows: 2 KS + 1 fragments of 16
 // elements per centre: high parts of c^ = -2^a c, low parts, and n^ / 2^15 in
 // three parts.  A centre with a coordinate that is not finite is never map1's
 // nearest: its row is far, as the padding rows are.
@@ -1786,7 +1835,7 @@ int kmeans_finalize(const KmDev &d, int update, hipStream_t st)
 {
     const double inv = ldexp(1.0, -d.shift);
     const dim3 g((unsigned)((d.K_pad + 3) / 4)), b(256);
-    if (d.wide) {
+    if (d.wide || d.NT == 3) {
         auto f = d.KS == 1 ? km_finalize_wide<1>
                            : (d.KS == 2 ? km_finalize_wide<2> : (d.KS == 4 ? km_finalize_wide<4> : km_finalize_wide<8>));
         hipLaunchKernelGGL(f, g, b, 0, st, d.c, d.K, d.K_pad, d.D, d.gsum, d.gcnt, d.gdsum, inv, update,
@@ -1794,19 +1843,14 @@ int kmeans_finalize(const KmDev &d, int update, hipStream_t st)
         PAT_LAUNCH_CHECK();
         return PAT_OK;
     }
-#define PAT_KF(KS_, NT_)                                                                                               \
-    hipLaunchKernelGGL((km_finalize<KS_, NT_>), g, b, 0, st, d.c, d.K, d.K_pad, d.D, d.gsum, d.gcnt, d.gdsum, inv,    \
-                       update, (__bf16 *)d.cb, d.cnorm, d.snap)
-    const int code = d.KS * 4 + d.NT;
-    switch (code) {
-    case 1 * 4 + 1: PAT_KF(1, 1); break;
-    case 2 * 4 + 1: PAT_KF(2, 1); break;
-    case 4 * 4 + 1: PAT_KF(4, 1); break;
-    case 8 * 4 + 1: PAT_KF(8, 1); break;
-    case 1 * 4 + 3: PAT_KF(1, 3); break;
-    case 2 * 4 + 3: PAT_KF(2, 3); break;
-    case 4 * 4 + 3: PAT_KF(4, 3); break;
-    case 8 * 4 + 3: PAT_KF(8, 3); break;
+#define PAT_KF(KS_)                                                                                                    \
+    hipLaunchKernelGGL((km_finalize<KS_>), g, b, 0, st, d.c, d.K, d.K_pad, d.D, d.gsum, d.gcnt, d.gdsum, inv, update,  \
+                       (__bf16 *)d.cb, d.cnorm, d.snap)
+    switch (d.KS) {
+    case 1: PAT_KF(1); break;
+    case 2: PAT_KF(2); break;
+    case 4: PAT_KF(4); break;
+    case 8: PAT_KF(8); break;
     default: pat::set_error("kmeans: D = %d or terms %d not supported", d.D, d.NT); return PAT_ERR_UNSUPPORTED;
     }
 #undef PAT_KF
@@ -1950,23 +1994,17 @@ int kmeans_assign_mfma(const KmDev &d, hipStream_t st)
     PAT_REQUIRE(!d.gc || d.NT == 3, PAT_ERR_STATE, "kmeans: global-row MFMA form needs three terms");
     const int64_t lds = mfma_lds_bytes(d.K, d.D, d.NT, d.gc != 0);
     PAT_REQUIRE(lds <= g_lds_limit, PAT_ERR_UNSUPPORTED, "kmeans: K=%d, D=%d too large for the MFMA path", d.K, d.D);
-    // Error-bound constants.  u = 2^-8 (BF16 unit roundoff); g = FP32
-    // accumulation over every term of the MFMA chain, with a factor 2 of
-    // slack for any internal rounding mode.
-    //  NT = 1: |x.c - bf(x).bf(c)| <= (2u + u^2) sum |x_d c_d|.
-    //  NT = 3: x = xh + xl + rx with |rx| <= u^2 |x|, |xl| <= u(1+u)|x| (same
-    //          for c); the dropped xl.cl + (terms with rx, rc) are bounded by
-    //          (3u^2 + 4u^3)(1+u)^2 sum |x_d c_d|.
-    //  Both scaled by 2 for the -2 factor; the norm split leaves u^3 ||c||^2.
-    const double u = ldexp(1.0, -8), g = 2.0 * (16.0 * (d.NT * d.KS + 1)) * ldexp(1.0, -24);
+    // Error-bound constants of the one-term form.  u = 2^-8 (BF16 unit
+    // roundoff); g = FP32 accumulation over every term of the MFMA chain, with
+    // a factor 2 of slack for any internal rounding mode.
+    // |x.c - bf(x).bf(c)| <= (2u + u^2) sum |x_d c_d|, scaled by 2 for the -2
+    // factor; the norm split leaves u^3 ||c||^2.
+    const double u = ldexp(1.0, -8), g = 2.0 * (16.0 * (d.KS + 1)) * ldexp(1.0, -24);
     MfmaBound bd;
-    if (d.NT == 3)
-        bd.c_dot = (float)((2 * (3 * u * u + 4 * u * u * u) * (1 + u) * (1 + u) +
-                            2 * g * (1 + u) * (1 + u) * (1 + 2 * u)) * 1.01);
-    else
-        bd.c_dot = (float)((4 * u + 2 * u * u + 4 * g * (1 + u) * (1 + u)) * 1.01);
+    bd.c_dot = (float)((4 * u + 2 * u * u + 4 * g * (1 + u) * (1 + u)) * 1.01);
     bd.c_norm = (float)((u * u * u + 2 * g * (1 + 2 * u)) * 1.01);
     bd.c_ref = (float)((3.0 + d.D + 16.0) * ldexp(1.0, -24) * 1.01);
+    const WideBound wb = wide_bound(d);
     // one workgroup per CU (the LDS holds one), BS_ / 64 wavefronts each.  While
     // the points do not fill the chip every wavefront takes one tile (rounded
     // down, a few took two, and 10 iterations of 3,000 x 4, K 8 took 165 us, not 137).  Smaller
@@ -1984,11 +2022,11 @@ int kmeans_assign_mfma(const KmDev &d, hipStream_t st)
         if (tail) {                                                                                                    \
             PAT_TRY(allow_lds((const void *)km_mfma<KS_, KB_, NT_, true, GC_, BS_>, lds));                             \
             hipLaunchKernelGGL((km_mfma<KS_, KB_, NT_, true, GC_, BS_>), dim3(grid_for(BS_)), dim3(BS_), (size_t)lds,  \
-                               st, a, (const __bf16 *)d.cb, d.cnorm, d.K_pad, bd, d.rescored);                         \
+                               st, a, (const void *)d.cb, d.cnorm, d.K_pad, bd, wb, d.rescored);                       \
         } else {                                                                                                       \
             PAT_TRY(allow_lds((const void *)km_mfma<KS_, KB_, NT_, false, GC_, BS_>, lds));                            \
             hipLaunchKernelGGL((km_mfma<KS_, KB_, NT_, false, GC_, BS_>), dim3(grid_for(BS_)), dim3(BS_), (size_t)lds, \
-                               st, a, (const __bf16 *)d.cb, d.cnorm, d.K_pad, bd, d.rescored);                         \
+                               st, a, (const void *)d.cb, d.cnorm, d.K_pad, bd, wb, d.rescored);                       \
         }                                                                                                              \
     } while (0)
 #define PAT_KM_GC(KS_, KB_, NT_, GC_) PAT_KM_BS(KS_, KB_, NT_, GC_, 512)
@@ -2009,10 +2047,17 @@ int kmeans_assign_mfma(const KmDev &d, hipStream_t st)
     case 2 * 4 + 1: PAT_KM(2, 8, 1); break;
     case 4 * 4 + 1: PAT_KM(4, 4, 1); break;
     case 8 * 4 + 1: PAT_KM(8, 2, 1); break;
-    case 1 * 4 + 3: PAT_KM_BS(1, 4, 3, false, 768); break;  // 3 wavefronts per SIMD
+    case 1 * 4 + 3: PAT_KM_BS(1, 1, 3, false, 768); break;  // 3 wavefronts per SIMD
     case 2 * 4 + 3: PAT_KM_BS(2, 1, 3, false, 768); break;  // 3 wavefronts per SIMD
-    case 4 * 4 + 3: PAT_KM_BS(4, 2, 3, false, 768); break;  // 3 wavefronts per SIMD
-    case 8 * 4 + 3: PAT_KM(8, 2, 3); break;
+    case 4 * 4 + 3:
+        // a full row stays in registers for the exact distances, at two
+        // wavefronts per SIMD (1 M x 64, K 150: 142 us a pass, 196 with three
+        // and the row read again); a row with a tail is read again in any case
+        // (1 M x 50, K 100: 131 us with three, 148 with two)
+        if (tail) PAT_KM_BS(4, 1, 3, false, 768);
+        else PAT_KM_BS(4, 1, 3, false, 512);
+        break;
+    case 8 * 4 + 3: PAT_KM(8, 1, 3); break;
     default: pat::set_error("kmeans: D too large"); return PAT_ERR_UNSUPPORTED;
     }
 #undef PAT_KM

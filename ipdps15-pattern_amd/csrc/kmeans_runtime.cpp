@@ -28,8 +28,6 @@ struct pat_kmeans {
     int mode = PAT_KM_MFMA;
     bool own_x = false;
     float *xbuf = nullptr;
-    void *rowbuf = nullptr;   // BF16 rows
-    void *widebuf = nullptr;  // FP16 rows (wide path)
     unsigned long long *maxbits = nullptr;
     hipStream_t stream = nullptr;
     float maxabs = 0.0f;
@@ -58,9 +56,9 @@ struct pat_kmeans {
         if (stream) (void)hipStreamSynchronize(stream);
         drop_graphs();
         for (void *p : {(void *)xbuf, (void *)d.c, (void *)d.assign, (void *)d.mindist, (void *)d.gsum, (void *)d.gcnt,
-                        (void *)d.gdsum, rowbuf, (void *)d.cnorm, (void *)d.rescored,
+                        (void *)d.gdsum, d.cb, (void *)d.cnorm, (void *)d.rescored,
                         (void *)maxbits, (void *)d.snap, (void *)d.bidx, (void *)d.bcnt, (void *)d.boff,
-                        (void *)d.bcur, (void *)d.bpart, widebuf})
+                        (void *)d.bcur, (void *)d.bpart})
             if (p) (void)pat::dev_free(p);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -167,8 +165,7 @@ int setup(pat_kmeans *h, const float *x, int64_t n, int d, int k, int mode, int 
     PAT_TRY(amalloc((void **)&D.gsum, 8 * (size_t)k * d));
     PAT_TRY(amalloc((void **)&D.gcnt, 8 * (size_t)k));
     PAT_TRY(amalloc((void **)&D.gdsum, 8 * (size_t)k));
-    PAT_TRY(amalloc(&h->rowbuf, 2 * (size_t)D.K_pad * 16 * (D.NT * D.KS + 1)));
-    D.cb = h->rowbuf;
+    PAT_TRY(amalloc(&D.cb, 2 * (size_t)pat::kmeans_wide_row_words(D.K_pad, d)));
     PAT_TRY(amalloc((void **)&D.cnorm, sizeof(float) * (size_t)k));
     // a reduction object too large for LDS is summed bucket by bucket
     D.bucketed = !pat::kmeans_object_in_lds(k, d) && n < (1LL << 31);
@@ -181,9 +178,7 @@ int setup(pat_kmeans *h, const float *x, int64_t n, int d, int k, int mode, int 
         PAT_TRY(amalloc((void **)&D.bpart, sizeof(int) * (size_t)pat::kmeans_bucket_part_words(n, k, D.cus)));
         // the assignment then leaves min_dist to the reduction, and its FP16
         // form is the faster one for every such shape
-        PAT_TRY(amalloc(&h->widebuf, 2 * (size_t)pat::kmeans_wide_row_words(D.K_pad, d)));
         D.wide = 1;
-        D.cb = h->widebuf;
     }
     PAT_TRY(amalloc((void **)&D.rescored, 8));
     PAT_TRY(amalloc((void **)&h->maxbits, 8));
@@ -273,7 +268,6 @@ int pat_kmeans_set_terms(pat_kmeans *h, int terms)
     if (D.NT != terms || D.wide) {
         D.NT = terms;
         D.wide = 0;
-        D.cb = h->rowbuf;
         PAT_TRY(pat::kmeans_finalize(D, 0, h->stream));
         PAT_HIP(hipStreamSynchronize(h->stream));
         h->drop_graphs();
@@ -291,15 +285,14 @@ int pat_kmeans_get_terms(pat_kmeans *h, int *terms)
 int pat_kmeans_set_centroids(pat_kmeans *h, const float *c)
 {
     PAT_REQUIRE(h && c, PAT_ERR_INVALID, "pat_kmeans_set_centroids: null argument");
-    if (h->d.wide) {  // the rows' scale covers the points and the centres
-        float m = h->maxabs;
-        for (int64_t i = 0; i < (int64_t)h->d.K * h->d.D; i++)
-            if (std::isfinite(c[i])) m = std::max(m, std::fabs(c[i]));
-        const int e = pat::kmeans_wide_exp(m);
-        if (e != h->d.wexp) {
-            h->d.wexp = e;
-            h->drop_graphs();
-        }
+    // the FP16 rows' scale covers the points and the centres
+    float m = h->maxabs;
+    for (int64_t i = 0; i < (int64_t)h->d.K * h->d.D; i++)
+        if (std::isfinite(c[i])) m = std::max(m, std::fabs(c[i]));
+    const int e = pat::kmeans_wide_exp(m);
+    if (e != h->d.wexp) {
+        h->d.wexp = e;
+        h->drop_graphs();
     }
     PAT_HIP(hipMemcpyAsync(h->d.c, c, sizeof(float) * (size_t)h->d.K * h->d.D, hipMemcpyHostToDevice, h->stream));
     PAT_TRY(pat::kmeans_finalize(h->d, 0, h->stream));

@@ -267,3 +267,43 @@ def test_wide_path_two_tiles(pa, orc, gpu):
         km.close()
         ra, rmd = orc.kmeans_assign(x, c)
         assert np.array_equal(a, ra) and np.array_equal(md, rmd)
+
+
+@pytest.mark.parametrize("n,d,k", [(31, 3, 1), (700, 8, 31), (1000, 8, 33), (3000, 16, 512), (3000, 16, 513),
+                                   (2500, 13, 257), (4000, 32, 255), (4000, 31, 64), (3000, 64, 129), (3000, 50, 70),
+                                   (2000, 128, 60), (2000, 99, 40)])
+@pytest.mark.parametrize("terms", [1, 3])
+def test_pair_keys_bitexact(pa, orc, gpu, n, d, k, terms):
+    """Objects in LDS: keys of pairs of adjacent centres up to 512 centres and
+    of single ones beyond, one or two 32-centre blocks to the end, rows with
+    and without a tail; then centres that repeat within a pair, across the two
+    halves of a block and across blocks (equal keys: the lowest index wins),
+    some far outside the points' range and one that is not finite."""
+    x = pa.gen_gmm(n, d, max(1, k // 2), sigma=1.0, seed=n + d + k)
+    km = pa.KMeans(x, k, mode=1)
+    if terms == 3 and km.terms() != 3:
+        pytest.skip("three terms do not fit")
+    km.set_terms(terms)
+    km.run(2)
+    c, a, md = km.get()
+    sums, counts, dsums, s, ds = km.get_object()
+    *_, (c1, ra, rmd, rsums, rcounts, rdsum) = oracle_iters(orc, pa, x, k, 2)
+    assert np.array_equal(a, ra) and np.array_equal(md, rmd)
+    assert np.array_equal(sums, rsums) and np.array_equal(counts, rcounts) and np.array_equal(dsums, rdsum)
+    assert np.array_equal(c, orc.kmeans_update(rsums, rcounts, s, c1))
+    odd = x[:k].copy()
+    for i, j in ((0, 1), (2, 6), (3, 4), (5, 37), (8, 9), (10, 14), (11, 12), (13, 140)):
+        if j < k:
+            odd[j] = odd[i]
+    if k > 24:
+        odd[20] *= 1024.0
+        odd[21] = -odd[20]
+        if terms == 3:
+            odd[22, 0] = np.inf
+            odd[23, -1] = np.nan
+    km.set_centroids(odd)
+    km.run(1)
+    _, a, md = km.get()
+    km.close()
+    ra, rmd = orc.kmeans_assign(x, odd)
+    assert np.array_equal(a, ra) and np.array_equal(md, rmd)
