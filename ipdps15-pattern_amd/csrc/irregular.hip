@@ -260,12 +260,12 @@ static inline unsigned row_sort_grid(int64_t N)
 // Two passes over the edge list and one over its entries, in place of a
 // degree histogram and a scatter by one returning atomic per entry into
 // global memory (13.3 M entries of 256,000 rows: 0.50 + 1.14 of 1.6 ms, bound
-// by the atomics; 0.27 ms now, csr_scatter 0.13 of it, bound by its partial
-// lines).  Rows are grouped into buckets of 2^shift; csr_count counts
-// each workgroup's entries per bucket in LDS and reserves its part of every
-// bucket with one atomic; csr_scatter writes the entries there, so a bucket
-// gets runs of neighbouring 8-byte words; csr_rows takes a bucket into LDS,
-// counts and places its rows, sorts them and writes row pointers and columns.
+// by the atomics; 0.15 ms now: 28 + 51 + 62 us).  Rows are grouped into buckets
+// of 2^shift; csr_count counts each workgroup's entries per bucket in LDS and
+// reserves its part of every bucket with one atomic; csr_scatter_runs, or
+// csr_scatter where an entry needs 8 bytes, writes the entries there; csr_rows
+// takes a bucket into LDS, counts and places its rows, sorts them and writes
+// row pointers and columns.
 //
 // Entry: the row within the bucket << 32 | a 32-bit key that orders the row:
 // the neighbour (rows in node order) or the place 2 e + side of this endpoint
@@ -276,6 +276,8 @@ enum CsrOut { kCsrEdgeOrder = 0, kCsrNodeOrder = 1, kCsrEdgeIds = 2 };
 
 constexpr int kCsrThreads = 512;
 constexpr int kCsrMaxBuckets = 8192;   // counted in LDS: 32 KB
+constexpr int kCsrStageThreads = 1024;
+constexpr int kCsrStageEdges = 13 * kCsrStageThreads;  // csr_scatter_runs: 104 KB of entries
 constexpr int kCsrCap = 10240;         // entries of a group of rows held in LDS (40 KB)
 constexpr int kCsrRows = 2048;         // rows counted in LDS at a time (8 KB): three workgroups per CU
 
@@ -359,13 +361,84 @@ __global__ __launch_bounds__(kCsrThreads) void csr_scatter(const int2 *__restric
     });
 }
 
+// The same with 4-byte entries (row << 32 - shift | key, where the keys fit) and
+// the workgroup's entries grouped by bucket in LDS first, so that a bucket gets
+// whole runs: 16 lanes write a bucket's run.  13.3 M entries in 2,000 buckets:
+// 51 us, 130 with csr_scatter, whose stores of single 8-byte words L2 takes one
+// by one.  The edges and their places within the bucket stay in registers
+// between the passes.
+__global__ __launch_bounds__(kCsrStageThreads) void csr_scatter_runs(const int2 *__restrict__ edges, int64_t E,
+                                                                     int64_t chunk, int shift, int B,
+                                                                     const int *__restrict__ start,
+                                                                     const int *__restrict__ part, int node_order,
+                                                                     unsigned *__restrict__ ent)
+{
+    constexpr int PER = kCsrStageEdges / kCsrStageThreads, T = kCsrStageThreads;
+    __shared__ unsigned buf[2 * kCsrStageEdges];
+    __shared__ int h[kCsrMaxBuckets + 1];
+    __shared__ int wsum[T / kWave];
+    const int t = (int)threadIdx.x, lane = t % kWave, wv = pat::wave_in_block();
+    const int64_t c0 = (int64_t)blockIdx.x * chunk;
+    const int n = (int)min(chunk, E - c0);
+    int2 ij[PER];
+    int ri[PER], rj[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) ij[u] = edges[c0 + min(u * T + t, n - 1)];
+    for (int b = t; b <= B; b += T) h[b] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+        if (u * T + t < n) {
+            ri[u] = atomicAdd(&h[ij[u].x >> shift], 1);
+            rj[u] = atomicAdd(&h[ij[u].y >> shift], 1);
+        }
+    __syncthreads();
+    // exclusive sums of h[0..B]
+    const int per = (B + T) / T, b0 = min(B + 1, t * per), b1 = min(B + 1, b0 + per);
+    int mine = 0;
+    for (int b = b0; b < b1; b++) mine += h[b];
+    int x = mine;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int y = __shfl_up(x, o, kWave);
+        if (lane >= o) x += y;
+    }
+    if (lane == kWave - 1) wsum[wv] = x;
+    __syncthreads();
+    int at = x - mine;
+    for (int v = 0; v < wv; v++) at += wsum[v];
+    for (int b = b0; b < b1; b++) {
+        const int c = h[b];
+        h[b] = at;
+        at += c;
+    }
+    __syncthreads();
+    const int low = (1 << shift) - 1, kb = 32 - shift;
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+        if (u * T + t < n) {
+            const unsigned e = (unsigned)(c0 + u * T + t);
+            const unsigned ki = node_order ? (unsigned)ij[u].y : 2u * e, kj = node_order ? (unsigned)ij[u].x : 2u * e + 1u;
+            buf[h[ij[u].x >> shift] + ri[u]] = (unsigned)((uint64_t)(ij[u].x & low) << kb) | ki;
+            buf[h[ij[u].y >> shift] + rj[u]] = (unsigned)((uint64_t)(ij[u].y & low) << kb) | kj;
+        }
+    __syncthreads();
+    for (int b = t / 16; b < B; b += T / 16) {
+        const int s = h[b], m = h[b + 1] - s;
+        if (m == 0) continue;
+        const int g = start[b] + part[(int64_t)blockIdx.x * B + b];
+        for (int i = t % 16; i < m; i += 16) ent[g + i] = buf[s + i];
+    }
+}
+
 // One workgroup per bucket.  Its rows are counted kCsrRows at a time and
 // taken into LDS in groups of rows of at most kCsrCap entries (usually the
 // whole bucket at once; further groups read the bucket's entries again).
 // Rows of at most 128 entries are sorted in registers, four per wavefront;
 // longer ones by the workgroup in LDS; a row beyond kCsrCap by ranks.
-template <int OUT>
-__global__ __launch_bounds__(kCsrThreads) void csr_rows(const unsigned long long *__restrict__ ent,
+// V: the entry's type, kb: the bits of its key.
+template <int OUT, typename V>
+__global__ __launch_bounds__(kCsrThreads) void csr_rows(const V *__restrict__ ent, int kb,
                                                         const int *__restrict__ start, int64_t N, int shift,
                                                         const int *__restrict__ flat, int *__restrict__ rowptr,
                                                         int *__restrict__ cols)
@@ -380,23 +453,26 @@ __global__ __launch_bounds__(kCsrThreads) void csr_rows(const unsigned long long
     auto out = [&](unsigned key) {
         return OUT == kCsrNodeOrder ? (int)key : (OUT == kCsrEdgeOrder ? flat[key ^ 1u] : (int)(key >> 1));
     };
+    const unsigned mask = (unsigned)((1ull << kb) - 1);
+    auto row_of = [&](V v) { return (int)((unsigned long long)v >> kb); };
+    auto key_of = [&](V v) { return (unsigned)v & mask; };
     // entries of rows [w, w + n) of the bucket, four in flight per thread
     auto entries = [&](int w, int n, auto f) {
         int i = s + t;
         for (; i + 3 * kCsrThreads < e; i += 4 * kCsrThreads) {
-            unsigned long long v[4];
+            V v[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) v[u] = ent[i + u * kCsrThreads];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const int r = (int)(v[u] >> 32) - w;
-                if (r >= 0 && r < n) f(r, (unsigned)v[u], i + u * kCsrThreads);
+                const int r = row_of(v[u]) - w;
+                if (r >= 0 && r < n) f(r, key_of(v[u]), i + u * kCsrThreads);
             }
         }
         for (; i < e; i += kCsrThreads) {
-            const unsigned long long v = ent[i];
-            const int r = (int)(v >> 32) - w;
-            if (r >= 0 && r < n) f(r, (unsigned)v, i);
+            const V v = ent[i];
+            const int r = row_of(v) - w;
+            if (r >= 0 && r < n) f(r, key_of(v), i);
         }
     };
     int base = s;  // place of the window's first entry
@@ -453,8 +529,8 @@ __global__ __launch_bounds__(kCsrThreads) void csr_rows(const unsigned long long
                 entries(w + g, 1, [&](int, unsigned key, int i) {
                     int rank = 0;
                     for (int j = s; j < e; j++) {
-                        const unsigned long long v = ent[j];
-                        rank += (int)(v >> 32) == w + g && ((unsigned)v < key || ((unsigned)v == key && j < i));
+                        const V v = ent[j];
+                        rank += row_of(v) == w + g && (key_of(v) < key || (key_of(v) == key && j < i));
                     }
                     cols[gs + rank] = out(key);
                 });
@@ -2030,13 +2106,19 @@ static int csr_buckets(const char *who, const int32_t *edges, int64_t E, int64_t
            ((N - 1) >> shift) + 1 > kCsrMaxBuckets)
         shift++;
     const int B = (int)(((N - 1) >> shift) + 1);
+    // 4-byte entries where the row within a bucket and the key fit: the
+    // neighbour, or twice the edge (csr_scatter_runs)
+    const int kb = 32 - shift;
+    const bool fits = (out == kCsrNodeOrder ? N : 2 * E) <= 1LL << kb;
     // Edges per workgroup: enough for runs of several entries per bucket, and
-    // about 400 workgroups where the list is that long.  The totals (B) and
+    // about 400 workgroups where the list is that long (or two for each CU, one
+    // at a time, with the entries in LDS).  The totals (B) and
     // the workgroups' parts (wgs x B) lie behind the starts (B + 1) where the
     // N + 1 words hold them, else in cols (2 E words) until csr_rows writes
     // it; one of the two holds them at the latest with one workgroup, since
     // buckets of fewer than four rows mean over 64 entries per row.
-    int64_t chunk = std::max<int64_t>(2048, std::min<int64_t>(16384, (E + 399) / 400));
+    int64_t chunk = fits ? std::max<int64_t>(2048, std::min<int64_t>(kCsrStageEdges, (E + 511) / 512))
+                         : std::max<int64_t>(2048, std::min<int64_t>(16384, (E + 399) / 400));
     int64_t wgs = (E + chunk - 1) / chunk;
     auto beside = [&] { return (wgs + 2) * B <= N; };
     while (wgs > 1 && !beside() && (wgs + 1) * B > 2 * E) {
@@ -2045,9 +2127,10 @@ static int csr_buckets(const char *who, const int32_t *edges, int64_t E, int64_t
     }
     PAT_REQUIRE(beside() || (wgs + 1) * B <= 2 * E, PAT_ERR_STATE, "%s: no room for the bucket counts", who);
     int *start = (int *)work, *total = beside() ? start + B + 1 : cols, *part = total + B;
-    // the entries: 2 E eight-byte words behind the N + 1 words (rounded up to
-    // 16 bytes within the work space's 256 spare ones)
-    auto *ent = (unsigned long long *)(((uintptr_t)work + sizeof(int) * (size_t)(N + 1) + 15) & ~(uintptr_t)15);
+    // the entries: 2 E words of 4 or 8 bytes behind the N + 1 words (rounded
+    // up to 16 bytes within the work space's 256 spare ones)
+    void *ent = (void *)(((uintptr_t)work + sizeof(int) * (size_t)(N + 1) + 15) & ~(uintptr_t)15);
+    const bool runs = fits && chunk <= kCsrStageEdges;
     const int2 *e2 = (const int2 *)edges;
     hipLaunchKernelGGL(fill_i32, dim3(grid_for(B)), dim3(256), 0, st, total, (int64_t)B, 0);
     PAT_LAUNCH_CHECK();
@@ -2055,13 +2138,22 @@ static int csr_buckets(const char *who, const int32_t *edges, int64_t E, int64_t
     PAT_LAUNCH_CHECK();
     hipLaunchKernelGGL(csr_starts, dim3(1), dim3(kScanBlock), 0, st, (const int *)total, B, start);
     PAT_LAUNCH_CHECK();
-    hipLaunchKernelGGL(csr_scatter, dim3((unsigned)wgs), dim3(kCsrThreads), 0, st, e2, E, chunk, shift, B,
-                       (const int *)start, (const int *)part, out == kCsrNodeOrder, ent);
+    if (runs)
+        hipLaunchKernelGGL(csr_scatter_runs, dim3((unsigned)wgs), dim3(kCsrStageThreads), 0, st, e2, E, chunk, shift, B,
+                           (const int *)start, (const int *)part, out == kCsrNodeOrder, (unsigned *)ent);
+    else
+        hipLaunchKernelGGL(csr_scatter, dim3((unsigned)wgs), dim3(kCsrThreads), 0, st, e2, E, chunk, shift, B,
+                           (const int *)start, (const int *)part, out == kCsrNodeOrder, (unsigned long long *)ent);
     PAT_LAUNCH_CHECK();
-    auto k = out == kCsrNodeOrder ? csr_rows<kCsrNodeOrder>
-                                  : (out == kCsrEdgeOrder ? csr_rows<kCsrEdgeOrder> : csr_rows<kCsrEdgeIds>);
-    hipLaunchKernelGGL(k, dim3((unsigned)B), dim3(kCsrThreads), 0, st, (const unsigned long long *)ent,
-                       (const int *)start, N, shift, (const int *)edges, rowptr, cols);
+    auto rows = [&](auto v, int bits) {
+        using V = decltype(v);
+        auto k = out == kCsrNodeOrder ? csr_rows<kCsrNodeOrder, V>
+                                      : (out == kCsrEdgeOrder ? csr_rows<kCsrEdgeOrder, V> : csr_rows<kCsrEdgeIds, V>);
+        hipLaunchKernelGGL(k, dim3((unsigned)B), dim3(kCsrThreads), 0, st, (const V *)ent, bits, (const int *)start, N,
+                           shift, (const int *)edges, rowptr, cols);
+    };
+    if (runs) rows(0u, kb);
+    else rows(0ull, 32);
     PAT_LAUNCH_CHECK();
     return PAT_OK;
 }

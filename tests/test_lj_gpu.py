@@ -122,6 +122,23 @@ def test_csr_build_forms(pa, gpu, kind, order):
     assert np.array_equal(cols.numpy(), both[:, 1])
 
 
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("n,e", [(50021, 1100003), (50021, 6900001), (3000017, 1500001), (1 << 21, 1 << 20)])
+def test_csr_build_long_lists(pa, gpu, n, e, order):
+    """Workgroups with a part and with all of the edges that LDS holds, more
+    than two workgroups per CU, and entries of 4 and 8 bytes on both sides of
+    the sizes where a row and its key fit 32 bits."""
+    edges = np.random.default_rng(n + e).integers(0, n, (e, 2), dtype=np.int32)
+    edges = edges[edges[:, 0] != edges[:, 1]]
+    rowptr, cols = pa.csr_build_dev(pa.DeviceArray.from_numpy(edges), len(edges), n, order=order)
+    row = np.concatenate([edges[:, 0], edges[:, 1]]).astype(np.int64)
+    col = np.concatenate([edges[:, 1], edges[:, 0]])
+    key = col if order else np.concatenate([np.arange(len(edges))] * 2)
+    by = np.argsort(row << 32 | key, kind="stable")
+    assert np.array_equal(rowptr.numpy(), np.concatenate([[0], np.cumsum(np.bincount(row, minlength=n))]))
+    assert np.array_equal(cols.numpy(), col[by])
+
+
 @pytest.mark.parametrize("lpr", [1, 4, 8, 16, 32, -4, -8, -16, -32, -64])
 def test_force_csr_vs_oracle(pa, orc, gpu, small, lpr):
     pos, box, edges = small
