@@ -464,9 +464,9 @@ constexpr float kFar = 3.0e38f;
 // reduction object from the registers holding its half rows.
 //
 // Bound by instruction issue, vector and matrix together: 2^24 x 32, K 256,
-// 1.16 ms a pass (1.31 with BF16 parts and a key for every value; the wider
-// bound of those left 2.3% of the points several candidates, of every second
-// tile one).  One block of centres per chunk at every KS: its two accumulators
+// 20 passes: 1.41 ms each (1.54 with BF16 parts and a key for every value; the
+// wider bound of those left 2.3% of the points several candidates, one in every
+// second tile; 0.3% now).  One block of centres per chunk at every KS: its two accumulators
 // and the registers around them fit without spills (1 M x 8, K 16: 41 us with
 // one, 54 with four; 1 M x 16, K 128: 55 and 64), and the matrix cores work on
 // the next block during a scan.
