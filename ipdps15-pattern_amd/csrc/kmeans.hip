@@ -931,7 +931,7 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const void *__restrict__
 //
 // Bound by the matrix cores: 3 KS + 1 MFMAs per 32 x 32 values, issued at 1.03
 // PFLOP/s at D = 128 (a large library product reaches 1.18 on this card); the
-// scan takes 4 vector instructions a value.  1 M x 128, K 1,000: 0.84 ms a pass,
+// scan takes 4 vector instructions a value.  1 M x 128, K 1,000: 0.80-0.84 ms a pass,
 // 0.7% of the points rescored (2.66 ms with BF16 terms and a second pass over
 // the centres in nearly every workgroup).
 template <int KS, int NB, int TILES, bool TAIL>
