@@ -176,7 +176,7 @@ int pat_stencil_set_table(pat_stencil *s, const pat_stencil_table *table);
 /* Selects the kernel variant and tile (0 = tuned). */
 int pat_stencil_set_variant(pat_stencil *s, int variant, int bx, int by, int zc);
 /* Copies a halo-inclusive host grid in (the app writes grid()->data(),
- * heat_3D/main.cpp:72-75). */
+ * heat_3D/main.cpp:72-75).  The halo's values are kept through the sweeps. */
 int pat_stencil_upload(pat_stencil *s, const void *host);
 /* StencilBegin for nsteps iterations (kmeans/lib/stencil_runtime.cu:576-614). */
 int pat_stencil_run(pat_stencil *s, int nsteps);
@@ -194,7 +194,9 @@ int pat_stencil_download(pat_stencil *s, void *host);
 /* Tile the runs use (tuned on the first run when none was set): x width,
  * tile height in rows, z-chunk in planes. */
 int pat_stencil_tile(pat_stencil *s, int *bx, int *by, int *zc);
-/* Device pointer of the current grid. */
+/* Device pointer of the current grid.  A halo written through it is read by
+ * the next sweep if that is a run of its own (one step); the values for runs
+ * of several steps are those of the last upload. */
 int pat_stencil_device_ptr(pat_stencil *s, void **dptr);
 /* StencilFinalize + delete. */
 int pat_stencil_destroy(pat_stencil *s);

@@ -1053,7 +1053,10 @@ int heat3d_steps(float *const buf[2], int start, int64_t nx, int64_t ny, int64_t
             c = 1 - c;
         }
     }
-    if (k < nsteps && t.fused == 3) {  // the sweeps left over, in launches of fewer
+    // the sweeps left over, in launches of fewer -- but a run of one sweep goes
+    // by the plain kernel, which reads the halo: a program that exchanges halos
+    // through the device pointer runs one sweep at a time
+    if (k < nsteps && t.fused == 3 && nsteps > 1) {
         HeatTile p = t;
         for (; k < nsteps; k += p.sweeps) {
             p.sweeps = strip_sweeps(nsteps - k);
@@ -1085,30 +1088,48 @@ int heat3d_steps(float *const buf[2], int start, int64_t nx, int64_t ny, int64_t
 // every tile gives the same bits on any grid.  The other kernels are no
 // candidates: strips were faster on every grid tried from 1 cell to 384^3 (us
 // per step, strips against the fastest other: 32^3 1.4 and 2.2, 64^3 1.6 and
-// 2.9, 128^3 3.3 and 5.3, 256^3 10.3 and 15.8, 384^3 32.0 and 59.1).
-static std::map<std::tuple<int, int, int>, HeatTile> g_tile_cache;
+// 2.9, 128^3 3.3 and 5.3, 256^3 10.3 and 15.8, 384^3 32.0 and 59.1) -- except
+// where the halo is not zero (zero_halo false), as the strips and the two-sweep
+// window take it to be between their sweeps: then the single sweeps and the LDS
+// cubes, which read it.
+static std::map<std::tuple<int, int, int, bool>, HeatTile> g_tile_cache;
 static std::mutex g_tile_mutex;
 
 static int size_class(int64_t n) { return (int)std::floor(2.0 * std::log2((double)n)); }
 
 int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha, hipStream_t st,
-                 HeatTile *t)
+                 bool zero_halo, HeatTile *t)
 {
-    const auto key = std::make_tuple(size_class(nx), size_class(ny), size_class(nz));
+    const auto key = std::make_tuple(size_class(nx), size_class(ny), size_class(nz), zero_halo);
     {
         std::lock_guard<std::mutex> g(g_tile_mutex);
         auto it = g_tile_cache.find(key);
+        if (it != g_tile_cache.end() && it->second.fused != 3) {
+            *t = it->second;
+            t->zc = (int)std::min<int64_t>(t->zc, nz);
+            return PAT_OK;
+        }
         if (it != g_tile_cache.end() &&
             strip_tile(it->second.shape, it->second.sweeps, it->second.fill, nx, ny, nz, t))
             return PAT_OK;
     }
-    if (!strip_default(nx, ny, nz, t)) {  // planes of 4 GiB and more
+    if (!zero_halo) {
+        t->fused = 0;
+        default_tile(nx, ny, nz, &t->bx, &t->by, &t->ry, &t->zc);
+    } else if (!strip_default(nx, ny, nz, t)) {  // planes of 4 GiB and more
         *t = HeatTile{1, 64, 4, 4, (int)std::min<int64_t>(64, nz)};
         return PAT_OK;
     }
     if (!pat::tuning_enabled()) return PAT_OK;
     std::vector<HeatTile> cands;
-    for (int c = 0; c < kNumStrips; c++)
+    if (!zero_halo) {
+        for (const auto &sh : kShapes)
+            for (int z : {2, 4, 8, 16, 32, 64})
+                if (z <= nz || z == 2) cands.push_back(HeatTile{0, sh.bx, sh.by, sh.ry, (int)std::min<int64_t>(z, nz)});
+        PAT_TRY(cube_prepare());  // before any capture
+        for (int c = 0; c < kNumCubes; c++) cands.push_back(HeatTile{2, c, 0, kCubes[c].t, 0});
+    }
+    for (int c = 0; zero_halo && c < kNumStrips; c++)
         for (int sweeps : {3, 4, 6})
             for (int fill : {1, 2, 3, 4}) {
                 HeatTile h;
@@ -1201,9 +1222,10 @@ int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz
         if (tm[c] < tm[bi]) bi = c;
     if (pat::tune_log())
         for (size_t c = 0; c < cands.size(); c++)
-            fprintf(stderr, "[tune heat3d %lldx%lldx%lld] %d x %d window, %d rows a strip, zc %d, %d sweeps: %.2f us/step%s\n",
-                    (long long)nx, (long long)ny, (long long)nz, cands[c].bx, cands[c].by * cands[c].ry, cands[c].ry,
-                    cands[c].zc, cands[c].sweeps, 1000.0f * tm[c], c == bi ? "  <- chosen" : "");
+            fprintf(stderr, "[tune heat3d %lldx%lldx%lld] form %d, %d x %d window, %d rows, zc %d, %d sweeps: %.2f us/step%s\n",
+                    (long long)nx, (long long)ny, (long long)nz, cands[c].fused, cands[c].bx, cands[c].by * cands[c].ry,
+                    cands[c].ry, cands[c].zc, heat3d_steps_per_launch(cands[c]), 1000.0f * tm[c],
+                    c == bi ? "  <- chosen" : "");
     *t = cands[bi];
     std::lock_guard<std::mutex> g(g_tile_mutex);
     g_tile_cache[key] = *t;
@@ -1257,7 +1279,7 @@ extern "C" int pat_heat3d_run_dev(float *a, float *b, int64_t nx, int64_t ny, in
     hipStream_t st = (hipStream_t)stream;
     pat::HeatTile t;
     if (variant == PAT_STENCIL_AUTO && bx == 0 && by == 0 && zc == 0) {
-        PAT_TRY(pat::heat3d_tuned(a, b, nx, ny, nz, alpha, st, &t));
+        PAT_TRY(pat::heat3d_tuned(a, b, nx, ny, nz, alpha, st, true, &t));  // both halos are 0
     } else if (variant == PAT_STENCIL_CUBES) {
         PAT_TRY(pat::heat3d_cube_tile(bx, &t));
     } else if (variant == PAT_STENCIL_TEMPORAL2) {

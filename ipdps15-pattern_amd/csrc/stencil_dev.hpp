@@ -58,7 +58,7 @@ int heat3d_launch(const float *in, float *out, int64_t nx, int64_t ny, int64_t n
 int heat3d_steps(float *const buf[2], int start, int64_t nx, int64_t ny, int64_t nz, float alpha, const HeatTile &t,
                  int variant, int nsteps, hipStream_t stream, int *end);
 int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha, hipStream_t st,
-                 HeatTile *t);
+                 bool zero_halo, HeatTile *t);
 void heat3d_default_tile(int64_t nx, int64_t ny, int64_t nz, int *bx, int *by, int *ry, int *zc);
 int heat3d_shapes(const int **triples);
 // The tile of LDS cube shape 'shape' (PAT_STENCIL_CUBES); PAT_ERR_UNSUPPORTED

@@ -36,6 +36,7 @@ struct pat_stencil {
     const pat_stencil_table *table = nullptr;  // application functors compiled for the device
     void *param_dev = nullptr;                  // the parameter bytes, for table functors
     bool loaded = false;
+    bool zero_halo = true;  // the uploaded field's halo is all zero bits (3-D FP32 grids of halo width 1)
     hipStream_t stream = nullptr;
     // captured step sequences keyed by (nsteps, starting buffer), with the
     // buffer each leaves the result in
@@ -70,6 +71,29 @@ struct pat_stencil {
         return PAT_OK;
     }
 
+    // Whether every halo cell of a 3-D FP32 field of halo width 1 is zero bits.
+    bool halo_is_zero(const uint32_t *g) const
+    {
+        const int64_t sx = n[0] + 2, sy = n[1] + 2, sz = n[2] + 2;
+        auto clear = [&](const uint32_t *p, int64_t cells) {
+            uint32_t any = 0;
+            for (int64_t i = 0; i < cells; i++) any |= p[i];
+            return any == 0;
+        };
+        for (int64_t z = 0; z < sz; z++) {
+            const uint32_t *p = g + z * sy * sx;
+            if (z == 0 || z == sz - 1) {
+                if (!clear(p, sy * sx)) return false;
+                continue;
+            }
+            if (!clear(p, sx) || !clear(p + (sy - 1) * sx, sx)) return false;
+            uint32_t any = 0;
+            for (int64_t y = 1; y < sy - 1; y++) any |= p[y * sx] | p[y * sx + sx - 1];
+            if (any) return false;
+        }
+        return true;
+    }
+
     // One sweep of the table functor from buffer c into 1 - c.
     int table_sweep(int c, hipStream_t st) const
     {
@@ -92,21 +116,23 @@ struct pat_stencil {
         return a;
     }
 
-    // The tile the runs use: tuned (plain or fused) for AUTO without an
-    // explicit tile, else the variant's default with the set fields.
+    // The tile the runs use: tuned for AUTO without an explicit tile, else the
+    // variant's default with the set fields (single sweeps in place of the
+    // two-sweep window where the halo is not zero: the same bits).
     int resolve_tile(pat::HeatTile *t)
     {
         if (variant == PAT_STENCIL_AUTO && bx == 0 && by == 0 && zc == 0 && loaded) {
-            PAT_TRY(pat::heat3d_tuned(buf[cur], buf[1 - cur], n[0], n[1], n[2], alpha(), stream, t));
+            PAT_TRY(pat::heat3d_tuned(buf[cur], buf[1 - cur], n[0], n[1], n[2], alpha(), stream, zero_halo, t));
             return PAT_OK;
         }
         if (variant == PAT_STENCIL_CUBES) return pat::heat3d_cube_tile(bx, t);
-        if (variant == PAT_STENCIL_TEMPORAL2) {
+        if (variant == PAT_STENCIL_TEMPORAL2 && zero_halo) {
             *t = pat::HeatTile{1, 64, 4, ry > 0 ? ry : 8, zc > 0 ? zc : (int)std::min<int64_t>(64, n[2])};
             return PAT_OK;
         }
         t->fused = 0;
         pat::heat3d_default_tile(n[0], n[1], n[2], &t->bx, &t->by, &t->ry, &t->zc);
+        if (variant == PAT_STENCIL_TEMPORAL2) return PAT_OK;
         if (bx > 0) t->bx = bx;
         if (by > 0) t->by = by;
         if (ry > 0) t->ry = ry;
@@ -262,6 +288,11 @@ int pat_stencil_upload(pat_stencil *s, const void *host)
     PAT_HIP(hipMemcpyAsync(s->buf[0], host, bytes, hipMemcpyHostToDevice, s->stream));
     PAT_HIP(hipMemcpyAsync(s->buf[1], host, bytes, hipMemcpyHostToDevice, s->stream));
     PAT_HIP(hipStreamSynchronize(s->stream));
+    // the multi-sweep kernels that take the halo to be zero are left out
+    // where it is not (heat3d_tuned)
+    const bool zero = s->ndims != 3 || s->width != 1 || s->unit != 4 || s->halo_is_zero((const uint32_t *)host);
+    if (zero != s->zero_halo) s->drop_graphs();
+    s->zero_halo = zero;
     s->cur = 0;
     s->loaded = true;
     return PAT_OK;

@@ -201,3 +201,36 @@ def test_strip_windows_vs_oracle(pa, orc, gpu, shape, sweeps):
             g[1, 1, 1], g[-2, -2, -2], g[2, -2, 3] = np.inf, np.nan, -np.inf
         got = strip_run(pa, g, shape, sweeps, zc)
         assert np.array_equal(got, orc.heat3d(g, sweeps), equal_nan=True), (nx, ny, nz, zc)
+
+
+@pytest.mark.parametrize("shape", [(20, 18, 22), (64, 64, 64), (70, 40, 33)])
+@pytest.mark.parametrize("variant", ["PAT_STENCIL_AUTO", "PAT_STENCIL_TEMPORAL2"])
+def test_halo_values_are_kept(pa, orc, gpu, shape, variant):
+    """A field whose halo is not zero (fixed boundary values): every step count
+    equals the single sweeps, also after a field with a zero halo on the same
+    handle, and a halo written through the device pointer holds for one step."""
+    nx, ny, nz = shape
+    rng = np.random.default_rng(3)
+    zero = pa.gen_heat3d(nx, ny, nz, seed=5)
+    fixed = rng.random((nz + 2, ny + 2, nx + 2), dtype=np.float32)
+    s = pa.Stencil(nx, ny, nz)
+    s.set_variant(getattr(pa, variant))
+    for g in (zero, fixed, zero):
+        s.upload(g)
+        done = 0
+        for steps in (1, 2, 7):
+            s.run(steps)
+            done += steps
+            assert np.array_equal(s.download(), orc.heat3d(g, done)), steps
+    s.upload(fixed)
+    tot, kms = s.run_timed(3)
+    assert np.array_equal(s.download(), orc.heat3d(fixed, 3))
+    s.upload(zero)
+    p = pa.c_vp()
+    pa.call("pat_stencil_device_ptr", s.h, pa.ctypes.byref(p))
+    pa.call("pat_memcpy_h2d", p, fixed.ctypes.data, fixed.nbytes, None)
+    pa.sync()
+    s.run(1)
+    inside = (slice(1, -1),) * 3
+    assert np.array_equal(s.download()[inside], orc.heat3d(fixed, 1)[inside])
+    s.close()
