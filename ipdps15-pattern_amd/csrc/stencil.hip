@@ -1081,21 +1081,63 @@ int heat3d_steps(float *const buf[2], int start, int64_t nx, int64_t ny, int64_t
 
 // Autotuner: times every strip shape with 3, 4 and 6 sweeps and 1 to 4
 // workgroups per CU on the caller's grid (in -> out; out is scratch until the
-// first real sweep writes it, and no kernel writes the halo), keeps the
-// fastest, and caches it for the process per size class: each extent's half
-// octave (floor(2 log2 n)), so a stream of grids of many sizes (a serving mix)
-// tunes once per class; the z-chunk is worked out again for each grid, and
-// every tile gives the same bits on any grid.  The other kernels are no
+// first real sweep writes it, and no kernel writes the halo) and keeps the
+// times for the process per size class: each extent's half octave
+// (floor(2 log2 n)), so a stream of grids of many sizes (a serving mix)
+// tunes once per class.  A grid takes the tile whose time, carried over from
+// the tuned grid by strip_cost, is the least: how well the windows of a shape
+// fit an extent varies within a class (128 x 16 windows, the best at 128^3,
+// at 129^3 need two windows in x), so the best tile itself does not carry
+// over (160^3 with the tile of 128^3: 7.3 us a step; chosen this way 4.5).
+// Every tile gives the same bits on any grid.  The other kernels are no
 // candidates: strips were faster on every grid tried from 1 cell to 384^3 (us
-// per step, strips against the fastest other: 32^3 1.4 and 2.2, 64^3 1.6 and
-// 2.9, 128^3 3.3 and 5.3, 256^3 10.3 and 15.8, 384^3 32.0 and 59.1) -- except
-// where the halo is not zero (zero_halo false), as the strips and the two-sweep
-// window take it to be between their sweeps: then the single sweeps and the LDS
-// cubes, which read it.
-static std::map<std::tuple<int, int, int, bool>, HeatTile> g_tile_cache;
+// per step, strips against the fastest other: 32^3 1.4 and 1.7, 64^3 1.6 and
+// 2.7, 128^3 3.5 and 4.9, 129^3 4.0 and 5.0, 150^3 4.4 and 5.8, 181^3 6.2 and
+// 9.1, 148 x 180 x 133 4.7 and 5.9, 256^3 10.3 and 15.2, 384^3 31.3 and 59.4)
+// -- except where the halo is not zero (zero_halo false), as the strips and
+// the two-sweep window take it to be between their sweeps: then the single
+// sweeps and the LDS cubes, which read it.
+struct HeatTimes {
+    int64_t n[3];  // the tuned grid
+    std::vector<std::pair<HeatTile, float>> tiles;
+};
+static std::map<std::tuple<int, int, int, bool>, HeatTimes> g_tile_cache;
 static std::mutex g_tile_mutex;
 
 static int size_class(int64_t n) { return (int)std::floor(2.0 * std::log2((double)n)); }
+
+// What a launch of strip tile t over a grid takes, up to a factor of the
+// tile: the cells of a window, the planes that it marches, and the rounds of
+// workgroups over the CUs.  From the times of one grid it chose, for another of
+// the class, a tile that took 0.8% longer than that grid's best (the mean over
+// 92 pairs of 16 grids; 16% at most).
+static double strip_cost(const HeatTile &t, int64_t nx, int64_t ny, int64_t nz)
+{
+    const int64_t wgs = strip_tiles(nx, t.bx, t.sweeps) * strip_tiles(ny, t.by * t.ry, t.sweeps) * ((nz + t.zc - 1) / t.zc);
+    return (double)((wgs + 255) / 256) * t.bx * t.by * t.ry * (t.zc + 2 * t.sweeps);
+}
+
+// The tile for a grid from the times measured on one of its class.
+static bool heat3d_choose(const HeatTimes &from, int64_t nx, int64_t ny, int64_t nz, HeatTile *t)
+{
+    double best = 0;
+    bool any = false;
+    for (const auto &[c, us] : from.tiles) {
+        HeatTile h = c;
+        double v = us;
+        if (c.fused == 3) {
+            if (!strip_tile(c.shape, c.sweeps, c.fill, nx, ny, nz, &h)) continue;
+            v *= strip_cost(h, nx, ny, nz) / strip_cost(c, from.n[0], from.n[1], from.n[2]);
+        } else {
+            h.zc = (int)std::min<int64_t>(c.zc, nz);
+        }
+        if (any && v >= best) continue;
+        any = true;
+        best = v;
+        *t = h;
+    }
+    return any;
+}
 
 int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha, hipStream_t st,
                  bool zero_halo, HeatTile *t)
@@ -1104,14 +1146,7 @@ int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz
     {
         std::lock_guard<std::mutex> g(g_tile_mutex);
         auto it = g_tile_cache.find(key);
-        if (it != g_tile_cache.end() && it->second.fused != 3) {
-            *t = it->second;
-            t->zc = (int)std::min<int64_t>(t->zc, nz);
-            return PAT_OK;
-        }
-        if (it != g_tile_cache.end() &&
-            strip_tile(it->second.shape, it->second.sweeps, it->second.fill, nx, ny, nz, t))
-            return PAT_OK;
+        if (it != g_tile_cache.end() && heat3d_choose(it->second, nx, ny, nz, t)) return PAT_OK;
     }
     if (!zero_halo) {
         t->fused = 0;
@@ -1122,6 +1157,7 @@ int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz
     }
     if (!pat::tuning_enabled()) return PAT_OK;
     std::vector<HeatTile> cands;
+    std::vector<std::pair<HeatTile, size_t>> same;  // tiles that are a candidate on this grid, though not on others
     if (!zero_halo) {
         for (const auto &sh : kShapes)
             for (int z : {2, 4, 8, 16, 32, 64})
@@ -1135,8 +1171,9 @@ int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz
                 HeatTile h;
                 if (!strip_tile(c, sweeps, fill, nx, ny, nz, &h)) continue;
                 if (!cands.empty() && cands.back().shape == c && cands.back().sweeps == sweeps && cands.back().zc == h.zc)
-                    continue;
-                cands.push_back(h);
+                    same.emplace_back(h, cands.size() - 1);
+                else
+                    cands.push_back(h);
             }
     pat::EventPair ev;
     PAT_HIP(ev.create());
@@ -1227,8 +1264,11 @@ int heat3d_tuned(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz
                     cands[c].ry, cands[c].zc, heat3d_steps_per_launch(cands[c]), 1000.0f * tm[c],
                     c == bi ? "  <- chosen" : "");
     *t = cands[bi];
+    HeatTimes times{{nx, ny, nz}, {}};
+    for (size_t c = 0; c < cands.size(); c++) times.tiles.emplace_back(cands[c], tm[c]);
+    for (const auto &e : same) times.tiles.emplace_back(e.first, tm[e.second]);
     std::lock_guard<std::mutex> g(g_tile_mutex);
-    g_tile_cache[key] = *t;
+    g_tile_cache[key] = std::move(times);
     return PAT_OK;
 }
 

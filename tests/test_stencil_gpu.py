@@ -234,3 +234,27 @@ def test_halo_values_are_kept(pa, orc, gpu, shape, variant):
     inside = (slice(1, -1),) * 3
     assert np.array_equal(s.download()[inside], orc.heat3d(fixed, 1)[inside])
     s.close()
+
+
+def test_tuned_tile_of_the_next_grid(pa, gpu):
+    """Grids that share a size class with one tuned before take a tile that
+    fits them: none is slower than the two-sweep window of 64 x 16 cells (the
+    tile they had before the strips), by the best of several runs in turn."""
+    steps = 60
+
+    def handle(n, variant=None):
+        s = pa.Stencil(*n)
+        if variant:
+            s.set_variant(*variant)
+        s.upload(pa.gen_heat3d(*n, seed=2))
+        s.run(steps)
+        return s
+
+    handle((128, 128, 128)).close()  # tunes the class
+    for n in ((129, 129, 129), (160, 160, 160), (176, 176, 176), (130, 170, 150), (148, 180, 133)):
+        a, b = handle(n), handle(n, (pa.PAT_STENCIL_TEMPORAL2, 64, 16, 4))
+        ta, tb = (min(s.run_graph_timed(steps) for _ in range(8)) for s in (a, b))
+        tile = a.tile()
+        a.close()
+        b.close()
+        assert ta <= tb, (n, tile, ta, tb)
