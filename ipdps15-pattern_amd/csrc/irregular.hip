@@ -457,22 +457,23 @@ __global__ __launch_bounds__(kCsrThreads) void csr_rows(const V *__restrict__ en
     auto row_of = [&](V v) { return (int)((unsigned long long)v >> kb); };
     auto key_of = [&](V v) { return (unsigned)v & mask; };
     // entries of rows [w, w + n) of the bucket, four in flight per thread
+    // (unsigned places: a list may have 2^31 - 2 entries)
     auto entries = [&](int w, int n, auto f) {
-        int i = s + t;
-        for (; i + 3 * kCsrThreads < e; i += 4 * kCsrThreads) {
+        unsigned i = (unsigned)s + t;
+        for (; i + 3 * kCsrThreads < (unsigned)e; i += 4 * kCsrThreads) {
             V v[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) v[u] = ent[i + u * kCsrThreads];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const int r = row_of(v[u]) - w;
-                if (r >= 0 && r < n) f(r, key_of(v[u]), i + u * kCsrThreads);
+                if (r >= 0 && r < n) f(r, key_of(v[u]), (int)(i + u * kCsrThreads));
             }
         }
-        for (; i < e; i += kCsrThreads) {
+        for (; i < (unsigned)e; i += kCsrThreads) {
             const V v = ent[i];
             const int r = row_of(v) - w;
-            if (r >= 0 && r < n) f(r, key_of(v), i);
+            if (r >= 0 && r < n) f(r, key_of(v), (int)i);
         }
     };
     int base = s;  // place of the window's first entry

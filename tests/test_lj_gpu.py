@@ -139,6 +139,41 @@ def test_csr_build_long_lists(pa, gpu, n, e, order):
     assert np.array_equal(cols.numpy(), col[by])
 
 
+def test_csr_build_longest_list(pa, gpu):
+    """2^30 - 1 edges, the longest list accepted: places up to 2^31 - 3.  32
+    copies of a list in which row r meets p(r) and p's inverse of r, short of
+    its very last edge; the last rows are compared."""
+    n, e = 1 << 25, (1 << 30) - 1
+    r = np.arange(n, dtype=np.int64)
+    p = (r * 5242881 + 12345) % n  # odd factor: a permutation; odd offset: no row meets itself
+    base = np.stack([r, p], 1).astype(np.int32)
+    edges = pa.DeviceArray((1 << 30, 2), np.int32)
+    pa.call("pat_memcpy_h2d", edges.ptr, base.ctypes.data, base.nbytes, None)
+    have = base.nbytes
+    while have < edges.nbytes:
+        pa.call("pat_memcpy_d2d", edges.ptr + have, edges.ptr, have, None)
+        have *= 2
+    rowptr, cols = pa.csr_build_dev(edges, e, n, order=pa.PAT_IR_ORDER_NODE)
+    inv = np.empty(n, np.int64)
+    inv[p] = r
+    count = np.full(n, 64)
+    count[[n - 1, p[n - 1]]] -= 1
+    expect = np.concatenate([[0], np.cumsum(count)])
+    assert np.array_equal(rowptr.numpy(), expect)
+    rows = 4096
+    tail = np.empty(int(expect[-1] - expect[n - rows]), np.int32)
+    pa.call("pat_memcpy_d2h", tail.ctypes.data, cols.ptr + 4 * int(expect[n - rows]), tail.nbytes, None)
+    want = []
+    for x in range(n - rows, n):
+        row = np.sort(np.repeat([p[x], inv[x]], 32))
+        if x == n - 1:
+            row = np.delete(row, np.flatnonzero(row == p[x])[0])
+        elif x == p[n - 1]:
+            row = np.delete(row, np.flatnonzero(row == n - 1)[0])
+        want.append(row)
+    assert np.array_equal(tail, np.concatenate(want))
+
+
 @pytest.mark.parametrize("lpr", [1, 4, 8, 16, 32, -4, -8, -16, -32, -64])
 def test_force_csr_vs_oracle(pa, orc, gpu, small, lpr):
     pos, box, edges = small
