@@ -11,6 +11,8 @@ another order and are held to 1e-5 relative L-infinity (max |a-b| / max |b|)
 per force evaluation.  The CSR must equal a NumPy construction exactly.
 Errors against the FP64 oracle are printed.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -102,6 +104,18 @@ def csr_list(kind):
         e = [np.stack([np.full(11000, 5), rng.integers(6, 600, 11000)], 1)]
         e += [np.stack([np.full(3000, r), rng.integers(100, 600, 3000)], 1) for r in (6, 7, 8, 20, 21)]
         return 600, np.concatenate(e)
+    if kind == "three nodes of many":  # every entry in one bucket, rows far beyond LDS
+        return 100000, rng.integers(70001, 70004, (300000, 2))
+    if kind == "one neighbour":  # a key met more often than LDS holds, and rows around it
+        e = [np.tile([[5, 7]], (25000, 1)), np.stack([np.full(9000, 5), rng.integers(8, 600, 9000)], 1)]
+        return 600, np.concatenate(e + [rng.integers(0, 600, (20000, 2))])
+    if kind == "clustered keys":  # a long row with most of its neighbours in one of its key ranges
+        far = np.stack([np.full(3000, 5), rng.integers(0, 1 << 20, 3000)], 1)
+        near = np.stack([np.full(40000, 5), rng.integers(700000, 700300, 40000)], 1)
+        return 1 << 20, np.concatenate([near, far])
+    if kind == "heavy windows":  # one bucket with more rows than LDS counts and more entries than it holds
+        n = 8192 * 2048 + 77
+        return n, rng.integers(4096 * 900 + 1500, 4096 * 900 + 2700, (200000, 2))
     if kind == "dense":  # duplicates, buckets of one row
         return 40, rng.integers(0, 40, (60000, 2))
     return 30011, rng.integers(0, 30011, (400000, 2))  # ragged: B, chunks and rows with remainders
@@ -109,7 +123,8 @@ def csr_list(kind):
 
 @pytest.mark.parametrize("order", [0, 1])
 @pytest.mark.parametrize("kind", ["two nodes", "one edge, many nodes", "rows in windows", "short and long rows", "hubs",
-                                  "dense", "ragged"])
+                                  "three nodes of many", "one neighbour", "clustered keys", "heavy windows", "dense",
+                                  "ragged"])
 def test_csr_build_forms(pa, gpu, kind, order):
     n, edges = csr_list(kind)
     edges = edges[edges[:, 0] != edges[:, 1]]
@@ -137,6 +152,29 @@ def test_csr_build_long_lists(pa, gpu, n, e, order):
     by = np.argsort(row << 32 | key, kind="stable")
     assert np.array_equal(rowptr.numpy(), np.concatenate([[0], np.cumsum(np.bincount(row, minlength=n))]))
     assert np.array_equal(cols.numpy(), col[by])
+
+
+@pytest.mark.parametrize("order", [0, 1])
+def test_csr_build_skewed_list_time(pa, gpu, order):
+    """A list whose edges touch 1% of the nodes has its entries in few buckets;
+    the build spreads them over the chip all the same (10 times the time of a
+    list among all nodes allowed, about 4 measured; one workgroup a bucket: 33)."""
+    n, e = 100000, 1000000
+    wb = pa.c_i64(0)
+    pa.call("pat_ir_csr_workspace", n, e, pa.ctypes.byref(wb))
+    work, rowptr, cols = (pa.DeviceArray((m,), t) for m, t in ((wb.value, np.uint8), (n + 1, np.int32), (2 * e, np.int32)))
+    best = []
+    for hot in (n, n // 100):
+        ed = pa.DeviceArray.from_numpy(np.random.default_rng(7).integers(0, hot, (e, 2), dtype=np.int32))
+        times = []
+        for _ in range(6):
+            pa.sync()
+            t0 = time.perf_counter()
+            pa.call("pat_ir_csr_build_dev", ed.ptr, e, n, order, rowptr.ptr, cols.ptr, work.ptr, wb.value, None)
+            pa.sync()
+            times.append(time.perf_counter() - t0)
+        best.append(min(times))
+    assert best[1] <= 10 * best[0], best
 
 
 def test_csr_build_longest_list(pa, gpu):
