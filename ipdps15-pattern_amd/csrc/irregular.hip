@@ -277,7 +277,8 @@ enum CsrOut { kCsrEdgeOrder = 0, kCsrNodeOrder = 1, kCsrEdgeIds = 2 };
 constexpr int kCsrThreads = 512;
 constexpr int kCsrMaxBuckets = 8192;   // counted in LDS: 32 KB
 constexpr int kCsrStageThreads = 1024;
-constexpr int kCsrStageEdges = 13 * kCsrStageThreads;  // csr_scatter_runs: 104 KB of entries
+constexpr int kCsrStageMost = 15;      // edges per thread of csr_scatter_runs: 120 KB of entries, the most beside its counts
+constexpr int kCsrCus = 256;
 constexpr int kCsrCap = 10240;         // entries of a group of rows held in LDS (40 KB)
 constexpr int kCsrRows = 2048;         // rows, or ranges of keys, counted in LDS at a time (8 KB): three workgroups per CU
 
@@ -381,15 +382,16 @@ __global__ __launch_bounds__(kCsrThreads) void csr_scatter(const int2 *__restric
 // whole runs: 16 lanes write a bucket's run.  13.3 M entries in 2,000 buckets:
 // 51 us, 130 with csr_scatter, whose stores of single 8-byte words L2 takes one
 // by one.  The edges and their places within the bucket stay in registers
-// between the passes.
+// between the passes.  PER: edges per thread (chunk <= 1,024 PER).
+template <int PER>
 __global__ __launch_bounds__(kCsrStageThreads) void csr_scatter_runs(const int2 *__restrict__ edges, int64_t E,
                                                                      int64_t chunk, int shift, int B,
                                                                      const int *__restrict__ start,
                                                                      const int *__restrict__ part, int node_order,
                                                                      unsigned *__restrict__ ent)
 {
-    constexpr int PER = kCsrStageEdges / kCsrStageThreads, T = kCsrStageThreads;
-    __shared__ unsigned buf[2 * kCsrStageEdges];
+    constexpr int T = kCsrStageThreads;
+    __shared__ unsigned buf[2 * PER * T];
     __shared__ int h[kCsrMaxBuckets + 1];
     __shared__ int wsum[T / kWave];
     const int t = (int)threadIdx.x, lane = t % kWave, wv = pat::wave_in_block();
@@ -444,6 +446,18 @@ __global__ __launch_bounds__(kCsrStageThreads) void csr_scatter_runs(const int2 
         const int g = start[b] + part[(int64_t)blockIdx.x * B + b];
         for (int i = t % 16; i < m; i += 16) ent[g + i] = buf[s + i];
     }
+}
+
+using CsrRunsKernel = void (*)(const int2 *, int64_t, int64_t, int, int, const int *, const int *, int, unsigned *);
+
+// csr_scatter_runs for so many edges per thread (2 to kCsrStageMost).
+template <int PER = 2>
+static CsrRunsKernel csr_runs_kernel(int per)
+{
+    if constexpr (PER < kCsrStageMost) {
+        if (per > PER) return csr_runs_kernel<PER + 1>(per);
+    }
+    return csr_scatter_runs<PER>;
 }
 
 // a[0..kCsrRows) = base + their exclusive sums; returns base + their sum.
@@ -2260,15 +2274,19 @@ static int csr_buckets(const char *who, const int32_t *edges, int64_t E, int64_t
     // neighbour, or twice the edge (csr_scatter_runs)
     const int kb = 32 - shift;
     const bool fits = (out == kCsrNodeOrder ? N : 2 * E) <= 1LL << kb;
-    // Edges per workgroup: enough for runs of several entries per bucket, and
-    // about 400 workgroups where the list is that long (or two for each CU, one
-    // at a time, with the entries in LDS).  The totals (B) and
+    // Edges per workgroup: with the entries in LDS, so many that the workgroups
+    // make whole rounds of one on every CU (where LDS holds one), two or as many
+    // as it takes (265,837 nodes, 6.91 M edges: 164 us; with a last round of
+    // eight workgroups 181); else for about 400 workgroups.  At least 2,048,
+    // for runs of several entries per bucket.  The totals (B) and
     // the workgroups' parts (wgs x B) lie behind the starts (B + 1) where the
     // N + 1 words hold them, else in cols (2 E words) until csr_rows writes
     // it; one of the two holds them at the latest with one workgroup, since
     // buckets of fewer than four rows mean over 64 entries per row.
-    int64_t chunk = fits ? std::max<int64_t>(2048, std::min<int64_t>(kCsrStageEdges, (E + 511) / 512))
-                         : std::max<int64_t>(2048, std::min<int64_t>(16384, (E + 399) / 400));
+    const int64_t most = kCsrStageMost * kCsrStageThreads;
+    const int64_t rounds = std::max<int64_t>(2, (E + kCsrCus * most - 1) / (kCsrCus * most));
+    int64_t chunk = std::max<int64_t>(2048, fits ? (E + rounds * kCsrCus - 1) / (rounds * kCsrCus)
+                                                 : std::min<int64_t>(16384, (E + 399) / 400));
     int64_t wgs = (E + chunk - 1) / chunk;
     auto beside = [&] { return (wgs + 2) * B <= N; };
     while (wgs > 1 && !beside() && (wgs + 1) * B > 2 * E) {
@@ -2281,7 +2299,7 @@ static int csr_buckets(const char *who, const int32_t *edges, int64_t E, int64_t
     // the entries: 2 E words of 4 or 8 bytes behind the N + 1 words (rounded
     // up to 16 bytes within the work space's 256 spare ones)
     void *ent = (void *)(((uintptr_t)work + sizeof(int) * (size_t)(N + 1) + 15) & ~(uintptr_t)15);
-    const bool runs = fits && chunk <= kCsrStageEdges;
+    const bool runs = fits && chunk <= most;
     const int2 *e2 = (const int2 *)edges;
     hipLaunchKernelGGL(fill_i32, dim3(grid_for(B)), dim3(256), 0, st, total, (int64_t)B, 0);
     PAT_LAUNCH_CHECK();
@@ -2291,8 +2309,9 @@ static int csr_buckets(const char *who, const int32_t *edges, int64_t E, int64_t
                        heavy);
     PAT_LAUNCH_CHECK();
     if (runs)
-        hipLaunchKernelGGL(csr_scatter_runs, dim3((unsigned)wgs), dim3(kCsrStageThreads), 0, st, e2, E, chunk, shift, B,
-                           (const int *)start, (const int *)part, out == kCsrNodeOrder, (unsigned *)ent);
+        hipLaunchKernelGGL(csr_runs_kernel((int)((chunk + kCsrStageThreads - 1) / kCsrStageThreads)), dim3((unsigned)wgs),
+                           dim3(kCsrStageThreads), 0, st, e2, E, chunk, shift, B, (const int *)start, (const int *)part,
+                           (int)(out == kCsrNodeOrder), (unsigned *)ent);
     else
         hipLaunchKernelGGL(csr_scatter, dim3((unsigned)wgs), dim3(kCsrThreads), 0, st, e2, E, chunk, shift, B,
                            (const int *)start, (const int *)part, out == kCsrNodeOrder, (unsigned long long *)ent);
