@@ -308,6 +308,10 @@ __global__ __launch_bounds__(BS) void km_plain(KmArgs a, int centres_in_lds)
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2;
 
+// Fragments of a centre's row (16 elements each): three terms take high and low
+// parts, one term one; and the norm.
+constexpr int mfma_fragments(int ks, int nt) { return (nt == 3 ? 2 : 1) * ks + 1; }
+
 constexpr float kWideOne = 32768.0f;  // the norm parts' factor 2^15
 constexpr float kWideFar = 60000.0f;  // first norm part of a row that never wins: above any value (2^28)
 
@@ -490,7 +494,7 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const void *__restrict__
 {
     constexpr bool F16 = NT == 3;
     constexpr int NS = NT * KS + 1;               // MFMAs per block of 32 centres
-    constexpr int NF = F16 ? 2 * KS + 1 : NS;     // fragments per block in cb (1 KiB each)
+    constexpr int NF = mfma_fragments(KS, NT);    // fragments per block in cb (1 KiB each)
     static_assert(KB * 16 <= 128, "pack_key indexes at most 128 values per chunk");
     extern __shared__ unsigned long long smem[];
     unsigned long long *acc_o, *cnt_o, *dsum_o;
@@ -1887,8 +1891,8 @@ int kmeans_assign_plain(const KmDev &d, hipStream_t st)
     return d.bucketed ? bucket_reduce(d, st) : PAT_OK;
 }
 
-// LDS bytes of the MFMA kernel with nt terms (staged BF16 rows plus the
-// reduction object when it is kept in LDS).
+// LDS bytes of the MFMA kernel with nt terms (staged rows plus the reduction
+// object when it is kept in LDS).
 static int64_t mfma_lds_bytes(int K, int D, int nt, bool gc = false)
 {
     const int ks = kmeans_ks_for(D);
@@ -1896,14 +1900,14 @@ static int64_t mfma_lds_bytes(int K, int D, int nt, bool gc = false)
     // all rows, or (gc) one chunk: KB blocks of 32 rows (KB = 8, 8, 4, 2 for
     // KS = 1, 2, 4, 8)
     const int kb = kmeans_kb_for(ks);
-    const int64_t cbb = gc ? 2LL * std::min(K_pad, 32 * kb) * 16 * (nt * ks + 1) : 2LL * K_pad * 16 * (nt * ks + 1);
+    const int64_t cbb = 2LL * (gc ? std::min(K_pad, 32 * kb) : K_pad) * 16 * mfma_fragments(ks, nt);
     const int64_t obj = object_bytes(K, D) <= std::min<int64_t>(96 * 1024, g_lds_limit - 32 * 1024)
                             ? object_bytes(K, D) : 0;
     return cbb + obj;
 }
 
-// Terms of the MFMA path for this shape: 3 (split BF16) when its rows fit in
-// LDS, else 1, 0 when neither fits.
+// Terms of the MFMA path for this shape: 3 (FP16 high and low parts) when its
+// rows fit in LDS, else 1 (BF16), 0 when neither fits.
 int kmeans_nt_for(int K, int D)
 {
     if (!kmeans_ks_for(D)) return 0;
@@ -1919,7 +1923,7 @@ bool kmeans_gc_for(int K, int D) { return kmeans_ks_for(D) != 0 && kmeans_nt_for
 bool kmeans_mfma_fits(int K, int D) { return kmeans_ks_for(D) != 0 && K <= 65536; }
 
 // Words (FP16) of the wide path's rows.
-int64_t kmeans_wide_row_words(int K_pad, int D) { return (int64_t)K_pad * 16 * (2 * kmeans_ks_for(D) + 1); }
+int64_t kmeans_wide_row_words(int K_pad, int D) { return (int64_t)K_pad * 16 * mfma_fragments(kmeans_ks_for(D), 3); }
 
 // Exponent a of the wide path's scale: 2^a times the largest coordinate lies
 // below 2^10 (2^126 is the largest FP32 power of two with an FP32 inverse).

@@ -12,7 +12,7 @@ struct KmDev {
     float *c;        // K x D centres (FP32)
     int64_t N;
     int D, K, K_pad, KS;  // K_pad: K rounded up to 32; KS: 16-wide K-steps of the data
-    int NT;               // MFMA data terms: 3 (split BF16), 1 (BF16), 0 (no MFMA path)
+    int NT;               // MFMA data terms: 3 (FP16 high and low parts), 1 (BF16), 0 (no MFMA path)
     int wide;             // FP16 rows and km_wide instead of the NT forms (bucketed handles)
     int wexp;             // its scale 2^wexp
     int gc;               // MFMA rows read from global memory (K x D too large for LDS)
@@ -21,7 +21,7 @@ struct KmDev {
     float *mindist;       // N
     unsigned long long *gsum, *gcnt, *gdsum;  // reduction object (K x D, K, K)
     unsigned long long *snap;                 // last pass's reduction object (K x D + 2 K)
-    void *cb;             // MFMA rows: BF16, K_pad x 16*(NT*KS+1), or FP16, K_pad x 16*(2*KS+1) (wide)
+    void *cb;             // MFMA rows: FP16, K_pad x 16*(2*KS+1) (wide, three terms), or BF16, K_pad x 16*(KS+1)
     float *cnorm;         // ||c_k|| (rounded up)
     unsigned long long *rescored;  // points with more than one candidate
     int cus;              // compute units

@@ -271,7 +271,8 @@ def test_wide_path_two_tiles(pa, orc, gpu):
 
 @pytest.mark.parametrize("n,d,k", [(31, 3, 1), (700, 8, 31), (1000, 8, 33), (3000, 16, 512), (3000, 16, 513),
                                    (2500, 13, 257), (4000, 32, 255), (4000, 31, 64), (3000, 64, 129), (3000, 50, 70),
-                                   (2000, 128, 60), (2000, 99, 40)])
+                                   (2000, 128, 60), (2000, 99, 40), (2000, 8, 800), (2000, 16, 640), (2000, 32, 350),
+                                   (2000, 64, 170), (2000, 128, 90)])
 @pytest.mark.parametrize("terms", [1, 3])
 def test_pair_keys_bitexact(pa, orc, gpu, n, d, k, terms):
     """Objects in LDS: keys of pairs of adjacent centres up to 512 centres and
@@ -281,8 +282,7 @@ def test_pair_keys_bitexact(pa, orc, gpu, n, d, k, terms):
     some far outside the points' range and one that is not finite."""
     x = pa.gen_gmm(n, d, max(1, k // 2), sigma=1.0, seed=n + d + k)
     km = pa.KMeans(x, k, mode=1)
-    if terms == 3 and km.terms() != 3:
-        pytest.skip("three terms do not fit")
+    assert km.terms() == 3  # both forms' rows fit in LDS beside the object for all of these
     km.set_terms(terms)
     km.run(2)
     c, a, md = km.get()
