@@ -435,11 +435,11 @@ __device__ __forceinline__ int key_mask()
 
 // base | i for a wavefront-uniform base, in one scalar register (a scalar
 // ALU operation, opaque to the compiler, which would otherwise fold the OR
-// into the packing as a second vector instruction).
+// into the packing as a second vector instruction).  It sets SCC.
 __device__ __forceinline__ int scalar_or(int base, int i)
 {
     int r;
-    asm("s_or_b32 %0, %1, %2" : "=s"(r) : "s"(base), "s"(i));
+    asm("s_or_b32 %0, %1, %2" : "=s"(r) : "s"(base), "s"(i) : "scc");
     return r;
 }
 
@@ -1900,7 +1900,7 @@ static int64_t mfma_lds_bytes(int K, int D, int nt, bool gc = false)
     // all rows, or (gc) one chunk: KB blocks of 32 rows (KB = 8, 8, 4, 2 for
     // KS = 1, 2, 4, 8)
     const int kb = kmeans_kb_for(ks);
-    const int64_t cbb = 2LL * (gc ? std::min(K_pad, 32 * kb) : K_pad) * 16 * mfma_fragments(ks, nt);
+    const int64_t cbb = 2LL * (gc ? 32 * kb : K_pad) * 16 * mfma_fragments(ks, nt);
     const int64_t obj = object_bytes(K, D) <= std::min<int64_t>(96 * 1024, g_lds_limit - 32 * 1024)
                             ? object_bytes(K, D) : 0;
     return cbb + obj;

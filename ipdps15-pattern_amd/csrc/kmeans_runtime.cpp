@@ -277,6 +277,23 @@ int pat_kmeans_set_terms(pat_kmeans *h, int terms)
     return PAT_OK;
 }
 
+// The handle's passes by the form of 2^31 and more points (rows staged chunk
+// by chunk, sums added directly), for the tests; not part of the public
+// interface.
+int pat_internal_kmeans_staged_rows(pat_kmeans *h)
+{
+    PAT_REQUIRE(h && h->d.KS, PAT_ERR_INVALID, "kmeans staged rows: no handle, or D too large");
+    auto &D = h->d;
+    D.NT = 3;
+    D.gc = 1;
+    D.wide = 0;
+    D.bucketed = 0;
+    h->drop_graphs();
+    PAT_TRY(pat::kmeans_finalize(D, 0, h->stream));
+    PAT_HIP(hipStreamSynchronize(h->stream));
+    return PAT_OK;
+}
+
 int pat_kmeans_get_terms(pat_kmeans *h, int *terms)
 {
     PAT_REQUIRE(h && terms, PAT_ERR_INVALID, "pat_kmeans_get_terms: null argument");

@@ -307,3 +307,39 @@ def test_pair_keys_bitexact(pa, orc, gpu, n, d, k, terms):
     km.close()
     ra, rmd = orc.kmeans_assign(x, odd)
     assert np.array_equal(a, ra) and np.array_equal(md, rmd)
+
+
+@pytest.mark.parametrize("n,d,k", [(1000, 16, 40), (3000, 16, 1500), (2000, 13, 700), (2000, 32, 33), (3000, 32, 385),
+                                   (3000, 29, 500), (2000, 64, 130), (2500, 64, 300), (2000, 47, 257), (700, 128, 60),
+                                   (2000, 128, 289), (2000, 100, 97), (1500, 5, 1200)])
+def test_staged_rows_bitexact(pa, orc, gpu, n, d, k):
+    """The form that handles of 2^31 and more points take when the object does
+    not fit in LDS, forced on small ones: every row width with and without a
+    tail, objects in and beyond LDS, partial chunks; then centres that repeat
+    across a block's halves, blocks and chunks, some far outside the points'
+    range and one that is not finite."""
+    x = pa.gen_gmm(n, d, max(1, k // 2), sigma=1.0, seed=n + d + k)
+    km = pa.KMeans(x, k, mode=1)
+    staged = pa.lib().pat_internal_kmeans_staged_rows
+    staged.argtypes = [pa.c_vp]
+    assert staged(km.h) == 0
+    km.run(2)
+    c, a, md = km.get()
+    sums, counts, dsums, s, ds = km.get_object()
+    *_, (c1, ra, rmd, rsums, rcounts, rdsum) = oracle_iters(orc, pa, x, k, 2)
+    assert np.array_equal(a, ra) and np.array_equal(md, rmd)
+    assert np.array_equal(sums, rsums) and np.array_equal(counts, rcounts) and np.array_equal(dsums, rdsum)
+    assert np.array_equal(c, orc.kmeans_update(rsums, rcounts, s, c1))
+    odd = x[:k].copy()
+    for i, j in ((0, 1), (2, 6), (3, 4), (5, 37), (8, 9), (10, 14), (11, 12), (13, 140), (7, 290)):
+        if j < k:
+            odd[j] = odd[i]
+    odd[20] *= 1024.0
+    odd[21] = -odd[20]
+    odd[22, 0] = np.nan
+    km.set_centroids(odd)
+    km.run(1)
+    _, a, md = km.get()
+    ra, rmd = orc.kmeans_assign(x, odd)
+    assert np.array_equal(a, ra) and np.array_equal(md, rmd)
+    km.close()
