@@ -37,6 +37,8 @@
 // steps against rows in global memory (km_wide).
 #include <algorithm>
 #include <cmath>
+#include <iterator>
+#include <vector>
 
 #include "pat_common.hpp"
 #include "pat_device.hpp"
@@ -1733,6 +1735,60 @@ static KmArgs make_args(const KmDev &d)
 }
 
 
+// The MFMA forms that kmeans_assign_mfma chooses from.  One block of centres per
+// chunk for three terms with the rows in LDS, at three wavefronts per SIMD; but
+// at 64 dimensions a full row stays in registers for the exact distances, at
+// two (1 M x 64, K 150: 142 us a pass, 196 with three and the row read again),
+// while a row with a tail is read again in any case (1 M x 50, K 100: 131 us
+// with three, 148 with two).
+using MfmaKernel = void (*)(KmArgs, const void *, const float *, int, MfmaBound, WideBound, unsigned long long *);
+struct MfmaForm {
+    int ks, nt;
+    bool tail, gc;
+    int threads;
+    MfmaKernel kernel;
+};
+template <int KS, int KB, int NT, bool TAIL, bool GC, int BS>
+constexpr MfmaForm mfma_form()
+{
+    return {KS, NT, TAIL, GC, BS, km_mfma<KS, KB, NT, TAIL, GC, BS>};
+}
+static const MfmaForm kMfmaForms[] = {
+    // one term
+    mfma_form<1, 8, 1, true, false, 512>(), mfma_form<1, 8, 1, false, false, 512>(),
+    mfma_form<2, 8, 1, true, false, 512>(), mfma_form<2, 8, 1, false, false, 512>(),
+    mfma_form<4, 4, 1, true, false, 512>(), mfma_form<4, 4, 1, false, false, 512>(),
+    mfma_form<8, 2, 1, true, false, 512>(), mfma_form<8, 2, 1, false, false, 512>(),
+    // three terms, rows in LDS
+    mfma_form<1, 1, 3, true, false, 768>(), mfma_form<1, 1, 3, false, false, 768>(),
+    mfma_form<2, 1, 3, true, false, 768>(), mfma_form<2, 1, 3, false, false, 768>(),
+    mfma_form<4, 1, 3, true, false, 768>(), mfma_form<4, 1, 3, false, false, 512>(),
+    mfma_form<8, 1, 3, true, false, 512>(), mfma_form<8, 1, 3, false, false, 512>(),
+    // three terms, rows staged chunk by chunk (kmeans_kb_for)
+    mfma_form<1, 8, 3, true, true, 512>(), mfma_form<1, 8, 3, false, true, 512>(),
+    mfma_form<2, 8, 3, true, true, 512>(), mfma_form<2, 8, 3, false, true, 512>(),
+    mfma_form<4, 4, 3, true, true, 512>(), mfma_form<4, 4, 3, false, true, 512>(),
+    mfma_form<8, 2, 3, true, true, 512>(), mfma_form<8, 2, 3, false, true, 512>()};
+
+// Those of assign_wide: NB blocks of 32 centres per LDS chunk (two chunks of up
+// to 72 KiB).
+using WideKernel = void (*)(KmArgs, const _Float16 *, const float *, int, WideBound, int *, int *, unsigned long long *);
+struct WideForm {
+    int ks, nb, tiles;
+    bool tail;
+    WideKernel kernel;
+};
+template <int KS, int NB, int TILES, bool TAIL>
+constexpr WideForm wide_form()
+{
+    return {KS, NB, TILES, TAIL, km_wide<KS, NB, TILES, TAIL>};
+}
+static const WideForm kWideForms[] = {
+    wide_form<1, 8, 1, true>(), wide_form<1, 8, 1, false>(), wide_form<1, 8, 2, true>(), wide_form<1, 8, 2, false>(),
+    wide_form<2, 8, 1, true>(), wide_form<2, 8, 1, false>(), wide_form<2, 8, 2, true>(), wide_form<2, 8, 2, false>(),
+    wide_form<4, 8, 1, true>(), wide_form<4, 8, 1, false>(), wide_form<4, 8, 2, true>(), wide_form<4, 8, 2, false>(),
+    wide_form<8, 4, 1, true>(), wide_form<8, 4, 1, false>(), wide_form<8, 4, 2, true>(), wide_form<8, 4, 2, false>()};
+
 // Raises every kmeans kernel's dynamic-LDS limit to what the device allows
 // per workgroup (160 KB on gfx950).  Best effort: the per-block limit the
 // device reports is what the launch checks use.  Called once before any
@@ -1745,31 +1801,11 @@ int kmeans_prepare_kernels()
     PAT_HIP(hipGetDevice(&dev));
     PAT_HIP(hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     g_lds_limit = lim - 256;  // room for the kernels' static LDS
-    const void *fns[] = {
-        (const void *)km_plain<8, 1024>, (const void *)km_plain<16, 1024>, (const void *)km_plain<32, 1024>,
-        (const void *)km_plain<64, 1024>, (const void *)km_plain<128, 512>,
-        // one term
-        (const void *)km_mfma<1, 8, 1, true, false>, (const void *)km_mfma<2, 8, 1, true, false>,
-        (const void *)km_mfma<4, 4, 1, true, false>, (const void *)km_mfma<8, 2, 1, true, false>,
-        (const void *)km_mfma<1, 8, 1, false, false>, (const void *)km_mfma<2, 8, 1, false, false>,
-        (const void *)km_mfma<4, 4, 1, false, false>, (const void *)km_mfma<8, 2, 1, false, false>,
-        // three terms, rows in LDS
-        (const void *)km_mfma<1, 4, 3, true, false, 768>, (const void *)km_mfma<1, 4, 3, false, false, 768>,
-        (const void *)km_mfma<2, 1, 3, true, false, 768>, (const void *)km_mfma<2, 1, 3, false, false, 768>,
-        (const void *)km_mfma<4, 2, 3, true, false, 768>, (const void *)km_mfma<4, 2, 3, false, false, 768>,
-        (const void *)km_mfma<8, 2, 3, true, false>, (const void *)km_mfma<8, 2, 3, false, false>,
-        // three terms, rows staged chunk by chunk
-        (const void *)km_mfma<1, 8, 3, true, true>, (const void *)km_mfma<2, 8, 3, true, true>,
-        (const void *)km_mfma<4, 4, 3, true, true>, (const void *)km_mfma<8, 2, 3, true, true>,
-        (const void *)km_mfma<1, 8, 3, false, true>, (const void *)km_mfma<2, 8, 3, false, true>,
-        (const void *)km_mfma<4, 4, 3, false, true>, (const void *)km_mfma<8, 2, 3, false, true>,
-        // FP16 high and low parts, for objects beyond LDS
-        (const void *)km_wide<1, 8, 1, true>, (const void *)km_wide<2, 8, 1, true>, (const void *)km_wide<4, 8, 1, true>,
-        (const void *)km_wide<8, 4, 1, true>, (const void *)km_wide<1, 8, 1, false>, (const void *)km_wide<2, 8, 1, false>,
-        (const void *)km_wide<4, 8, 1, false>, (const void *)km_wide<8, 4, 1, false>, (const void *)km_wide<1, 8, 2, true>,
-        (const void *)km_wide<2, 8, 2, true>, (const void *)km_wide<4, 8, 2, true>, (const void *)km_wide<8, 4, 2, true>,
-        (const void *)km_wide<1, 8, 2, false>, (const void *)km_wide<2, 8, 2, false>, (const void *)km_wide<4, 8, 2, false>,
-        (const void *)km_wide<8, 4, 2, false>};
+    std::vector<const void *> fns = {(const void *)km_plain<8, 1024>, (const void *)km_plain<16, 1024>,
+                                     (const void *)km_plain<32, 1024>, (const void *)km_plain<64, 1024>,
+                                     (const void *)km_plain<128, 512>};
+    for (const MfmaForm &f : kMfmaForms) fns.push_back((const void *)f.kernel);
+    for (const WideForm &f : kWideForms) fns.push_back((const void *)f.kernel);
     for (const void *f : fns)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g_lds_limit) != hipSuccess)
             (void)hipGetLastError();
@@ -1828,7 +1864,7 @@ static int bucket_reduce(const KmDev &d, hipStream_t st)
     return PAT_OK;
 }
 
-static int allow_lds(const void *, int64_t bytes)
+static int check_lds(int64_t bytes)
 {
     PAT_REQUIRE(bytes <= g_lds_limit, PAT_ERR_UNSUPPORTED, "kmeans: %lld bytes of LDS requested, device allows %lld",
                 (long long)bytes, (long long)g_lds_limit);
@@ -1874,7 +1910,7 @@ int kmeans_assign_plain(const KmDev &d, hipStream_t st)
 #define PAT_KP(DM)                                                                                                     \
     do {                                                                                                               \
         constexpr int bs = DM <= 64 ? 1024 : 512;                                                                      \
-        PAT_TRY(allow_lds((const void *)km_plain<DM, bs>, lds));                                                       \
+        PAT_TRY(check_lds(lds));                                                                                       \
         hipLaunchKernelGGL((km_plain<DM, bs>), dim3(grid), dim3(bs), (size_t)lds, st, a, in_lds);                      \
     } while (0)
     if (d.D <= 8) PAT_KP(8);
@@ -1951,37 +1987,24 @@ static WideBound wide_bound(const KmDev &d)
     return b;
 }
 
-// Blocks of 32 centres per LDS chunk of km_wide: two chunks of up to 72 KiB.
-static int wide_nb(int ks) { return ks == 8 ? 4 : 8; }
-
 static int assign_wide(const KmDev &d, hipStream_t st)
 {
     const KmArgs a = make_args(d);
     const WideBound bd = wide_bound(d);
-    const size_t lds = 2 * (size_t)wide_nb(d.KS) * (2 * d.KS + 1) * 1024;
-    PAT_REQUIRE((int64_t)lds <= g_lds_limit, PAT_ERR_UNSUPPORTED, "kmeans: %zu bytes of LDS requested, device allows %lld",
-                lds, (long long)g_lds_limit);
     // two tiles per wavefront (each centre fragment feeds two MFMAs) where
     // that leaves every CU a workgroup, else one
     const bool two = d.N >= 512LL * d.cus;
     const int64_t per = two ? 512 : 256;
     const unsigned grid = (unsigned)std::min<int64_t>((d.N + per - 1) / per, d.cus);
     const bool tail = d.D != 16 * d.KS || ((uintptr_t)d.x % 16) != 0;
-#define PAT_KW(KS_, NB_)                                                                                               \
-    do {                                                                                                               \
-        auto k = two ? (tail ? km_wide<KS_, NB_, 2, true> : km_wide<KS_, NB_, 2, false>)                               \
-                     : (tail ? km_wide<KS_, NB_, 1, true> : km_wide<KS_, NB_, 1, false>);                              \
-        hipLaunchKernelGGL(k, dim3(grid), dim3(512), lds, st, a, (const _Float16 *)d.cb, d.cnorm, d.K_pad, bd,        \
-                           d.bidx, d.bcnt + d.K, d.rescored);                                                          \
-    } while (0)
-    switch (d.KS) {
-    case 1: PAT_KW(1, 8); break;
-    case 2: PAT_KW(2, 8); break;
-    case 4: PAT_KW(4, 8); break;
-    case 8: PAT_KW(8, 4); break;
-    default: pat::set_error("kmeans: D too large"); return PAT_ERR_UNSUPPORTED;
-    }
-#undef PAT_KW
+    const WideForm *f = std::find_if(std::begin(kWideForms), std::end(kWideForms), [&](const WideForm &w) {
+        return w.ks == d.KS && w.tiles == (two ? 2 : 1) && w.tail == tail;
+    });
+    PAT_REQUIRE(f != std::end(kWideForms), PAT_ERR_UNSUPPORTED, "kmeans: D too large");
+    const size_t lds = 2 * (size_t)f->nb * (2 * d.KS + 1) * 1024;
+    PAT_TRY(check_lds((int64_t)lds));
+    hipLaunchKernelGGL(f->kernel, dim3(grid), dim3(512), lds, st, a, (const _Float16 *)d.cb, (const float *)d.cnorm,
+                       d.K_pad, bd, d.bidx, d.bcnt + d.K, d.rescored);
     PAT_LAUNCH_CHECK();
     hipLaunchKernelGGL(km_rescore, dim3((unsigned)std::min<int64_t>((d.N + 63) / 64, 4LL * d.cus)), dim3(256), 0, st, a,
                        (const int *)d.bidx, (const int *)(d.bcnt + d.K));
@@ -2009,64 +2032,22 @@ int kmeans_assign_mfma(const KmDev &d, hipStream_t st)
     bd.c_norm = (float)((u * u * u + 2 * g * (1 + 2 * u)) * 1.01);
     bd.c_ref = (float)((3.0 + d.D + 16.0) * ldexp(1.0, -24) * 1.01);
     const WideBound wb = wide_bound(d);
-    // one workgroup per CU (the LDS holds one), BS_ / 64 wavefronts each.  While
+    // no tail: every K-step full and 16-byte aligned rows
+    const bool tail = d.D != 16 * d.KS || ((uintptr_t)d.x % 16) != 0;
+    const MfmaForm *f = std::find_if(std::begin(kMfmaForms), std::end(kMfmaForms), [&](const MfmaForm &m) {
+        return m.ks == d.KS && m.nt == d.NT && m.gc == (d.gc != 0) && m.tail == tail;
+    });
+    PAT_REQUIRE(f != std::end(kMfmaForms), PAT_ERR_UNSUPPORTED, "kmeans: D too large");
+    // one workgroup per CU (the LDS holds one).  While
     // the points do not fill the chip every wavefront takes one tile (rounded
     // down, a few took two, and 10 iterations of 3,000 x 4, K 8 took 165 us, not 137).  Smaller
     // workgroups on more CUs are slower: each stages the rows and flushes its
     // object (10 iterations of 20,000 x 8, K 16: 158 us with 256 threads, 149
     // with 768; of 100,000 x 16, K 32: 275 and 253).
-    auto grid_for = [&](int bs) {
-        const int64_t want = ((d.N + 31) / 32 + bs / 64 - 1) / (bs / 64);
-        return (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)d.cus));
-    };
-    // no tail: every K-step full and 16-byte aligned rows
-    const bool tail = d.D != 16 * d.KS || ((uintptr_t)d.x % 16) != 0;
-#define PAT_KM_BS(KS_, KB_, NT_, GC_, BS_)                                                                             \
-    do {                                                                                                               \
-        if (tail) {                                                                                                    \
-            PAT_TRY(allow_lds((const void *)km_mfma<KS_, KB_, NT_, true, GC_, BS_>, lds));                             \
-            hipLaunchKernelGGL((km_mfma<KS_, KB_, NT_, true, GC_, BS_>), dim3(grid_for(BS_)), dim3(BS_), (size_t)lds,  \
-                               st, a, (const void *)d.cb, d.cnorm, d.K_pad, bd, wb, d.rescored);                       \
-        } else {                                                                                                       \
-            PAT_TRY(allow_lds((const void *)km_mfma<KS_, KB_, NT_, false, GC_, BS_>, lds));                            \
-            hipLaunchKernelGGL((km_mfma<KS_, KB_, NT_, false, GC_, BS_>), dim3(grid_for(BS_)), dim3(BS_), (size_t)lds, \
-                               st, a, (const void *)d.cb, d.cnorm, d.K_pad, bd, wb, d.rescored);                       \
-        }                                                                                                              \
-    } while (0)
-#define PAT_KM_GC(KS_, KB_, NT_, GC_) PAT_KM_BS(KS_, KB_, NT_, GC_, 512)
-#define PAT_KM(KS_, KB_, NT_) PAT_KM_GC(KS_, KB_, NT_, false)
-    if (d.gc) {
-        switch (d.KS) {
-        case 1: PAT_KM_GC(1, 8, 3, true); break;
-        case 2: PAT_KM_GC(2, 8, 3, true); break;
-        case 4: PAT_KM_GC(4, 4, 3, true); break;
-        case 8: PAT_KM_GC(8, 2, 3, true); break;
-        default: pat::set_error("kmeans: D too large"); return PAT_ERR_UNSUPPORTED;
-        }
-        PAT_LAUNCH_CHECK();
-        return d.bucketed ? bucket_reduce(d, st) : PAT_OK;
-    }
-    switch (d.KS * 4 + d.NT) {
-    case 1 * 4 + 1: PAT_KM(1, 8, 1); break;
-    case 2 * 4 + 1: PAT_KM(2, 8, 1); break;
-    case 4 * 4 + 1: PAT_KM(4, 4, 1); break;
-    case 8 * 4 + 1: PAT_KM(8, 2, 1); break;
-    case 1 * 4 + 3: PAT_KM_BS(1, 1, 3, false, 768); break;  // 3 wavefronts per SIMD
-    case 2 * 4 + 3: PAT_KM_BS(2, 1, 3, false, 768); break;  // 3 wavefronts per SIMD
-    case 4 * 4 + 3:
-        // a full row stays in registers for the exact distances, at two
-        // wavefronts per SIMD (1 M x 64, K 150: 142 us a pass, 196 with three
-        // and the row read again); a row with a tail is read again in any case
-        // (1 M x 50, K 100: 131 us with three, 148 with two)
-        if (tail) PAT_KM_BS(4, 1, 3, false, 768);
-        else PAT_KM_BS(4, 1, 3, false, 512);
-        break;
-    case 8 * 4 + 3: PAT_KM(8, 1, 3); break;
-    default: pat::set_error("kmeans: D too large"); return PAT_ERR_UNSUPPORTED;
-    }
-#undef PAT_KM
-#undef PAT_KM_GC
-#undef PAT_KM_BS
+    const int64_t tiles = (d.N + 31) / 32, waves = f->threads / 64;
+    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((tiles + waves - 1) / waves, d.cus));
+    hipLaunchKernelGGL(f->kernel, dim3(grid), dim3((unsigned)f->threads), (size_t)lds, st, a, (const void *)d.cb,
+                       (const float *)d.cnorm, d.K_pad, bd, wb, d.rescored);
     PAT_LAUNCH_CHECK();
     return d.bucketed ? bucket_reduce(d, st) : PAT_OK;
 }
