@@ -549,15 +549,17 @@ typedef struct pat_gr_object { /* device memory of one run, set up by the librar
     int64_t unit_bytes, num_units;
     const void *param;         /* the functors' parameter (may be NULL) */
     uint32_t *wave_tables;     /* waves tables of (table_buckets + table_pool_words) words */
-    int32_t *wave_counts;      /* per wavefront: entries of its table's buckets in use */
-    uint32_t *matrix;          /* table_buckets rows of waves words, all 0 before and after a run */
-    unsigned long long *final_buckets; /* table_buckets */
-    int32_t *slots;            /* table_buckets: the final buckets taken */
     uint32_t *final_pool;      /* table_pool_words: the final records, back to back */
     int32_t *status;           /* 0 before a run.  [0] error bits (1 a wavefront's table full, 2 a unit's values
                                   do not fit an empty LDS table, 4 a map's insert refused after another was
                                   taken, 8 the final table full), [1] LDS merges, [2] maps run again, [3] keys,
                                   [4] words of final records */
+    int64_t layout;            /* 0.  Tables built for the earlier layouts of this struct find 0 wavefronts or a
+                                  null pointer here and refuse the call, as this one's do where it is not 0 */
+    int32_t *wave_counts;      /* per wavefront: entries of its table's buckets in use */
+    uint32_t *matrix;          /* table_buckets rows of waves words, all 0 before and after a run */
+    unsigned long long *final_buckets; /* table_buckets */
+    int32_t *slots;            /* table_buckets: the final buckets taken */
     int32_t waves, table_buckets, table_pool_words, lds_buckets, lds_pool_words;
 } pat_gr_object;
 typedef struct pat_gr_table {

@@ -360,7 +360,7 @@ int ro_dispatch(int mi, int ri, const pat_gr_object &a, hipStream_t st, std::ind
 template <class Tab>
 int ro_entry(int map_idx, int reduce_idx, const pat_gr_object *obj, void *stream)
 {
-    if (!obj || obj->waves <= 0 || !obj->wave_tables || !obj->wave_counts || !obj->matrix || !obj->final_buckets ||
+    if (!obj || obj->layout != 0 || obj->waves <= 0 || !obj->wave_tables || !obj->wave_counts || !obj->matrix || !obj->final_buckets ||
         !obj->slots || !obj->final_pool || !obj->status || obj->lds_buckets <= 0 || obj->lds_buckets > kRoLdsBuckets ||
         (obj->lds_buckets & (obj->lds_buckets - 1)) || obj->lds_pool_words <= 0 ||
         obj->lds_pool_words > kRoLdsPool || obj->table_buckets <= 0 ||

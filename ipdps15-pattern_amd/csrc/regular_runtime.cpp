@@ -167,6 +167,7 @@ struct pat_regular {
             lpw = (int)std::min<int64_t>(lpw, (int64_t)lds_keys * (2 + (max_record_bytes + 3) / 4));
         }
         pat_gr_object o;
+        o.layout = 0;
         o.data = input;
         o.offsets = offsets;
         o.unit_bytes = unit_bytes;
@@ -189,8 +190,9 @@ struct pat_regular {
         matrix_clear = false;  // until the run has ended well: its fold leaves the matrix clear
         PAT_HIP(hipMemsetAsync(o.status, 0, kStatusWords * sizeof(int32_t), stream));
         const int rc = table->map_reduce(map_idx, reduce_idx, &o, stream);
-        PAT_REQUIRE(rc == PAT_OK, rc, "pat_regular_start: the table's kernels for map %d / reduce %d failed (%d)",
-                    map_idx, reduce_idx, rc);
+        PAT_REQUIRE(rc == PAT_OK, rc,
+                    "pat_regular_start: the table's kernels for map %d / reduce %d failed (%d)%s", map_idx, reduce_idx,
+                    rc, rc == PAT_ERR_INVALID ? "; a table built against another version of the library is refused" : "");
         const int64_t head = std::min(pw, kFirstWords);
         PAT_HIP(hipMemcpyAsync(host, final, sizeof(uint32_t) * (size_t)(kStatusWords + head), hipMemcpyDeviceToHost,
                                stream));

@@ -109,6 +109,39 @@ def test_serving_structs_match_the_header(pa, tmp_path):
             assert int(got[f"{t}.{f}"]) == getattr(cls, f).offset, (t, f)
 
 
+def test_keyed_tables_of_other_layouts_are_refused(pa):
+    """A keyed table refuses an object struct whose layout word (at the place
+    where the first layout had its number of wavefronts) is not 0, before it
+    launches anything; the library passes 0, which a table built for an earlier
+    layout refuses in turn (no wavefronts, or a null pointer)."""
+    import ctypes
+
+    class Object(ctypes.Structure):
+        _fields_ = ([(n, ctypes.c_uint64) for n in ("data", "offsets", "unit_bytes", "num_units", "param", "wave_tables",
+                                                    "final_pool", "status", "layout", "wave_counts", "matrix",
+                                                    "final_buckets", "slots")]
+                    + [(n, ctypes.c_int32) for n in ("waves", "table_buckets", "table_pool_words", "lds_buckets",
+                                                     "lds_pool_words")])
+
+    class Table(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_int) for n in ("map_count", "reduce_count", "max_lds_buckets", "max_lds_pool_words")] + [
+            ("map_reduce", ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.POINTER(Object),
+                                            ctypes.c_void_p))]
+
+    assert Object.layout.offset == 64
+    text = open(os.path.join(ROOT, "include", "pattern.h")).read()
+    body = text[text.index("typedef struct pat_gr_object"):text.index("} pat_gr_object;")]
+    body = re.sub(r"/\*.*?\*/", "", body, flags=re.S)
+    names = [n for line in re.findall(r"[^;{]+;", body) for n in re.findall(r"\*?(\w+)\s*(?=[,;])", line)]
+    assert names == [f[0] for f in Object._fields_]
+    table = Table.from_address(pa.app_table("keys", "gr"))
+    some = {n: 4096 for n, t in Object._fields_ if t is ctypes.c_uint64}  # never dereferenced
+    o = Object(**some, waves=1, table_buckets=16, table_pool_words=64, lds_buckets=16, lds_pool_words=64)
+    assert table.map_reduce(table.map_count, 0, ctypes.byref(o), None) == pa.PAT_ERR_INVALID
+    o.layout = 0
+    assert table.map_reduce(table.map_count, 0, ctypes.byref(o), None) != pa.PAT_OK  # no such map
+
+
 def test_python_constants_match_the_header(pa):
     """Every integer #define of include/pattern.h that the Python binding
     mirrors has the header's value; the status codes are all mirrored."""
