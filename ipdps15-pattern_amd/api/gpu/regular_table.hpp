@@ -97,11 +97,13 @@ __device__ bool ro_insert_wave(const pat_gr_object &a, ro_word *bk, ro_word *poo
                 if ((int64_t)at + need > a.table_pool_words) return false;  // the bucket stays claimed: the result is void
                 ro_word *r = pool + at;
                 for (int i = 0; i < need; i++) r[i] = rec[i];
+                __threadfence_block();  // the record before its place: other lanes may read it as soon as they see that
                 atomicExch((uint32_t *)&bk[b], at + 1u);
                 return true;
             }
         }
         if (st == kRoPending) continue;
+        __threadfence_block();  // the place before the record
         ro_word *r = pool + (st - 1u);
         if (r[0] == rec[0] && ro_equal(r + 1, key, ks)) {
             reduce((void *)(r + 1 + RoTable::key_words(ks)), (unsigned short)vs, (void *)val, (unsigned short)vs);

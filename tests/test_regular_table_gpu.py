@@ -190,3 +190,18 @@ def test_key_and_value_forms(pa, gpu, m, n, lds_keys):
         r.set_capacity(2048, 96, lds_keys)  # another geometry on the same buffers
         assert r.run(m, reduce_idx=0) == want
     r.close()
+
+
+def test_spilled_tables_hold_records_of_the_run_before(pa, gpu):
+    """The wavefronts' tables in device memory are not cleared between starts:
+    runs of several functors in turn on one handle, spilling all the time, find
+    other records of the run before at every place, some of the same keys."""
+    v = np.random.default_rng(5).integers(0, 2 ** 31, 40003, dtype=np.uint32)
+    r = pa.Regular(v, len(v), 4, table=pa.app_table("keys", "gr"))
+    r.set_capacity(1024, 96, 6)
+    want = {m: keyed_by_hand(v, m) for m in (0, 1, 2)}
+    for m in (0, 1, 2, 1, 0, 2, 2, 0, 0, 1):
+        assert r.run(m, reduce_idx=0) == want[m], m
+    merges, reruns, waves = r.stats()
+    assert merges > waves and reruns > 0
+    r.close()
