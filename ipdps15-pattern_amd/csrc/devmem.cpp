@@ -138,3 +138,23 @@ size_t arena_largest_free(const Arena *a)
 }
 
 }  // namespace pat
+
+// For the tests; not part of the public interface.  Binds an arena of so many
+// bytes to the calling thread, whose allocations then come from it (and fail
+// beyond it); unbinding frees it.
+extern "C" int pat_internal_arena_bind(int64_t bytes, void **arena)
+{
+    PAT_REQUIRE(arena && bytes > 0, PAT_ERR_INVALID, "arena: bad arguments");
+    pat::Arena *a = pat::arena_create((size_t)bytes);
+    if (!a) return PAT_ERR_NOMEM;
+    pat::arena_bind(a);
+    *arena = a;
+    return PAT_OK;
+}
+
+extern "C" int pat_internal_arena_unbind(void *arena)
+{
+    pat::arena_bind(nullptr);
+    pat::arena_destroy((pat::Arena *)arena);
+    return PAT_OK;
+}

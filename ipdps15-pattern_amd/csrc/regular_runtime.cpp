@@ -13,6 +13,7 @@
 // one start is one device pass and the object comes back whole.
 #include <algorithm>
 #include <cstring>
+#include <utility>
 #include <vector>
 
 #include "pat_common.hpp"
@@ -26,7 +27,8 @@ constexpr int64_t kDefaultRecordBytes = 256;
 // them), and no more than eight per CU, beyond which the fold's rows grow and
 // the map gains nothing.  Each holds a table of the object's full capacity in
 // case its LDS table overflows: their number is also held to kTableWords, or
-// to one per kUnitsFew units where that takes more.
+// to one per kUnitsFew units where that takes more, and halved as long as the
+// device has not that much memory.
 constexpr int kMaxWaves = 2048;
 constexpr int64_t kUnitsPerWave = 256;
 constexpr int64_t kUnitsFew = 4096;
@@ -155,10 +157,20 @@ struct pat_regular {
         const int64_t fit = std::max(few, kTableWords / per_wave);
         waves = (int)std::min<int64_t>(std::min<int64_t>(kMaxWaves, fit),
                                        std::max<int64_t>(1, (num_units + kUnitsPerWave - 1) / kUnitsPerWave));
-        PAT_TRY(grow(&tables, &tables_words, (nb + pw) * waves + (waves + (waves & 1)) + 3 * nb));
-        if (nb * waves > matrix_words) matrix_clear = false;
-        PAT_TRY(grow(&matrix, &matrix_words, nb * waves));
         PAT_TRY(grow(&final, &final_words, kStatusWords + pw));
+        // where memory is short, fewer wavefronts do
+        for (;; waves = (waves + 1) / 2) {
+            if (nb * waves > matrix_words) matrix_clear = false;
+            int rc = grow(&tables, &tables_words, (nb + pw) * waves + (waves + (waves & 1)) + 3 * nb);
+            if (rc == PAT_OK) rc = grow(&matrix, &matrix_words, nb * waves);
+            if (rc == PAT_OK) break;
+            if (rc != PAT_ERR_NOMEM || waves == 1) return rc;
+            for (auto [p, words] : {std::make_pair(&tables, &tables_words), std::make_pair(&matrix, &matrix_words)}) {
+                if (*p) (void)pat::dev_free(*p);
+                *p = nullptr;
+                *words = 0;
+            }
+        }
         // LDS table: buckets a power of two covering lds_keys (or the
         // kernels' largest), pool words for that many records
         int lnb = table->max_lds_buckets, lpw = table->max_lds_pool_words;

@@ -205,3 +205,28 @@ def test_spilled_tables_hold_records_of_the_run_before(pa, gpu):
     merges, reruns, waves = r.stats()
     assert merges > waves and reruns > 0
     r.close()
+
+
+@pytest.mark.parametrize("room", [300, 40])
+def test_start_with_little_device_memory(pa, gpu, tab, room):
+    """A start whose tables do not fit the memory at hand runs on fewer
+    wavefronts: a million units at the default capacity in 300 MB (a wavefront
+    for 4,096 units) and in 40; the counts stay exact."""
+    vals = np.random.default_rng(17).integers(0, 2 ** 31, 1000000, dtype=np.uint32) % 2003
+    arena = pa.c_vp()
+    bind, unbind = pa.lib().pat_internal_arena_bind, pa.lib().pat_internal_arena_unbind
+    bind.argtypes, unbind.argtypes = [pa.c_i64, pa.ctypes.POINTER(pa.c_vp)], [pa.c_vp]
+    assert bind(room << 20, pa.ctypes.byref(arena)) == 0
+    try:
+        r = pa.Regular(vals, len(vals), 4, table=tab)
+        try:
+            out = r.run(3)
+            again = r.run(3)
+            waves = r.stats()[2]
+        finally:
+            r.close()
+    finally:
+        unbind(arena)
+    assert again == out and waves < 936
+    cnt = np.bincount(vals, minlength=2003)
+    assert {u32(k): int(np.frombuffer(v[:8], np.int64)[0]) for k, v in out.items()} == dict(enumerate(cnt.tolist()))
