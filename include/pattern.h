@@ -192,7 +192,9 @@ int pat_stencil_run_timed(pat_stencil *s, int nsteps, float *total_ms, float *ke
 /* Copies the current halo-inclusive grid out. */
 int pat_stencil_download(pat_stencil *s, void *host);
 /* Tile the runs use (tuned on the first run when none was set): x width,
- * tile height in rows, z-chunk in planes. */
+ * tile height in rows, z-chunk in planes.  For an application table's kernels:
+ * the consecutive cells of the interior's rows that a workgroup takes, 1, and
+ * the planes. */
 int pat_stencil_tile(pat_stencil *s, int *bx, int *by, int *zc);
 /* Device pointer of the current grid.  A halo written through it is read by
  * the next sweep if that is a run of its own (one step); the values for runs

@@ -28,6 +28,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "gpu/stencil_planes.hpp"
 #include "pattern.h"
 
 namespace pat_gpu {
@@ -71,14 +72,14 @@ __device__ __forceinline__ int divide(int t, Divisor v)
 // the XCDs' chunks: 23.8, 65.4 and 111; in 64 x 4 blocks, whose last column of
 // blocks is nearly empty at 200 and 300: 19.5, 35.8 and 119.
 template <class Tab, int I, int P>
-__global__ __launch_bounds__(256) void stencil_sweep(const void *__restrict__ in, void *__restrict__ out,
+__global__ __launch_bounds__(kStencilCells) void stencil_sweep(const void *__restrict__ in, void *__restrict__ out,
                                                      StencilGrid g, const void *param, Divisor blocks, Divisor nx,
                                                      int plane)
 {
     // workgroups are dealt to the 8 XCDs in turn: each takes a run of planes
     const int per = (int)gridDim.x / 8, bid = (int)blockIdx.x;
     const int t = bid < per * 8 ? bid % 8 * per + bid / 8 : bid;
-    const int tz = divide(t, blocks), i = (t - tz * blocks.d) * 256 + (int)threadIdx.x;
+    const int tz = divide(t, blocks), i = (t - tz * blocks.d) * kStencilCells + (int)threadIdx.x;
     const int z = g.lo[2] + tz * P;
     if (i >= plane) return;
     const int row = divide(i, nx);
@@ -103,12 +104,7 @@ int stencil_launch(const void *in, void *out, const StencilGrid &grid, const voi
         return PAT_ERR_UNSUPPORTED;
     } else {
         const int nx = grid.hi[0] - grid.lo[0], ny = grid.hi[1] - grid.lo[1], nz = grid.hi[2] - grid.lo[2];
-        // More planes a thread save loads, fewer leave more wavefronts: 4
-        // planes from 8 workgroups per CU (128^3 FP32 heat 5.8 us a sweep, 6.2
-        // with 2; 64^3 star 3.4 and 3.4), 2 from 1 per CU (100^3 star 4.9, 5.6
-        // with 1; at 32^3 star 3.1, 3.0 with 1).
-        const int64_t b256 = ((int64_t)nx * ny + 255) / 256;
-        const int P = b256 * ((nz + 3) / 4) >= 2048 ? (nz >= 4 ? 4 : 1) : (b256 * ((nz + 1) / 2) >= 256 && nz >= 2 ? 2 : 1);
+        const int P = stencil_planes(nx, ny, nz);
         const int chunks = (nz + P - 1) / P;
         // rows per launch: indexes within a plane and workgroups below 2^31
         const int rows = (int)std::max<int64_t>(1, std::min<int64_t>(ny, (1LL << 30) / ((int64_t)nx * chunks)));
@@ -116,10 +112,10 @@ int stencil_launch(const void *in, void *out, const StencilGrid &grid, const voi
             StencilGrid g = grid;
             g.lo[1] = grid.lo[1] + y0;
             g.hi[1] = std::min(grid.hi[1], g.lo[1] + rows);
-            const int plane = nx * (g.hi[1] - g.lo[1]), blocks = (plane + 255) / 256;
+            const int plane = nx * (g.hi[1] - g.lo[1]), blocks = (plane + kStencilCells - 1) / kStencilCells;
             auto launch = [&](auto planes) {
                 hipLaunchKernelGGL((stencil_sweep<Tab, I, decltype(planes)::value>), dim3((unsigned)(blocks * chunks)),
-                                   dim3(256), 0, st, in, out, g, param, divisor(blocks), divisor(nx), plane);
+                                   dim3(kStencilCells), 0, st, in, out, g, param, divisor(blocks), divisor(nx), plane);
             };
             if (P == 4) launch(std::integral_constant<int, 4>{});
             else if (P == 2) launch(std::integral_constant<int, 2>{});
@@ -154,7 +150,7 @@ int stencil_sweep_entry(int idx, const void *in, void *out, const int32_t *size,
         g.hi[d] = used ? size[d] - width : 1;
         if (g.hi[d] <= g.lo[d]) return PAT_ERR_INVALID;
     }
-    if (g.hi[2] - g.lo[2] > 65535) return PAT_ERR_UNSUPPORTED;  // one grid row per plane
+    if (g.hi[2] - g.lo[2] > 65535) return PAT_ERR_UNSUPPORTED;  // as pat_stencil_create
     return stencil_dispatch<Tab>(idx, in, out, g, param, (hipStream_t)stream,
                                  std::make_index_sequence<(std::size_t)Tab::count>{});
 }

@@ -20,6 +20,7 @@
 
 #include "pat_common.hpp"
 
+#include "../api/gpu/stencil_planes.hpp"
 #include "stencil_dev.hpp"
 
 struct pat_stencil {
@@ -438,10 +439,10 @@ int pat_stencil_download(pat_stencil *s, void *host)
 int pat_stencil_tile(pat_stencil *s, int *bx, int *by, int *zc)
 {
     PAT_REQUIRE(s, PAT_ERR_INVALID, "pat_stencil_tile: null handle");
-    if (!s->tuned()) {  // the table kernels' fixed shape: 64 x 4 cells per workgroup, one plane deep
-        if (bx) *bx = 64;
-        if (by) *by = 4;
-        if (zc) *zc = 1;
+    if (!s->tuned()) {  // the table kernels: consecutive cells of the rows, 1 to 4 planes deep
+        if (bx) *bx = pat_gpu::kStencilCells;
+        if (by) *by = 1;
+        if (zc) *zc = pat_gpu::stencil_planes(s->n[0], s->n[1], s->n[2]);
         return PAT_OK;
     }
     pat::HeatTile t;

@@ -154,3 +154,12 @@ def test_table_errors(pa, gpu):
     with pytest.raises(pa.PatternError, match="byte elements"):
         st.run(1)
     st.close()
+
+
+@pytest.mark.parametrize("shape,planes", [((32, 32, 32), 1), ((100, 100, 100), 2), ((200, 186, 210), 4),
+                                          ((2000, 1000, 3), 1), ((300, 200, None), 1)])
+def test_tile_of_table_kernels(pa, gpu, shape, planes):
+    """pat_stencil_tile names the tile that the table's kernels run with."""
+    s = pa.Stencil(*shape, width=3, table=pa.app_table("stencil2"), idx=0)
+    assert s.tile() == (256, 1, planes)
+    s.close()
