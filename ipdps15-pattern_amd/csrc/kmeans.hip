@@ -1302,7 +1302,11 @@ __device__ __forceinline__ void retire_object(int k, int lane, int K, int D, uns
 // One wavefront per centre: applies the Lloyd update from the reduction
 // object (c = (sum * 2^-s) / count in FP64, rounded to FP32; empty clusters
 // keep their centre), writes the BF16 MFMA row and the norm, and clears the
-// object for the next pass.  With update == 0 only the rows are prepared.
+// object for the next pass.  With update == 0 only the rows are prepared.  A
+// centre with a coordinate that is not finite is never map1's nearest: its row
+// is far, as the padding rows are.  So is that of one whose squared norm FP32
+// does not hold, but its norm then makes every bound infinite, so that every
+// centre is rescored.
 template <int KS>
 __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K, int K_pad, int D,
                                                    unsigned long long *__restrict__ gsum,
@@ -1331,13 +1335,15 @@ __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K,
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
+    const bool fine = isfinite((float)ss);
     for (int d = lane; d < 16 * KS; d += kWave) {
-        const float v = d < D ? -2.0f * c[(int64_t)k * D + d] : 0.0f;  // exact
+        const float v = fine && d < D ? -2.0f * c[(int64_t)k * D + d] : 0.0f;  // exact
         cb[frag_index(k, d, KW / 16)] = (__bf16)v;
     }
     if (lane < 16) {
-        const __bf16 n1 = (__bf16)(float)ss;
-        const double r1 = ss - (double)(float)n1;
+        const double nn = fine ? ss : 1.0e30;
+        const __bf16 n1 = (__bf16)(float)nn;
+        const double r1 = nn - (double)(float)n1;
         const __bf16 n2 = (__bf16)(float)r1;
         const double r2 = r1 - (double)(float)n2;
         const __bf16 n3 = (__bf16)(float)r2;
@@ -1347,7 +1353,7 @@ __global__ __launch_bounds__(256) void km_finalize(float *__restrict__ c, int K,
         if (lane == 2) v = n3;
         cb[frag_index(k, NB + lane, KW / 16)] = v;
     }
-    if (lane == 0) cnorm[k] = (float)sqrt(ss) * 1.0001f;
+    if (lane == 0) cnorm[k] = fine ? (float)sqrt(ss) * 1.0001f : (isfinite(ss) ? INFINITY : 0.0f);
     retire_object(k, lane, K, D, gsum, gcnt, gdsum, update, snap);
 }
 
@@ -1381,7 +1387,7 @@ __global__ __launch_bounds__(256) void km_finalize_wide(float *__restrict__ c, i
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
-        fine = isfinite(ss) && isfinite((float)ss);
+        fine = isfinite(ss);  // (also where FP32 does not hold it: it is scaled below)
     }
     for (int d = lane; d < 16 * KS; d += kWave) {
         const float v = fine && d < D ? -(c[(int64_t)k * D + d] * sx) : 0.0f;

@@ -343,3 +343,24 @@ def test_staged_rows_bitexact(pa, orc, gpu, n, d, k):
     ra, rmd = orc.kmeans_assign(x, odd)
     assert np.array_equal(a, ra) and np.array_equal(md, rmd)
     km.close()
+
+
+@pytest.mark.parametrize("n,d,k,terms", [(5000, 8, 16, 1), (5000, 8, 16, 3), (3000, 32, 64, 1), (3000, 32, 64, 3),
+                                         (3000, 40, 600, 0), (3000, 128, 300, 0), (2000, 8, 1000, 0)])
+@pytest.mark.parametrize("magnitude", [3e19, 1e37])
+def test_coordinates_whose_squares_overflow(pa, orc, gpu, n, d, k, terms, magnitude):
+    """A third of the points, and of the centres, at coordinates whose squares
+    FP32 does not hold, some of them repeated: a point that equals a centre is
+    given that centre, every other one beyond map1's initial minimum centre 0."""
+    x = np.random.default_rng(5).standard_normal((n, d)).astype(np.float32)
+    x[::3] *= np.float32(magnitude)
+    x[1::50] = x[0]
+    x[7::90] = x[3]
+    km = pa.KMeans(x, k, mode=1)
+    if terms:
+        km.set_terms(terms)
+    km.run(1)
+    _, a, md = km.get()
+    km.close()
+    ra, rmd = orc.kmeans_assign(x, x[:k].copy())
+    assert np.array_equal(a, ra) and np.array_equal(md, rmd)
