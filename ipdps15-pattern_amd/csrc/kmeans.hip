@@ -459,12 +459,13 @@ constexpr float kFar = 3.0e38f;
 //
 // Per 32-point tile a wavefront (lanes l and l+32 hold halves of point l):
 // computes the approximate values of every centre with MFMAs, packs the
-// smaller of every two with their index (pack_key) and keeps the three
-// smallest keys of each half (the two smallest values per chunk when the index
-// bits cannot tell the chunks apart).  The threshold is the minimum plus the
-// error bound plus the packing error; when only the smallest key is under it
-// (the usual case) its two centres are rescored, one by each half, when a
-// half's third key lies above it the kept keys under it are, and otherwise
+// smaller of every two (one term: every value) with their index (pack_key) and
+// keeps the three smallest keys of each half (the two smallest values per chunk
+// when the index bits cannot tell the chunks apart).  The threshold is the
+// minimum plus the error bound plus the packing error; when only the smallest
+// key is under it (the usual case) its centres are rescored, of two one by each
+// half, when a half's third key lies above it the kept keys under it are, and
+// otherwise
 // every centre under it is (the values recomputed chunk by chunk).  The exact
 // FP32 results decide with map1's rule, and the point is added to the LDS
 // reduction object from the registers holding its half rows.
@@ -673,25 +674,29 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const void *__restrict__
                             : bd.c_dot * xn * cmax + bd.c_norm * (cc_max + xx);
 
         f32x16 acc[KB];
-        // The three smallest keys of this half.  When the pairs of a lane's
-        // values in all chunks fit the 7 index bits (gidx: at most 128), a key
-        // is the smaller of two adjacent centres' values with the pair's index
-        // (values i and i + 1 of block blk -> 8 blk + i / 2): five instructions
-        // for two values, and the halves rescore one centre of a pair each.
-        // One sorted triple runs over all chunks.  Otherwise the keys are
-        // single values, each chunk's two smallest are merged with their
-        // chunk recorded and k3 stays unknown (kFar, never used).
-        const bool gidx = nchunks * KB <= 16;  // uniform
+        // The three smallest keys of this half.  With three terms, when the pairs
+        // of a lane's values in all chunks fit the 7 index bits (gidx: at most
+        // 128), a key is the smaller of two adjacent centres' values with the
+        // pair's index (values i and i + 1 of block blk -> 8 blk + i / 2): five
+        // instructions for two values, and the halves rescore one centre of a
+        // pair each.  With one term, whose bound leaves many points several
+        // candidates, a key is a value (16 blk + i, while those fit): 5 M x 32, K
+        // 32: 405 us an iteration, 565 with pairs.  One sorted triple runs over
+        // all chunks.  Otherwise the keys are single values, each chunk's two
+        // smallest are merged with their chunk recorded and k3 stays unknown
+        // (kFar, never used).
+        const bool gidx = nchunks * KB <= (F16 ? 16 : 8);  // uniform
         float k1 = kFar, k2 = kFar, k3 = kFar;
         int ch1 = 0;
         auto scan3 = [&](int ch, const f32x16 (&v)[KB]) {
+            constexpr int STEP = F16 ? 2 : 1;
 #pragma unroll
             for (int b = 0; b < KB; b++) {
                 if (b > 0 && ch * KB + b >= kblocks) break;  // uniform; block 0 of a chunk always exists
 #pragma unroll
-                for (int i = 0; i < 16; i += 2) {
-                    const float lo = __builtin_amdgcn_fmed3f(v[b][i], v[b][i + 1], -kFar);  // min (finite)
-                    const float key = pack_key(lo, scalar_or((ch * KB + b) * 8, i / 2), keep);
+                for (int i = 0; i < 16; i += STEP) {
+                    const float lo = F16 ? __builtin_amdgcn_fmed3f(v[b][i], v[b][i + STEP - 1], -kFar) : v[b][i];  // min (finite)
+                    const float key = pack_key(lo, scalar_or((ch * KB + b) * (16 / STEP), i / STEP), keep);
                     k3 = __builtin_amdgcn_fmed3f(k2, k3, key);
                     k2 = __builtin_amdgcn_fmed3f(k1, k2, key);
                     k1 = __builtin_amdgcn_fmed3f(k1, key, -kFar);
@@ -768,7 +773,7 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const void *__restrict__
         const bool multi = !(m2 > thr);
         // points whose candidates may lie beyond the keys they kept: every
         // value under the threshold is then visited again (full)
-        const bool full = multi && (!gidx || !(fminf(k3, o3) > thr));
+        const bool full = multi && (!gidx || !((F16 ? fminf(k3, o3) : k3) > thr));
         // the whole point row in registers (full K-steps) where the form has
         // the registers to spare (the others would spill: they reload it)
         constexpr bool ROW = !TAIL && !GC && KB == 1 && (KS <= 2 || (KS == 4 && BS <= 512));
@@ -793,7 +798,7 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const void *__restrict__
             const int id = __float_as_int(key) & 127, i = 2 * (id & 7);
             return (id >> 3) * 32 + 8 * (i >> 2) + 4 * h + (i & 3) + half;
         };
-        if (gidx) {
+        if (F16 && gidx) {
             // the kept pairs under the threshold are all of its candidates
             // (the third smallest of each half lies above it): the smallest,
             // and of several the other three as far as they are under it
@@ -807,8 +812,12 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const void *__restrict__
                 if (more && !(u > thr)) rescore(pair_centre(u, second ? half : 1 - half));
                 if (more && !(w > thr)) rescore(pair_centre(w, second ? 1 - half : half));
             }
-        } else if (live && !multi && k1 < o1) {
-            rescore(centre_of(ch1, __float_as_int(k1) & 127));
+        } else if (live && !full) {
+            // one candidate: rescored by the half that holds it; several (gidx
+            // only): each half rescores its kept keys under the threshold, which
+            // are all of its candidates since its third lies above it
+            if (multi ? !(k1 > thr) : k1 < o1) rescore(centre_of(gidx ? 0 : ch1, __float_as_int(k1) & 127));
+            if (multi && !(k2 > thr)) rescore(centre_of(0, __float_as_int(k2) & 127));
         }
         // Every value under the threshold for the full lanes.  Taken by the
         // whole wavefront (a vote), because recomputing a chunk's values
