@@ -319,7 +319,7 @@ def bench_stencil(n, steps, cpu=False):
 def bench_kmeans(iters=20, cpu=False):
     """kmeans: N = 2^24, D = 32, K = 256 (256-component mixture, sigma 1,
     centres in [-10, 10]^32), K centres from the first K points, 20 Lloyd
-    iterations; BF16-MFMA with FP32 rescoring vs the plain FP32 kernel."""
+    iterations; MFMA distances with FP32 rescoring vs the plain FP32 kernel."""
     n, d, k = 1 << 24, 32, 256
     t0 = time.perf_counter()
     x = pa.gen_gmm(n, d, 256, sigma=1.0, lo=-10, hi=10, seed=2024)

@@ -453,7 +453,7 @@ int pat_md_destroy(pat_md *h);
  * ---------------------------------------------------------------------- */
 
 #define PAT_KM_PLAIN 0 /* FP32 difference form over every centre (map1's arithmetic) */
-#define PAT_KM_MFMA 1  /* BF16 MFMA distances + exact FP32 rescoring inside the error margin */
+#define PAT_KM_MFMA 1  /* MFMA distances + exact FP32 rescoring inside the error margin */
 
 /* Fixed-point shift s used for the order-independent sums of n values of
  * magnitude below maxabs (maxabs * 2^s <= 2^30 and n * maxabs * 2^s < 2^62). */
@@ -468,8 +468,9 @@ typedef struct pat_kmeans pat_kmeans;
  * device pointer the handle reads in place. */
 int pat_kmeans_create(const float *x, int64_t n, int d, int k, int mode, int x_on_device, pat_kmeans **out);
 int pat_kmeans_set_mode(pat_kmeans *h, int mode);
-/* BF16 terms of the MFMA path's distance values: 3 (x and -2c split into
- * high and low parts) or 1 (rounded once, a wider rescoring margin).  Both
+/* Terms of the MFMA path's distance values: 3 (x and c split into FP16 high
+ * and low parts) or 1 (x and -2c rounded to BF16 once, a wider rescoring
+ * margin).  Both
  * give the plain path's assignments bit for bit; by default the faster one
  * on the handle's data is kept (timed at creation when both fit in LDS and
  * N >= 2^20; three terms otherwise).
@@ -682,7 +683,7 @@ typedef struct pat_serve pat_serve;
  *   LJ (boxes of at least three neighbour bins, up to 2^21 atoms): pat_mdb,
  *   one fused force and update launch per step over every system, the steps
  *   between neighbour rebuilds replayed from a captured hipGraph;
- *   heat3D (sides up to 128, up to 2^23 cells): two sweeps per launch over
+ *   heat3D (sides up to 128, up to 2^23 cells): four sweeps per launch over
  *   every grid, the launches captured as one hipGraph.
  * Each job's result is the same bits either way; the batch's jobs share its
  * start and end times. */

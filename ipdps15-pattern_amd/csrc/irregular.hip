@@ -10,9 +10,9 @@
 // device hash (rog.cu:11-100).
 //
 // Here the edges are reordered once on the device into a by-destination CSR
-// (every half edge (i, j) appears in row i and in row j): a degree histogram,
-// an exclusive scan, a scatter, and a per-row sort that makes the layout --
-// and so every later force sum -- deterministic.  The force kernel then gives
+// (every half edge (i, j) appears in row i and in row j): entries counted and
+// scattered by buckets of rows, and every bucket's rows placed and sorted from
+// LDS, which makes the layout -- and so every later force sum -- deterministic.  The force kernel then gives
 // each row to a group of LPR lanes of a wavefront: the lanes stride the row's
 // neighbour list, each computing the pair force with exactly the functor's
 // arithmetic, and the group reduces its partial sums with cross-lane

@@ -63,7 +63,7 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
 constexpr float kInitMin = 65536 * 65;  // map1's initial min_dist (kmeans/regular.h:86)
 
-// Position of element e of centre row k in the BF16 MFMA operand array,
+// Position of element e of centre row k in the MFMA operand array,
 // stored in fragment order: for 32-row block b and K-step s, lane
 // l = (k % 32) + 32 * ((e % 16) / 8) holds elements 8*(l/32) .. +8 of row
 // b*32 + l%32 at 16-byte slot (b*NS + s)*64 + l, so a wavefront's operand
@@ -481,7 +481,7 @@ constexpr float kFar = 3.0e38f;
 // K-step is full and the loads need no per-element guard.
 // GC: the form for K x D too large for LDS.  The workgroup's wavefronts
 // step through the centre chunks together: before each chunk the
-// workgroup copies its KB blocks of BF16 rows from global memory into one
+// workgroup copies its KB blocks of rows from global memory into one
 // LDS chunk buffer (between two barriers) and every wavefront computes its
 // own tile against it, so each copy of the rows serves 8 tiles.  Tiles are
 // taken block-uniformly (a wavefront past the last tile computes with every
@@ -590,7 +590,7 @@ __global__ __launch_bounds__(BS) void km_mfma(KmArgs a, const void *__restrict__
     const int64_t ntiles = (a.N + 31) / 32;
     const int64_t nw = (int64_t)gridDim.x * (blockDim.x / kWave);
     // this lane's half of tile t's point row (dimensions 16s + 8*half + e);
-    // dead lanes read a valid row and keep zeros
+    // dead lanes read a valid row (their values reach no result)
     auto load_half_row = [&](int64_t t, float (&xo)[8 * KS]) {
         const int64_t p = t * 32 + col;
         const bool live = p < a.N;

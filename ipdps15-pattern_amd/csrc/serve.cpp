@@ -24,7 +24,7 @@
 // batch.  LJ jobs become one MD batch (pat_mdb): every step is one force +
 // velocity-Verlet launch over all their systems, and the steps between
 // neighbour rebuilds replay a captured hipGraph; each system's sums keep
-// their own order.  Heat3D grids are swept two steps per launch over every
+// their own order.  Heat3D grids are swept four steps per launch over every
 // grid, the launches captured as one hipGraph; any tiling gives the serial
 // sweep's values.  So every job gets the bits it gets alone.  kmeans jobs
 // run alone (their D and K select different kernels).
@@ -239,9 +239,9 @@ struct pat_serve {
         return rc;
     }
 
-    // Several heat3D jobs as one batch: their sweeps run two per launch over
-    // every grid (the fused-window kernel, each workgroup finding its grid
-    // in a device table), captured as one hipGraph.  Same bits as each job
+    // Several heat3D jobs as one batch: their sweeps run four per launch over
+    // every grid (the strip kernel, each workgroup finding its grid in a
+    // device table), captured as one hipGraph.  Same bits as each job
     // alone: every tiling gives the serial sweep's results.
     int run_heat_batch(const std::vector<Job> &g, hipStream_t st, double *part, std::vector<pat_job_result> &res)
     {

@@ -17,7 +17,9 @@
 //     and stores;
 //   * tiles are ordered so that consecutive tile indices land on the same XCD
 //     (the dispatcher deals workgroups round-robin over the 8 XCDs), keeping
-//     neighbouring tiles' shared halo rows in one XCD's L2.
+//     neighbouring tiles' shared halo rows in one XCD's L2;
+//   * fields with a zero halo are swept several steps per launch, by strips
+//     held in registers (strip_window), unless a variant asks for a form.
 // Grid layout is the reference's (GET_FLOAT3, heat_3D/lib/macro.h:70):
 // halo-inclusive (nx+2)(ny+2)(nz+2), x fastest.
 // Compiled with -ffp-contract=off: each cell's arithmetic rounds exactly as
@@ -311,8 +313,8 @@ __global__ __launch_bounds__(256) void heat_tb2(const float *__restrict__ in, fl
 // shift that the add itself does.  So a cell update takes 10 to 11 vector
 // instructions and 4 / RY LDS ones, where a window held in LDS (tb2_window)
 // reads four neighbours from LDS and writes one cell.  Measured per step, us,
-// two-sweep windows or cubes before: 64^3 2.74 -> 1.55, 128^3 5.0 -> 3.6,
-// 384^3 59.3 -> 32; at 384^3 vector issue bounds it (72 M instructions of a
+// two-sweep windows or cubes before: 64^3 2.7 -> 1.55, 128^3 4.9 -> 3.5,
+// 384^3 59.4 -> 31.3; at 384^3 vector issue bounds it (72 M instructions of a
 // launch take 123 of its 134 us, 430 MB of traffic).
 //
 // Each cell is read and written once per T steps, plus the window's margins:
@@ -977,7 +979,7 @@ int heat3d_strip(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz
 }
 
 // One launch of tile t: a single sweep (fused == 0), two (fused == 1), t.ry
-// on LDS cubes (fused == 2) or t.ry by strips (fused == 3).
+// on LDS cubes (fused == 2) or t.sweeps by strips (fused == 3).
 int heat3d_launch(const float *in, float *out, int64_t nx, int64_t ny, int64_t nz, float alpha, const HeatTile &t,
                   int variant, hipStream_t stream)
 {

@@ -811,7 +811,8 @@ class KMeans:
         call("pat_kmeans_set_mode", self.h, mode)
 
     def set_terms(self, terms):
-        """BF16 terms of the MFMA distance values (1 or 3; same bits)."""
+        """Terms of the MFMA distance values (1: BF16, 3: FP16 high and low
+        parts; same bits)."""
         call("pat_kmeans_set_terms", self.h, terms)
 
     def terms(self):

@@ -225,7 +225,8 @@ def test_kmeans_workload_full_size(pa, orc, gpu):
                                    (3000, 16, 700), (4000, 8, 2049), (1500, 5, 1500), (9000, 97, 260)])
 @pytest.mark.parametrize("scale", [1.0, 1e-12, 3e15])
 def test_wide_path_bitexact(pa, orc, gpu, n, d, k, scale):
-    """Objects beyond LDS (FP16 high and low parts): partial blocks, chunks and
+    """Objects beyond LDS (FP16 high and low parts; 1500 x 5, K 1500 has its
+    object in LDS and rows that do not fit beside it): partial blocks, chunks and
     groups of centres, one and two tiles a wavefront, rows with a tail, points
     of small and large magnitude; then centres far outside the points' range
     and one that is not finite, which no point may choose."""
