@@ -142,7 +142,7 @@ __global__ __launch_bounds__(64) void ro_map(pat_gr_object a)
         ro_wave_sync();
         for (int b0 = 0; b0 < so.t.nb; b0 += 64) {
             const uint32_t st = b0 + lane < so.t.nb ? so.t.bk[b0 + lane] : 0u;
-            if (st != 0u && st != kRoDead && !ro_insert_wave(a, wbk, wpool, wtop, so.t.pool + (st - 1u), reduce))
+            if (st != 0u && !ro_insert_wave(a, wbk, wpool, wtop, so.t.pool + (st - 1u), reduce))
                 err |= kRoWaveFull;
             // the next records may fold into the ones just written
             __threadfence_block();
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(64) void ro_map(pat_gr_object a)
         count = 0;
         for (int b0 = 0; b0 < so.t.nb; b0 += 64) {
             const uint32_t st = b0 + lane < so.t.nb ? so.t.bk[b0 + lane] : 0u;
-            const bool have = st != 0u && st != kRoDead;
+            const bool have = st != 0u;
             const unsigned long long m = __ballot(have);
             const int at = count + __popcll(m & ((1ull << lane) - 1ull));
             if (have && at < a.table_buckets) wbk[at] = st;

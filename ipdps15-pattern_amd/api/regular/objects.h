@@ -117,10 +117,9 @@ __device__ __forceinline__ void ro_wave_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
-// Bucket states of an LDS table besides 0 (empty) and 1 + a record's word
+// Bucket state of an LDS table besides 0 (empty) and 1 + a record's word
 // offset in the pool.
 constexpr uint32_t kRoClaim = 0x40000000u;  // | (63 - lane): being taken, within one insert only
-constexpr uint32_t kRoDead = 0xffffffffu;   // taken by a key the pool had no room for
 
 // A wavefront's LDS hash table: nb buckets (a power of two), then the pool's
 // fill counter, then pw pool words.  Record: a header word (key_size << 16 |
@@ -146,7 +145,8 @@ struct RoTable {
     // no pool room is left.  Keys of up to eight bytes.  The lanes probe
     // together; where several want one empty bucket the lowest takes it, and
     // new records take pool room in lane order, so that the same lanes are
-    // refused every run.  Lanes with one key probe in step, so they get one
+    // refused every run.  A refused key leaves its bucket empty to the others
+    // that wanted it.  Lanes with one key probe in step, so they get one
     // record in one round.
     __device__ uint32_t place(const void *key, int ks, int vs, bool &fresh)
     {
@@ -163,18 +163,21 @@ struct RoTable {
         uint32_t rec = 0u;
         bool open = true;
         fresh = false;
-        for (int p = 0; __ballot(open); p++) {
-            if (p == nb) break;  // every bucket seen: the lanes still open are refused
+        int p = 0;  // buckets seen: all of them, and the lane is refused
+        // (every round an open lane goes on by a bucket, or one is closed)
+        for (int round = 0; __ballot(open) && round < nb + 64; round++) {
             const int b = (int)((h + (uint32_t)p) & (uint32_t)(nb - 1));
             bool want = false;
             if (open) {
                 const uint32_t st = bk[b];
                 want = st == 0u;
-                if (!want && st != kRoDead) {
+                if (!want) {
                     const ro_word *r = pool + (st - 1u);
                     if (r[0] == hdr && (ks < 1 || r[1] == k0) && (ks < 5 || r[2] == k1)) {
                         rec = st;
                         open = false;
+                    } else {
+                        open = ++p < nb;
                     }
                 }
             }
@@ -216,16 +219,20 @@ struct RoTable {
                     rec = (uint32_t)off + 1u;
                     fresh = true;
                 }
-                bk[b] = off >= 0 ? rec : kRoDead;
+                bk[b] = rec;
                 open = false;
             }
             ro_wave_sync();
             const uint32_t wh = (uint32_t)__shfl((int)hdr, w), w0 = (uint32_t)__shfl((int)k0, w),
                            w1 = (uint32_t)__shfl((int)k1, w), wr = (uint32_t)__shfl((int)rec, w);
-            if (want && !won && wh == hdr && w0 == k0 && w1 == k1) {  // the winner's key: its record or its refusal
-                rec = wr;
-                fresh = wr != 0u;
-                open = false;
+            if (want && !won) {
+                if (wh == hdr && w0 == k0 && w1 == k1) {  // the winner's key: its record or its refusal
+                    rec = wr;
+                    fresh = wr != 0u;
+                    open = false;
+                } else if (wr != 0u) {
+                    open = ++p < nb;
+                }
             }
         }
         return rec;
@@ -253,7 +260,6 @@ struct RoTable {
                 fresh = true;
                 return rec + 1u;
             }
-            if (st == kRoDead) continue;
             ro_word *r = pool + (st - 1u);
             if (r[0] == hdr && ro_equal(r + 1, key, ks)) return st;
         }

@@ -7,7 +7,9 @@
 //                 {v mod 97, 5}; value 1 + v mod 97 mod 3 unsigned ints, each
 //                 v mod 1000;
 //   2  wide       key {v mod 33}, value 20 unsigned ints {v mod 1000 + i};
-//   3  two        two inserts: key {v mod 50} and key {50 + v mod 7}, value 1.
+//   3  two        two inserts: key {v mod 50} and key {50 + v mod 7}, value 1;
+//   4  uneven     two inserts: key {v mod 33}, value 20 unsigned ints {v mod 1000 + i},
+//                 and where that is taken key {1000 + v mod 3}, value 1.
 // Every reduce adds unsigned ints, so any fold order gives the same bytes.
 #ifndef KEYS_H_
 #define KEYS_H_
@@ -58,7 +60,14 @@ DEVICE bool two(SO *object, void *global_data, unsigned long long index, void *,
     return object->insert(&b, sizeof(b), &one, sizeof(one), reduce_ptr) && first;
 }
 
-CONSTANT map_fp map_function_table[] = {long_key, mixed, wide, two};
+DEVICE bool uneven(SO *object, void *global_data, unsigned long long index, void *param, int type, reduce_fp reduce_ptr)
+{
+    if (!wide(object, global_data, index, param, type, reduce_ptr)) return false;
+    unsigned key = 1000 + *(const unsigned *)((char *)global_data + index) % 3, one = 1;
+    return object->insert(&key, sizeof(key), &one, sizeof(one), reduce_ptr);
+}
+
+CONSTANT map_fp map_function_table[] = {long_key, mixed, wide, two, uneven};
 CONSTANT reduce_fp reduce_function_table[] = {add};
 
 }  // namespace FFGPU

@@ -163,9 +163,12 @@ def keyed_by_hand(v, m):
             add([k, 5] if k % 2 else [k], np.full(1 + k % 3, r, np.uint32))
         elif m == 2:
             add([x % 33], r + np.arange(20, dtype=np.uint32))
-        else:
+        elif m == 3:
             add([x % 50], np.ones(1, np.uint32))
             add([50 + x % 7], np.ones(1, np.uint32))
+        else:
+            add([x % 33], r + np.arange(20, dtype=np.uint32))
+            add([1000 + x % 3], np.ones(1, np.uint32))
     return {k: a.astype(np.uint32).tobytes() for k, a in want.items()}
 
 
@@ -230,3 +233,19 @@ def test_start_with_little_device_memory(pa, gpu, tab, room):
     assert again == out and waves < 936
     cnt = np.bincount(vals, minlength=2003)
     assert {u32(k): int(np.frombuffer(v[:8], np.int64)[0]) for k, v in out.items()} == dict(enumerate(cnt.tolist()))
+
+
+def test_refused_records_leave_their_buckets(pa, gpu):
+    """Maps that insert a large record and, where it is taken, a small one, into
+    LDS tables of eight buckets with room for five large records and the three
+    small ones: the lanes whose large record is refused take no bucket from the
+    small ones, so no map is refused half done."""
+    v = np.random.default_rng(3).integers(0, 2 ** 31, 20011, dtype=np.uint32)
+    r = pa.Regular(v, len(v), 4, table=pa.app_table("keys", "gr"))
+    r.set_capacity(1024, 96, 5)
+    want = keyed_by_hand(v, 4)
+    assert r.run(4, reduce_idx=0) == want
+    assert r.run(4, reduce_idx=0) == want
+    merges, reruns, waves = r.stats()
+    assert merges > waves and reruns > 0
+    r.close()
