@@ -203,6 +203,22 @@ def test_strip_windows_vs_oracle(pa, orc, gpu, shape, sweeps):
         assert np.array_equal(got, orc.heat3d(g, sweeps), equal_nan=True), (nx, ny, nz, zc)
 
 
+@pytest.mark.parametrize("sweeps", [1, 4, 6])
+@pytest.mark.parametrize("shape", range(5))
+def test_strip_windows_where_values_are_not_finite(pa, orc, gpu, shape, sweeps):
+    """Grids of two windows and a cell (whose cells need no test against the
+    grid's end): infinities and NaN at the faces and where the windows meet
+    stay where the single sweep has them."""
+    wx, wy = STRIPS[shape]
+    nx, ny, nz = 2 * wx - 2 * sweeps + 1, 2 * wy - 2 * sweeps + 1, 9
+    g = pa.gen_heat3d(nx, ny, nz, seed=4)
+    for z, y, x, v in ((1, 1, 1, np.inf), (nz, ny, nx, np.nan), (1, ny, 3, -np.inf), (5, wy - sweeps, wx - sweeps, np.inf),
+                       (7, wy - sweeps + 1, wx - sweeps + 1, np.nan), (4, 1, nx, -np.inf)):
+        g[z, y, x] = v
+    got = strip_run(pa, g, shape, sweeps, 4)
+    assert np.array_equal(got, orc.heat3d(g, sweeps), equal_nan=True)
+
+
 @pytest.mark.parametrize("shape", [(20, 18, 22), (64, 64, 64), (70, 40, 33)])
 @pytest.mark.parametrize("variant", ["PAT_STENCIL_AUTO", "PAT_STENCIL_TEMPORAL2"])
 def test_halo_values_are_kept(pa, orc, gpu, shape, variant):
