@@ -158,25 +158,26 @@ def test_csr_build_long_lists(pa, gpu, n, e, order):
 def test_csr_build_time_per_edge(pa, gpu, order):
     """No list is much dearer per edge than one a little shorter: 6,911,762
     edges (the moldyn list at 40 cells) and 6,600,000, by the best of several
-    builds (5% allowed, 1% measured; with a last round of eight workgroups 12%
-    in node order)."""
+    builds in turn (8% allowed, 1% measured; with a last round of eight
+    workgroups 12% in node order)."""
     n = 256000
-    us = []
+    lists = []
     for e in (6600000, 6911762):
         wb = pa.c_i64(0)
         pa.call("pat_ir_csr_workspace", n, e, pa.ctypes.byref(wb))
         buf = [pa.DeviceArray((m,), t) for m, t in ((wb.value, np.uint8), (n + 1, np.int32), (2 * e, np.int32))]
         ed = pa.DeviceArray.from_numpy(np.random.default_rng(7).integers(0, n, (e, 2), dtype=np.int32))
-        times = []
-        for _ in range(20):
+        lists.append((e, wb.value, buf, ed, []))
+    for _ in range(20):
+        for e, wb, buf, ed, times in lists:
             pa.sync()
             t0 = time.perf_counter()
             for _ in range(4):
-                pa.call("pat_ir_csr_build_dev", ed.ptr, e, n, order, buf[1].ptr, buf[2].ptr, buf[0].ptr, wb.value, None)
+                pa.call("pat_ir_csr_build_dev", ed.ptr, e, n, order, buf[1].ptr, buf[2].ptr, buf[0].ptr, wb, None)
             pa.sync()
             times.append(time.perf_counter() - t0)
-        us.append(min(times) / e)
-    assert us[1] <= 1.05 * us[0], us
+    per_edge = [min(times) / e for e, _, _, _, times in lists]
+    assert per_edge[1] <= 1.08 * per_edge[0], per_edge
 
 
 @pytest.mark.parametrize("order", [0, 1])
